@@ -28,6 +28,11 @@
 
 using namespace cms;
 
+// Level 0 of fewer cells takes the 64 x 8 tile untimed: at 20 000 to 84 000
+// cells it runs in 5.3 us where the 2048-cell tiles take 6.8-10 us; from 400 000
+// cells (780 tiles of 512) the shapes are within a microsecond and are timed.
+static constexpr int MG_SMALL_LEVEL0 = 400000;
+
 // Fixed grid of the Krylov kernels (4 workgroups per CU on 256 CUs).
 static constexpr int KRY_BLOCKS = 1024;
 
@@ -142,7 +147,7 @@ struct cms2d_flow {
     Mg mg{};                   // pp preconditioner hierarchy (level 0 z is Kpp.zp / Kpp.zs)
     KrySys<1, float> Kin{};    // inner FP32 solve of the refinement form (pp)
     KrySys<2, float> Kin2{};   // inner FP32 solves of the refinement form (u, v)
-    float *a32[4]{};           // their FP32 coefficients
+    float4 *a32 = nullptr;     // their FP32 coefficients
     KryScal *d_sc = nullptr;   // [6]: pp, u, v, inner FP32 pp, inner FP32 u, v
     KryScal *h_sc = nullptr;   // pinned mirror
     int *h_flags = nullptr;    // pinned
@@ -166,6 +171,7 @@ struct cms2d_flow {
     bool use_graphs = false;
     hipGraphExec_t kgraph[6]{};
     int mg_tile = 128;         // level-0 tile width of the multigrid cycle (timed at creation)
+    int mg_tile_small = 0;     // its 64-wide tile has 8 rows, not 32
     // the reference's cell order for the three order-dependent loops: the
     // buffers of consecutive passes (dry-to-wet u, v, vis; fix-up face values
     // [4*npad]; corner values)
@@ -466,32 +472,58 @@ static int run_bicg(KryCtx &X, KrySys<NS, T> &K, Op A, int sc0, Pre pre = Pre())
 
 static int mg_nblk(const MgLevel &L) { return (L.nx * L.ny + BLOCK - 1) / BLOCK; }
 
+// The coarse operators from level 0's (levels of the tail in one launch).
+static void mg_coarsen_levels(cms2d_flow *F) {
+    const Mg &M = F->mg;
+    for (int l = 0; l < M.lt; l++) LAUNCH(k_mg_coarsen, mg_nblk(M.L[l + 1]), M.L[l], M.L[l + 1]);
+    if (M.lt + 1 < M.nlev) hipLaunchKernelGGL(k_mg_coarsen_tail, dim3(1), dim3(MG_TAIL_NT), 0, F->st, M, M.lt + 1);
+}
 // Builds the hierarchy from the assembled pp system (after the solve prologue
 // has written ap).
 static void mg_setup_from(cms2d_flow *F, const double *aN, const double *aE, const double *aS, const double *aW,
                           const double *ap) {
-    Mg &M = F->mg;
-    LAUNCH(k_mg_setup0, mg_nblk(M.L[0]), F->g, aN, aE, aS, aW, ap, M.L[0]);
-    for (int l = 0; l + 1 < M.nlev; l++) LAUNCH(k_mg_coarsen, mg_nblk(M.L[l + 1]), M.L[l], M.L[l + 1]);
+    LAUNCH(k_mg_setup0, mg_nblk(F->mg.L[0]), F->g, aN, aE, aS, aW, ap, F->mg.L[0]);
+    mg_coarsen_levels(F);
 }
 static void mg_setup(cms2d_flow *F) {
     const St &s = F->s;
     mg_setup_from(F, s.aN, s.aE, s.aS, s.aW, F->Kpp.ap_w[0]);
 }
 
-// The level-0 launch of the cycle (down or up) with tile width TX.
-template <int TX, class TB>
-static void mg_level0_tx(cms2d_flow *F, KTimer *tm, bool down, const MgLevel &L0, const TB *b0, const KryScal *sc) {
-    using T = MTile<TX>;
-    const dim3 tiles((L0.nx + T::X - 1) / T::X, (L0.ny + T::Y - 1) / T::Y), tb(MT_THREADS);
-    if (down) tlaunch(tm, TG_MG_DOWN0, k_mg_down<TX, TB>, tiles, tb, 0, F->st, L0, b0, F->mg.L[1], sc);
-    else tlaunch(tm, TG_MG_UP0, k_mg_up<TX, TB>, tiles, tb, 0, F->st, L0, b0, F->mg.L[1], sc);
+// The launch of one level of the cycle (down or up) on tiles of TX x TY cells.
+template <int TX, int TY, int NT, class TB>
+static void mg_level_tile(cms2d_flow *F, KTimer *tm, bool down, const MgLevel &L, const TB *b, const MgLevel &C,
+                          const KryScal *sc) {
+    const dim3 tiles((L.nx + TX - 1) / TX, (L.ny + TY - 1) / TY), tb(NT);
+    if (down) tlaunch(tm, TG_MG_DOWN0, k_mg_down<TX, TY, NT, TB>, tiles, tb, 0, F->st, L, b, C, sc);
+    else tlaunch(tm, TG_MG_UP0, k_mg_up<TX, TY, NT, TB>, tiles, tb, 0, F->st, L, b, C, sc);
 }
 template <class TB>
 static void mg_level0(cms2d_flow *F, KTimer *tm, bool down, const MgLevel &L0, const TB *b0, const KryScal *sc) {
-    if (F->mg_tile == 64) mg_level0_tx<64>(F, tm, down, L0, b0, sc);
-    else if (F->mg_tile == 256) mg_level0_tx<256>(F, tm, down, L0, b0, sc);
-    else mg_level0_tx<128>(F, tm, down, L0, b0, sc);
+    const MgLevel &C = F->mg.L[1];
+    if (F->mg_tile == 64 && F->mg_tile_small) mg_level_tile<64, 8, 128>(F, tm, down, L0, b0, C, sc);
+    else if (F->mg_tile == 64) mg_level_tile<64, 32, 256>(F, tm, down, L0, b0, C, sc);
+    else if (F->mg_tile == 256) mg_level_tile<256, 8, 256>(F, tm, down, L0, b0, C, sc);
+    else mg_level_tile<128, 16, 256>(F, tm, down, L0, b0, C, sc);
+}
+// Levels 1 .. lt-1 (64 x 16 needs 400 workgroups to fill the chip: 5.7 us on
+// 750 000 cells, 6.6 with 64 x 8).
+static void mg_level(cms2d_flow *F, bool down, int l, const KryScal *sc) {
+    const MgLevel &L = F->mg.L[l], &C = F->mg.L[l + 1];
+    const float *b = L.b;
+    if ((long)L.nx * L.ny >= 400000) mg_level_tile<64, 16, 256>(F, nullptr, down, L, b, C, sc);
+    else mg_level_tile<64, 8, 128>(F, nullptr, down, L, b, C, sc);
+}
+// A thread per block of the tail's first level.
+static int mg_tail_threads(int nblk) { return nblk <= 256 ? 256 : nblk <= 512 ? 512 : MG_TAIL_NT; }
+template <class TB>
+static void mg_tail(cms2d_flow *F, const TB *b, float *zo, const KryScal *sc) {
+    const MgTail &T = F->mg.tail;
+    const int nt = mg_tail_threads(T.L[0].nblk);
+    const dim3 one(1), tb(nt);
+    if (nt == 256) hipLaunchKernelGGL((k_mg_tail<256, TB>), one, tb, T.lds, F->st, T, b, zo, sc);
+    else if (nt == 512) hipLaunchKernelGGL((k_mg_tail<512, TB>), one, tb, T.lds, F->st, T, b, zo, sc);
+    else hipLaunchKernelGGL((k_mg_tail<1024, TB>), one, tb, T.lds, F->st, T, b, zo, sc);
 }
 
 // z0 = V(b0): one V(1,1) cycle (mg.h) on the stream of F; every launch
@@ -499,37 +531,36 @@ static void mg_level0(cms2d_flow *F, KTimer *tm, bool down, const MgLevel &L0, c
 template <class TB>
 static void mg_vcycle(cms2d_flow *F, const TB *b0, float *z0, const KryScal *sc) {
     const Mg &M = F->mg;
-    MgLevel L0 = M.L[0];
-    L0.zo = z0;
-    const MgLevel &Lc = M.nlev == 1 ? L0 : M.L[M.nlev - 1];
-    const size_t lds = sizeof(float) * (size_t)Lc.nxp * (Lc.ny + 2);
-    KTimer *tm = F->tm_active;
-    if (M.nlev == 1) {
-        hipLaunchKernelGGL(k_mg_coarsest<TB>, dim3(1), dim3(MG_CT), lds, F->st, L0, b0, sc);
+    if (M.lt == 0) {
+        mg_tail(F, b0, z0, sc);
         return;
     }
+    MgLevel L0 = M.L[0];
+    L0.zo = z0;
+    KTimer *tm = F->tm_active;
     mg_level0(F, tm, true, L0, b0, sc);
     hipEvent_t ea, eb;
     const bool span = tm && tm->take(TG_MG_COARSE, ea, eb);
     if (span) (void)hipEventRecord(ea, F->st);
-    for (int l = 1; l + 1 < M.nlev; l++)
-        LAUNCH(k_mg_down_pc<float>, mg_nblk(M.L[l + 1]), M.L[l], (const float *)M.L[l].b, M.L[l + 1], sc);
-    hipLaunchKernelGGL(k_mg_coarsest<float>, dim3(1), dim3(MG_CT), lds, F->st, Lc, (const float *)Lc.b, sc);
-    for (int l = M.nlev - 2; l >= 1; l--)
-        LAUNCH(k_mg_up_pc<float>, mg_nblk(M.L[l + 1]), M.L[l], (const float *)M.L[l].b, M.L[l + 1], sc);
+    for (int l = 1; l < M.lt; l++) mg_level(F, true, l, sc);
+    mg_tail(F, (const float *)M.L[M.lt].b, M.L[M.lt].zo, sc);
+    for (int l = M.lt - 1; l >= 1; l--) mg_level(F, false, l, sc);
     if (span) (void)hipEventRecord(eb, F->st);
     mg_level0(F, tm, false, L0, b0, sc);
 }
 
-// Picks the level-0 tile width of the cycle by timing the down and up launches
-// of each candidate on this grid; every width gives the same values.
+// Picks the level-0 tile of the cycle by timing the down and up launches of
+// each candidate on this grid; every tile gives the same values.
 static int tune_mg_tile(cms2d_flow *F) {
-    static constexpr int cand[3] = {64, 128, 256};
-    if (F->mg.nlev < 2) return 0;
+    static constexpr struct { int tile, small; } cand[4] = {{64, 1}, {64, 0}, {128, 0}, {256, 0}};
+    F->mg_tile_small = F->g.nact < MG_SMALL_LEVEL0;
+    if (F->mg_tile_small) F->mg_tile = 64;
+    if (F->mg.lt == 0) return 0;
     if (const char *e = getenv("CMS2D_MG_TILE")) {   // fixed width (tests)
         const int t = atoi(e);
         if (t == 64 || t == 128 || t == 256) { F->mg_tile = t; return 0; }
     }
+    if (F->mg_tile_small) return 0;
     MgLevel L0 = F->mg.L[0];
     L0.zo = F->Kpp.zp;
     const double *b0 = F->Kpp.p[0];
@@ -538,9 +569,10 @@ static int tune_mg_tile(cms2d_flow *F) {
     HIPCHK(hipEventCreate(&ev[0]));
     HIPCHK(hipEventCreate(&ev[1]));
     float best = 0.0f;
-    int pick = F->mg_tile;
-    for (int t : cand) {
-        F->mg_tile = t;
+    int pick = 0;
+    for (int q = 0; q < 4; q++) {
+        F->mg_tile = cand[q].tile;
+        F->mg_tile_small = cand[q].small;
         mg_level0(F, nullptr, true, L0, b0, F->d_sc);          // warm-up
         mg_level0(F, nullptr, false, L0, b0, F->d_sc);
         HIPCHK(hipEventRecord(ev[0], F->st));
@@ -552,11 +584,12 @@ static int tune_mg_tile(cms2d_flow *F) {
         HIPCHK(hipEventSynchronize(ev[1]));
         float ms = 0.0f;
         HIPCHK(hipEventElapsedTime(&ms, ev[0], ev[1]));
-        if (t == cand[0] || ms < best) { best = ms; pick = t; }
+        if (q == 0 || ms < best) { best = ms; pick = q; }
     }
     (void)hipEventDestroy(ev[0]);
     (void)hipEventDestroy(ev[1]);
-    F->mg_tile = pick;
+    F->mg_tile = cand[pick].tile;
+    F->mg_tile_small = cand[pick].small;
     return 0;
 }
 
@@ -604,8 +637,7 @@ static KryCtx inner_ctx(const KryCtx &X) {
     return Xi;
 }
 static StencilOp32 inner_op(const cms2d_flow *F) {
-    const MgLevel &L0 = F->mg.L[0];
-    return StencilOp32{F->g, L0.aN, L0.aE, L0.aS, L0.aW};
+    return StencilOp32{F->g, F->mg.L[0].a};
 }
 
 // The pp solve of the FP32 form: FP32 BiCGStab (FP32 operator and vectors,
@@ -646,11 +678,10 @@ static int uv_solve_refine(cms2d_flow *F, KryCtx &X, StencilOp A) {
     const int nb = F->nblk_kry;
     hipLaunchKernelGGL((k_bicg_p<StencilOp, 2, double>), dim3(1), dim3(KBLOCK), 0, F->st, A, K, 0, nb, X.kmax,
                        X.rtol, X.atol, 1);
-    hipLaunchKernelGGL(k_uv_to32, dim3(nb), dim3(KBLOCK), 0, F->st, A, K, F->a32[0], F->a32[1], F->a32[2],
-                       F->a32[3], Ki);
+    hipLaunchKernelGGL(k_uv_to32, dim3(nb), dim3(KBLOCK), 0, F->st, A, K, F->a32, Ki);
     HIPCHK(hipMemcpyAsync(F->h_sc + 1, F->d_sc + 1, 2 * sizeof(KryScal), hipMemcpyDeviceToHost, F->st));
     HIPCHK(hipStreamSynchronize(F->st));
-    const StencilOp32 A32{F->g, F->a32[0], F->a32[1], F->a32[2], F->a32[3]};
+    const StencilOp32 A32{F->g, F->a32};
     KryCtx Xi = inner_ctx(X);
     Xi.rtol = REF_RTOL_UV;
     int total[2] = {0, 0};
@@ -743,7 +774,7 @@ static int capture_graphs(cms2d_flow *F) {
     const KryCtx X = flow_ctx(F, false);
     if (F->precision == CMS2D_PREC_FP32_REFINE) {
         // the inner FP32 pairs of the refinement form (u and v; pp)
-        const StencilOp32 A32{F->g, F->a32[0], F->a32[1], F->a32[2], F->a32[3]};
+        const StencilOp32 A32{F->g, F->a32};
         if (int rc = capture_bicg_pair<StencilOp32, 2, 0, float>(inner_ctx(X), F->Kin2, A32, F->kgraph[4])) return rc;
         if (int rc = capture_bicg_pair<StencilOp32, 1, 1, float>(inner_ctx(X), F->Kin, inner_op(F), F->kgraph[3],
                                                                  InnerPre{F}))
@@ -1083,33 +1114,129 @@ static int init_state(cms2d_flow *F) {
     return 0;
 }
 
-// Multigrid hierarchy on an nx x ny grid (level 0 in the padded layout of the
-// flow arrays): 2x2 coarsening until the coarsest fits one workgroup.
-static int mg_alloc(cms2d_flow *F, int nx, int ny) {
-    Mg &M = F->mg;
-    M.nlev = 0;
-    for (;;) {
-        MgLevel &L = M.L[M.nlev];
-        L.nx = nx; L.ny = ny; L.nxp = nx + 2;
-        const size_t n = (size_t)(nx + 2) * (ny + 2);
-        float **arrs[] = {&L.aN, &L.aE, &L.aS, &L.aW, &L.dinv, &L.e};
-        for (float **a : arrs)
-            if (int rc = dalloc(F, a, n)) return rc;
-        if (int rc = dalloc(F, &L.z, n)) return rc;
-        if (M.nlev > 0) {
-            if (int rc = dalloc(F, &L.zo, n)) return rc;
-            if (int rc = dalloc(F, &L.b, n)) return rc;
-        } else {
-            if (int rc = dalloc(F, &L.ap, n)) return rc;
+// The tail of the hierarchy if it began at level l (mg.h): its LDS layout, or
+// false if it does not fit the workgroup.
+static bool mg_tail_layout(const Mg &M, int l, MgTail &T) {
+    T = MgTail{};
+    T.n = M.nlev - l;
+    T.sweeps = M.sweeps;
+    T.w0 = M.w0;
+    T.w1 = M.w1;
+    T.lds1 = 1;
+    T.deep = T.n;
+    int nt = 0;                                        // threads (mg_tail)
+    if (T.n > MG_TAIL_LEVELS) return false;
+    size_t off = 0;                                    // floats
+    auto take = [&](size_t n) {
+        const size_t o = off;
+        off += n;
+        return (int)o;
+    };
+    for (int k = 0; k < T.n; k++) {
+        const MgLevel &L = M.L[l + k];
+        TailLev &V = T.L[k];
+        V.nx = L.nx; V.ny = L.ny; V.nxp = L.nxp; V.nbx = L.nbx;
+        V.nblk = L.nbx * ((L.ny + 1) / 2);
+        V.npad = L.nxp * (L.ny + 2);
+        V.a = L.a; V.dinv = L.dinv;
+        if (k == 0) nt = mg_tail_threads(V.nblk);
+        if (V.nblk > nt || 5 * (long)T.nlds > MG_TAIL_LDS) return false;
+        if (k == 1) T.lds1 = V.nblk > 64 ? 2 : 1;
+        if (k >= 1 && k >= T.lds1) {
+            if (V.nblk <= 64) T.deep = std::min(T.deep, k);
+            V.oa = 4 * T.nlds;                         // (levels side by side, 16-byte entries)
+            V.od = T.nlds;
+            T.nlds += V.npad;
         }
-        M.nlev++;
-        const bool fits = (long)nx * ny <= MG_COARSE_MAX && (long)(nx + 2) * (ny + 2) <= MG_COARSE_LDS;
-        if (fits && (M.nlev >= MG_MIN_LEVELS || (nx == 1 && ny == 1))) break;
-        if (M.nlev == MG_MAX_LEVELS) return set_err(CMS2D_ERR_ARG, "grid too large for the multigrid hierarchy");
-        nx = (nx + 1) / 2;
-        ny = (ny + 1) / 2;
     }
+    T.ga = T.L[0].a;
+    T.gd = T.L[0].dinv;
+    if (T.lds1 < T.n) {
+        T.ga = T.L[T.lds1].a;
+        T.gd = T.L[T.lds1].dinv;
+        for (int k = T.lds1; k < T.n; k++) T.L[k].od += 4 * T.nlds;
+        off = 5 * (size_t)T.nlds;
+    }
+    T.zero0 = (int)off;
+    for (int k = 0; k < T.n && off <= MG_TAIL_LDS; k++) {
+        TailLev &V = T.L[k];
+        // one more row: a block that hangs over an odd edge reads the row beyond the ring
+        V.oz = take((size_t)V.npad + V.nxp + 2);
+        if (k >= 1) V.ob = take(V.npad);
+    }
+    T.zero1 = (int)off;
+    T.lds = (unsigned)(off * sizeof(float));
+    return off * sizeof(float) <= MG_TAIL_LDS;
+}
+
+// Multigrid hierarchy on an nx x ny grid (level 0 in the padded layout of the
+// flow arrays), short or deep (mg.h); ratio: the off-diagonal coefficients of
+// level 0 over its storage term, 0 for the short one whatever it is.
+static int mg_alloc(cms2d_flow *F, int nx, int ny, double ratio) {
+    Mg &M = F->mg;
+    size_t ncoarse = 0;                                // padded cells of levels 1 ..
+    auto levels = [&](bool deep, double &r) -> int {
+        M.nlev = 0;
+        M.w0 = deep ? 0.5f : 1.0f;
+        M.w1 = deep ? 0.25f : 0.0f;
+        M.sweeps = deep ? MG_DEEP_SWEEPS : MG_SHORT_SWEEPS;
+        ncoarse = 0;
+        r = ratio;
+        for (int mx = nx, my = ny;; r *= 0.25) {
+            MgLevel &L = M.L[M.nlev];
+            L.nx = mx; L.ny = my; L.nxp = mx + 2; L.nbx = (mx + 1) / 2;
+            L.w0 = M.w0; L.w1 = M.w1;
+            if (M.nlev > 0) ncoarse += (size_t)(mx + 2) * (my + 2);
+            M.nlev++;
+            MgTail T;
+            const bool end = deep ? r <= MG_DEEP_RATIO : M.nlev >= MG_SHORT_LEVELS;
+            if (mg_tail_layout(M, M.nlev - 1, T) && (end || (mx == 1 && my == 1))) return 0;
+            if (M.nlev == MG_MAX_LEVELS) return set_err(CMS2D_ERR_ARG, "grid too large for the multigrid hierarchy");
+            mx = (mx + 1) / 2;
+            my = (my + 1) / 2;
+        }
+    };
+    double r;                                          // of the coarsest level
+    if (int rc = levels(false, r)) return rc;
+    if (r > MG_SHORT_RATIO)
+        if (int rc = levels(true, r)) return rc;
+    float4 *ac;
+    float *dc;
+    if (int rc = dalloc(F, &ac, ncoarse)) return rc;
+    if (int rc = dalloc(F, &dc, ncoarse)) return rc;
+    for (int l = 0; l < M.nlev; l++) {
+        MgLevel &L = M.L[l];
+        const size_t n = (size_t)L.nxp * (L.ny + 2);
+        if (int rc = dalloc(F, &L.e, n)) return rc;
+        if (int rc = dalloc(F, &L.zb, (size_t)L.nbx * L.ny)) return rc;
+        if (l == 0) {
+            if (int rc = dalloc(F, &L.a, n)) return rc;
+            if (int rc = dalloc(F, &L.dinv, n)) return rc;
+            if (int rc = dalloc(F, &L.ap, n)) return rc;
+            continue;
+        }
+        L.a = ac;
+        L.dinv = dc;
+        ac += n;
+        dc += n;
+        if (int rc = dalloc(F, &L.zo, n)) return rc;
+        if (int rc = dalloc(F, &L.b, n)) return rc;
+    }
+    for (M.lt = 0; !mg_tail_layout(M, M.lt, M.tail); M.lt++) {}
+    const void *tails[] = {(const void *)k_mg_tail<256, double>, (const void *)k_mg_tail<512, double>,
+                           (const void *)k_mg_tail<1024, double>, (const void *)k_mg_tail<256, float>,
+                           (const void *)k_mg_tail<512, float>, (const void *)k_mg_tail<1024, float>};
+    for (const void *k : tails)
+        HIPCHK(hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)MG_TAIL_LDS));
     return 0;
+}
+// g h dt^2 / dx^2 at the largest depth (bed below the datum plus the tide).
+static double mg_ratio(const cms2d_flow_desc *d, int ncells) {
+    double h = 0.0, amp = 0.0;
+    for (int c = 0; c < ncells; c++) h = std::max(h, -d->zb[c]);
+    for (int k = 0; k < d->ntc; k++) amp += std::fabs(d->amp[k]);
+    const double dx = std::min(d->dx, d->dy);
+    return GRAV * (h + amp) * d->dt * d->dt / (dx * dx);
 }
 
 static int create_impl(const cms2d_flow_desc *d, cms2d_flow *F) {
@@ -1349,7 +1476,7 @@ static int create_impl(const cms2d_flow_desc *d, cms2d_flow *F) {
     F->solver = d->solver;
     {
         Mg &M = F->mg;
-        if (int rc = mg_alloc(F, g.nx, g.ny)) return rc;
+        if (int rc = mg_alloc(F, g.nx, g.ny, d->precision == CMS2D_PREC_FP64 ? mg_ratio(d, g.nact) : 0.0)) return rc;
         if (int rc = dalloc(F, &F->Kpp.zp, N)) return rc;
         if (int rc = dalloc(F, &F->Kpp.zs, N)) return rc;
         KrySys<1, float> &Ki = F->Kin;
@@ -1382,8 +1509,7 @@ static int create_impl(const cms2d_flow_desc *d, cms2d_flow *F) {
                 for (float **v : vec)
                     if (int rc = dalloc(F, v, N)) return rc;
             }
-            for (int k = 0; k < 4; k++)
-                if (int rc = dalloc(F, &F->a32[k], N)) return rc;
+            if (int rc = dalloc(F, &F->a32, N)) return rc;
             double *ri;
             const size_t nbk = F->nblk_kry;
             if (int rc = dalloc(F, &ri, 2 * 5 * nbk)) return rc;
@@ -1846,7 +1972,7 @@ extern "C" int cms2d_flow_set_wind(cms2d_flow *F, double wndx, double wndy) {
 
 extern "C" int cms2d_flow_tuning(cms2d_flow *F, int *mg_tile_x, int *graphs) {
     if (!F || !mg_tile_x || !graphs) return set_err(CMS2D_ERR_ARG, "null argument");
-    *mg_tile_x = F->mg.nlev > 1 ? F->mg_tile : 0;
+    *mg_tile_x = F->mg.lt > 0 ? F->mg_tile : 0;
     *graphs = F->use_graphs ? 1 : 0;
     return CMS2D_OK;
 }

@@ -99,10 +99,9 @@ __device__ __forceinline__ void grid_walk(const Geo &g, F &&f) {
 
 // Matrix operators: y_i = ap_i z_i - sum_k a_k(i) z_nb(k).  apply() is the
 // Jacobi-preconditioned form, z = M^-1 x = x/ap with 1/ap stored (dinv), so
-// y_i = x_i - sum_k a_k(i) x_nb dinv_nb; z = 0 on ghost cells.  C is the type
-// of the coefficients and of the result.
-template <class C>
-struct StencilOpT {
+// y_i = x_i - sum_k a_k(i) x_nb dinv_nb; z = 0 on ghost cells.
+struct StencilOp {
+    using C = double;
     Geo g;
     const C *aN, *aE, *aS, *aW;
     __device__ __forceinline__ int n() const { return g.nact; }
@@ -139,8 +138,30 @@ struct StencilOpT {
         return ap[c] * (C)z[c] - sum;
     }
 };
-using StencilOp = StencilOpT<double>;
-using StencilOp32 = StencilOpT<float>;
+// The same operator in FP32, the four coefficients of a cell side by side (N, E, S, W).
+struct StencilOp32 {
+    Geo g;
+    const float4 *a;
+    __device__ __forceinline__ int n() const { return g.nact; }
+    template <class F>
+    __device__ __forceinline__ void each(F &&f) const { grid_walk(g, f); }
+    __device__ __forceinline__ float sum(const float *z, const float *dinv, const Idx &x) const {
+        const int c = x.c;
+        const int nb[4] = {c + g.nxp, c + 1, c - g.nxp, c - 1};
+        const bool in[4] = {x.j < g.ny - 1, x.i < g.nx - 1, x.j > 0, x.i > 0};
+        float v[4];
+#pragma unroll
+        for (int k = 0; k < 4; k++) v[k] = !in[k] ? 0.0f : dinv ? z[nb[k]] * dinv[nb[k]] : z[nb[k]];
+        const float4 q = a[c];
+        return ((q.x * v[0] + q.y * v[1]) + q.z * v[2]) + q.w * v[3];
+    }
+    __device__ __forceinline__ float apply(const float *xv, const float *dinv, const Idx &x) const {
+        return xv[x.c] - sum(xv, dinv, x);
+    }
+    __device__ __forceinline__ float apply_z(const float *z, const float *ap, const Idx &x) const {
+        return ap[x.c] * z[x.c] - sum(z, nullptr, x);
+    }
+};
 
 // The reference's general cell list: acoef(4,ncellsD) and cell2cell(4,ncellsD)
 // (0-based, ghosts numbered from ncells, -1 for no face).

@@ -351,11 +351,11 @@ __global__ void __launch_bounds__(KBLOCK) k_ref_update(Op A, KrySys<1, double> K
 
 // The u and v solves of the FP32 form (two systems, Jacobi): FP32 copies of
 // the shared coefficients and of each system's diagonal.
-__global__ void __launch_bounds__(KBLOCK) k_uv_to32(StencilOp A, KrySys<2, double> K, float *aN, float *aE, float *aS,
-                                                   float *aW, KrySys<2, float> Ki) {
+__global__ void __launch_bounds__(KBLOCK) k_uv_to32(StencilOp A, KrySys<2, double> K, float4 *a,
+                                                   KrySys<2, float> Ki) {
     A.each([&](const Idx &x) {
         const int c = x.c;
-        aN[c] = (float)A.aN[c]; aE[c] = (float)A.aE[c]; aS[c] = (float)A.aS[c]; aW[c] = (float)A.aW[c];
+        a[c] = make_float4((float)A.aN[c], (float)A.aE[c], (float)A.aS[c], (float)A.aW[c]);
 #pragma unroll
         for (int q = 0; q < 2; q++) {
             Ki.ap_w[q][c] = (float)K.ap_w[q][c];

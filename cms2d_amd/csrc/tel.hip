@@ -87,10 +87,7 @@ __global__ void __launch_bounds__(BLOCK) k_tl_mg_setup0(TelG T, const int *blk, 
     }
     const int c = L.idx(b % T.nbx, b / T.nbx);
     const double apb = es + ((a4[KN] + a4[KE]) + (a4[KS] + a4[KW]));
-    L.aN[c] = (float)a4[KN];
-    L.aE[c] = (float)a4[KE];
-    L.aS[c] = (float)a4[KS];
-    L.aW[c] = (float)a4[KW];
+    L.a[c] = make_float4((float)a4[KN], (float)a4[KE], (float)a4[KS], (float)a4[KW]);
     L.e[c] = (float)es;
     L.ap[c] = (float)apb;
     L.dinv[c] = apb > 0.0 ? (float)(1.0 / apb) : 0.0f;
@@ -634,8 +631,7 @@ static int tel_flow_imp(cms2d_flow *F) {
                 for (int k = 1; k < H.top; k++)
                     TLAUNCH(k_tl_cs_setup, tl_nblk(H.lv[k].nk), T, H.lv[k], (const double *)s.apc,
                             (const double *)H.Kpp.ap_w[0]);
-                for (int l = 0; l + 1 < F->mg.nlev; l++)
-                    LAUNCH(k_mg_coarsen, mg_nblk(F->mg.L[l + 1]), F->mg.L[l], F->mg.L[l + 1]);
+                mg_coarsen_levels(F);
                 if (F->precision == CMS2D_PREC_FP32_REFINE) {
                     if (int rc = tel_pp_solve_refine(F, X, Ap)) return rc;
                 } else {
@@ -1369,10 +1365,11 @@ static int tel_create(const cms2d_flow_desc *d, const cms2d_tel_grid *tg, cms2d_
             K2.sc = F->d_sc + 4;
         }
     }
-    if (int rc = mg_alloc(F, d->nx, d->ny)) return rc;
+    if (int rc = mg_alloc(F, d->nx, d->ny, 0.0)) return rc;
     if (int rc = dalloc(F, &F->mg.L[0].zo, (size_t)(d->nx + 2) * (d->ny + 2))) return rc;
     if (int rc = dalloc(F, &H.b0, (size_t)(d->nx + 2) * (d->ny + 2))) return rc;
-    F->mg_tile = 128;
+    F->mg_tile = d->nx * d->ny < MG_SMALL_LEVEL0 ? 64 : 128;
+    F->mg_tile_small = d->nx * d->ny < MG_SMALL_LEVEL0;
     if (const char *e = getenv("CMS2D_MG_TILE")) {
         const int tt = atoi(e);
         if (tt == 64 || tt == 128 || tt == 256) F->mg_tile = tt;

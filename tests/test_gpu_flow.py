@@ -102,6 +102,25 @@ def test_tidal_multigrid_levels_matches_oracle(gpu_available):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("precision", [_lib.PREC_FP64, _lib.PREC_FP32_REFINE])
+@pytest.mark.parametrize("shape", [(5, 4), (64, 64), (65, 64), (129, 9), (63, 71), (301, 8), (8, 517), (131, 135)],
+                         ids=lambda s: f"{s[0]}x{s[1]}")
+def test_multigrid_shapes_match_oracle(gpu_available, shape, precision):
+    """Shapes at the edges of the cycle's kernels: the largest first level of
+    the one-workgroup part (64 x 64) and one beyond it, one cell more or less
+    than a 64 x 8 tile, odd sides on every level, long strips; the deep
+    hierarchy (FP64: dx 10 m at dt 60 s) and the short one (FP32 form).  The
+    iteration bound is the cycle's quality: a wrong one still converges."""
+    nx, ny = shape
+    c = cases.basin(nx=nx, ny=ny, dx=10.0, seed=3, dt=60.0)
+    o, g = run_pair(c, 3, precision=precision)
+    compare(o, g)
+    info = g.step(0)
+    limit = 10 if precision == _lib.PREC_FP64 else 18
+    assert info["kry"][0] <= limit * info["niter"], info
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("shape", [(3, 3), (3, 40), (40, 3), (3, 5), (7, 3)],
                          ids=lambda s: f"{s[0]}x{s[1]}")
 def test_small_shapes_match_oracle(gpu_available, shape):
