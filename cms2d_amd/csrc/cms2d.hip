@@ -1359,7 +1359,10 @@ static int create_impl(const cms2d_flow_desc *d, cms2d_flow *F) {
     F->npad = g.nxp * g.nyp;
     F->nblk_act = (g.nact + BLOCK - 1) / BLOCK;
     F->nblk_pad = (F->npad + BLOCK - 1) / BLOCK;
-    F->nblk_kry = std::min(KRY_BLOCKS, F->nblk_act);
+    // a block per pass of the walk's rows where that is more (narrow grids: a
+    // 48 x 32 one walked three passes a block on 6 of them)
+    F->nblk_kry = std::min(KRY_BLOCKS, std::max(F->nblk_act, (g.nx + KW_STRIP - 1) / KW_STRIP *
+                                                                 ((g.ny + KW_ROWS - 1) / KW_ROWS)));
     F->use_graphs = true;
     if (const char *e = getenv("CMS2D_GRAPHS")) F->use_graphs = atoi(e) != 0;   // 0: direct launches, 1: graphs
     Par &P = F->P;

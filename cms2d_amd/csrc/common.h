@@ -61,6 +61,15 @@ __device__ __forceinline__ bool act_thread(const Geo &g, int &i, int &j, int &c)
     return true;
 }
 
+// A value that every lane of the wave holds, moved to scalar registers.
+__device__ __forceinline__ int uni(int v) { return __builtin_amdgcn_readfirstlane(v); }
+__device__ __forceinline__ double uni(double v) {
+    const unsigned long long b = __builtin_bit_cast(unsigned long long, v);
+    const unsigned lo = __builtin_amdgcn_readfirstlane((int)(unsigned)b);
+    const unsigned hi = __builtin_amdgcn_readfirstlane((int)(unsigned)(b >> 32));
+    return __builtin_bit_cast(double, (unsigned long long)hi << 32 | lo);
+}
+
 // --- deterministic reductions -------------------------------------------------
 template <int NV, int BS = BLOCK>
 __device__ __forceinline__ void block_sum(double (&v)[NV]) {

@@ -62,6 +62,26 @@ __device__ __forceinline__ Chunk block_chunk(int n) {
     return ch;
 }
 
+// Walk over the chunk.
+struct ChunkWalk {
+    int t, end;
+    __device__ __forceinline__ bool at(Idx &x) const {
+        x.c = t;
+        x.i = x.j = 0;
+        return t < end;
+    }
+    __device__ __forceinline__ explicit ChunkWalk(int n) {
+        const Chunk ch = block_chunk(n);
+        t = ch.begin + (int)threadIdx.x;
+        end = ch.end;
+    }
+    __device__ __forceinline__ bool first(Idx &x) { return at(x); }
+    __device__ __forceinline__ bool next(Idx &x) {
+        t += KBLOCK;
+        return at(x);
+    }
+};
+
 // Cells of this block on the fixed Krylov grid of a structured grid: strips
 // KW_STRIP columns wide; the rows of a strip go in groups of RP (one pass of
 // the block) to its blocks in turn, so in every pass the blocks of a strip
@@ -70,41 +90,59 @@ __device__ __forceinline__ Chunk block_chunk(int n) {
 // neighbours load at the same time and meet in that XCD's L2; a thread walks
 // one column.  Every active cell is visited once, whatever the grid size.
 constexpr int KW_STRIP = 256;
-template <class F>
-__device__ __forceinline__ void grid_walk(const Geo &g, F &&f) {
-    constexpr int RP = KBLOCK / KW_STRIP;                 // rows per pass
-    const int G = (int)gridDim.x;
-    const int sx = (g.nx + KW_STRIP - 1) / KW_STRIP;
-    const int bands = max(1, G / sx);                     // blocks per strip
-    const int nbx = G / bands;                            // strips in parallel (>= 1)
-    const int b = xcd_block(blockIdx.x, G);
-    const int bx = b / bands, by = b % bands;
-    if (bx >= nbx) return;
-    const int ngroups = (g.ny + RP - 1) / RP;
-    const int tx = (int)threadIdx.x % KW_STRIP, ty = (int)threadIdx.x / KW_STRIP;
-    for (int s = bx; s < sx; s += nbx) {
-        const int col = s * KW_STRIP + tx;
-        if (col >= g.nx) continue;
-        for (int grp = by; grp < ngroups; grp += bands) {
-            const int row = grp * RP + ty;
-            if (row >= g.ny) continue;
-            Idx x;
+constexpr int KW_ROWS = KBLOCK / KW_STRIP;                // rows per pass
+struct GridWalk {
+    const Geo &g;
+    int s, grp, nbx, by, bands, sx, ngroups, tx, ty;
+    __device__ __forceinline__ explicit GridWalk(const Geo &g_) : g(g_) {
+        const int G = (int)gridDim.x;
+        sx = (g.nx + KW_STRIP - 1) / KW_STRIP;
+        bands = max(1, G / sx);                           // blocks per strip
+        nbx = G / bands;                                  // strips in parallel (>= 1)
+        const int b = xcd_block(blockIdx.x, G);
+        s = b / bands;
+        by = grp = b % bands;
+        if (s >= nbx) s = sx;                             // no strip
+        ngroups = (g.ny + KW_ROWS - 1) / KW_ROWS;
+        tx = (int)threadIdx.x % KW_STRIP;
+        ty = (int)threadIdx.x / KW_STRIP;
+    }
+    // the walk's position, or the next one that is a cell
+    __device__ __forceinline__ bool first(Idx &x) {
+        for (; s < sx; s += nbx, grp = by) {
+            const int col = s * KW_STRIP + tx, row = grp * KW_ROWS + ty;
+            if (col >= g.nx || grp >= ngroups || row >= g.ny) continue;
             x.i = col;
             x.j = row;
             x.c = cidx(g, col, row);
-            f(x);
+            return true;
         }
+        return false;
     }
+    __device__ __forceinline__ bool next(Idx &x) {
+        grp += bands;
+        return first(x);
+    }
+};
+template <class F>
+__device__ __forceinline__ void grid_walk(const Geo &g, F &&f) {
+    GridWalk w(g);
+    Idx x;
+    for (bool ok = w.first(x); ok; ok = w.next(x)) f(x);
 }
 
 // Matrix operators: y_i = ap_i z_i - sum_k a_k(i) z_nb(k).  apply() is the
 // Jacobi-preconditioned form, z = M^-1 x = x/ap with 1/ap stored (dinv), so
-// y_i = x_i - sum_k a_k(i) x_nb dinv_nb; z = 0 on ghost cells.
+// y_i = x_i - sum_k a_k(i) x_nb dinv_nb; z = 0 on ghost cells, where the
+// vectors, z and dinv hold 0 (allocated so, written on active cells only): the
+// neighbours are read without a bounds test, whose branches would each wait
+// for their own load.
 struct StencilOp {
     using C = double;
     Geo g;
     const C *aN, *aE, *aS, *aW;
     __device__ __forceinline__ int n() const { return g.nact; }
+    __device__ __forceinline__ GridWalk walk() const { return GridWalk(g); }
     template <class F>
     __device__ __forceinline__ void each(F &&f) const { grid_walk(g, f); }
     __device__ __forceinline__ Idx at(int t) const {
@@ -114,15 +152,18 @@ struct StencilOp {
         x.c = cidx(g, x.i, x.j);
         return x;
     }
-    // V: the vectors' type (double; float in the inner solves of the FP32 form)
+    // of NS vectors at once (V: their type)
+    template <int NS, class V>
+    __device__ __forceinline__ void apply_n(const V *const (&xv)[NS], const V *const (&dinv)[NS], const Idx &x,
+                                            V (&y)[NS]) const {
+#pragma unroll
+        for (int q = 0; q < NS; q++) y[q] = apply(xv[q], dinv[q], x);
+    }
     template <class V>
     __device__ __forceinline__ V apply(const V *xv, const V *dinv, const Idx &x) const {
         const int c = x.c;
         const int cN = c + g.nxp, cE = c + 1, cS = c - g.nxp, cW = c - 1;
-        const V zN = x.j == g.ny - 1 ? V(0) : xv[cN] * dinv[cN];
-        const V zE = x.i == g.nx - 1 ? V(0) : xv[cE] * dinv[cE];
-        const V zS = x.j == 0 ? V(0) : xv[cS] * dinv[cS];
-        const V zW = x.i == 0 ? V(0) : xv[cW] * dinv[cW];
+        const V zN = xv[cN] * dinv[cN], zE = xv[cE] * dinv[cE], zS = xv[cS] * dinv[cS], zW = xv[cW] * dinv[cW];
         const V sum = (((V)aN[c] * zN + (V)aE[c] * zE) + (V)aS[c] * zS) + (V)aW[c] * zW;
         return xv[c] - sum;
     }
@@ -130,10 +171,7 @@ struct StencilOp {
     // vector z (FP32, zero on the ghost ring), evaluated in C.
     __device__ __forceinline__ C apply_z(const float *z, const C *ap, const Idx &x) const {
         const int c = x.c;
-        const C zN = x.j == g.ny - 1 ? C(0) : (C)z[c + g.nxp];
-        const C zE = x.i == g.nx - 1 ? C(0) : (C)z[c + 1];
-        const C zS = x.j == 0 ? C(0) : (C)z[c - g.nxp];
-        const C zW = x.i == 0 ? C(0) : (C)z[c - 1];
+        const C zN = (C)z[c + g.nxp], zE = (C)z[c + 1], zS = (C)z[c - g.nxp], zW = (C)z[c - 1];
         const C sum = ((aN[c] * zN + aE[c] * zE) + aS[c] * zS) + aW[c] * zW;
         return ap[c] * (C)z[c] - sum;
     }
@@ -143,20 +181,23 @@ struct StencilOp32 {
     Geo g;
     const float4 *a;
     __device__ __forceinline__ int n() const { return g.nact; }
+    __device__ __forceinline__ GridWalk walk() const { return GridWalk(g); }
     template <class F>
     __device__ __forceinline__ void each(F &&f) const { grid_walk(g, f); }
     __device__ __forceinline__ float sum(const float *z, const float *dinv, const Idx &x) const {
         const int c = x.c;
         const int nb[4] = {c + g.nxp, c + 1, c - g.nxp, c - 1};
-        const bool in[4] = {x.j < g.ny - 1, x.i < g.nx - 1, x.j > 0, x.i > 0};
         float v[4];
 #pragma unroll
-        for (int k = 0; k < 4; k++) v[k] = !in[k] ? 0.0f : dinv ? z[nb[k]] * dinv[nb[k]] : z[nb[k]];
+        for (int k = 0; k < 4; k++) v[k] = dinv ? z[nb[k]] * dinv[nb[k]] : z[nb[k]];
         const float4 q = a[c];
         return ((q.x * v[0] + q.y * v[1]) + q.z * v[2]) + q.w * v[3];
     }
-    __device__ __forceinline__ float apply(const float *xv, const float *dinv, const Idx &x) const {
-        return xv[x.c] - sum(xv, dinv, x);
+    template <int NS>
+    __device__ __forceinline__ void apply_n(const float *const (&xv)[NS], const float *const (&dinv)[NS], const Idx &x,
+                                            float (&y)[NS]) const {
+#pragma unroll
+        for (int q = 0; q < NS; q++) y[q] = xv[q][x.c] - sum(xv[q], dinv[q], x);
     }
     __device__ __forceinline__ float apply_z(const float *z, const float *ap, const Idx &x) const {
         return ap[x.c] * z[x.c] - sum(z, nullptr, x);
@@ -171,16 +212,12 @@ struct EllOp {
     const int *c2c;
     const double *a;
     __device__ __forceinline__ int n() const { return ncells; }
-    template <class F>
-    __device__ __forceinline__ void each(F &&f) const {
-        const Chunk ch = block_chunk(ncells);
-        for (int t = ch.begin + threadIdx.x; t < ch.end; t += KBLOCK) f(at(t));
-    }
-    __device__ __forceinline__ Idx at(int t) const {
-        Idx x;
-        x.c = t;
-        x.i = x.j = 0;
-        return x;
+    __device__ __forceinline__ ChunkWalk walk() const { return ChunkWalk(ncells); }
+    template <int NS>
+    __device__ __forceinline__ void apply_n(const double *const (&xv)[NS], const double *const (&dinv)[NS],
+                                            const Idx &x, double (&y)[NS]) const {
+#pragma unroll
+        for (int q = 0; q < NS; q++) y[q] = apply(xv[q], dinv[q], x);
     }
     __device__ __forceinline__ double apply(const double *xv, const double *dinv, const Idx &x) const {
         const int c = x.c;

@@ -18,14 +18,6 @@ namespace cms {
 #define SMALL F4(1.0e-15)
 #endif
 
-template <int NS, class T>
-__device__ __forceinline__ bool kdone(const KrySys<NS, T> &K) {
-#pragma unroll
-    for (int q = 0; q < NS; q++)
-        if (!K.sc[q].done) return false;
-    return true;
-}
-
 // solve() prologue for u (n=2) and v (n=3), relax(2)=relax(3)=0.8
 // (solvers.f90:232-240), then the BiCGStab start (pbicgstab.f90:21-31).
 __global__ void __launch_bounds__(KBLOCK) k_uv_prologue(Geo g, St s, KrySys<2> K) {
@@ -65,13 +57,50 @@ __global__ void __launch_bounds__(KBLOCK) k_uv_prologue(Geo g, St s, KrySys<2> K
     kry_reset(K.sc[1]);
 }
 
+// The five sweeps.  On a small grid a block makes one pass and a launch lasts
+// as long as its longest chain of loads, so each kernel issues the loads of its
+// first cell, of the stopping flags and of the scalars before it sums the
+// partials and before it tests a flag; only the stores wait for those (in
+// turn, flag, partials, scalars and operands took 1.5-2 us more per launch).
+
 // Finishes iteration it-1 (or starts the solve when it == 0) and, unless
 // fin_only, updates p.  Launched with fin_only on one block at the end of a
 // batch so the host can read the state; the next batch repeats the same
 // finish (same inputs, same result) before its first p update.
 template <class Op, int NS, class T = double>
-__global__ void __launch_bounds__(KBLOCK) k_bicg_p(Op A, KrySys<NS, T> K, int it, int nb, int kmax, double rtol,
+__global__ void __launch_bounds__(KBLOCK, NS == 2 ? 8 : 1) k_bicg_p(Op A, KrySys<NS, T> K, int it, int nb, int kmax, double rtol,
                                                   double atol, int fin_only) {
+    auto w = A.walk();
+    Idx x;
+    T r[NS], p[NS], v[NS];
+    auto load = [&]() {
+#pragma unroll
+        for (int q = 0; q < NS; q++) {
+            r[q] = K.r[q][x.c];
+            p[q] = v[q] = T(0);
+        }
+        // the first iteration starts from p = r (p and v of an earlier solve are not read)
+        if (it > 0)
+#pragma unroll
+            for (int q = 0; q < NS; q++) {
+                p[q] = K.p[q][x.c];
+                v[q] = K.v[q][x.c];
+            }
+    };
+    // (two systems' operands and scalars together exceed the registers of eight
+    // waves a SIMD: there they are loaded after the sums)
+    constexpr bool PRE = NS == 1;
+    bool ok = !fin_only && w.first(x);
+    if (PRE && ok) load();
+    const int pq = (it - 1) & 1, cq = it & 1;
+    int sdone[NS], siter[NS];
+    double sthr[NS], srho[NS], sr0n[NS], salp[NS], somg[NS];
+    auto scalars = [&](int q) {
+        const KryScal &sc = K.sc[q];
+        sdone[q] = sc.done; siter[q] = sc.iters[pq]; sthr[q] = sc.thr; srho[q] = sc.rho[pq];
+        sr0n[q] = sc.r0n[pq]; salp[q] = sc.alpha[pq]; somg[q] = sc.omega[pq];
+    };
+    if (PRE) scalars(0);
     double tot[2 * NS];
     const double *src[2 * NS];
 #pragma unroll
@@ -85,8 +114,9 @@ __global__ void __launch_bounds__(KBLOCK) k_bicg_p(Op A, KrySys<NS, T> K, int it
     for (int q = 0; q < NS; q++) {
         KryScal &sc = K.sc[q];
         act[q] = false; rst[q] = 0; beta[q] = 0.0; om[q] = 1.0;
-        if (sc.done) continue;
-        const double rr = tot[2 * q], nr = sqrt(rr);
+        if (!PRE) scalars(q);
+        if (uni(sdone[q])) continue;
+        const double rr = uni(tot[2 * q]), nr = uni(sqrt(rr));
         if (it == 0) {
             const double thr = fmax(rtol * nr, atol * sqrt((double)A.n()));
             act[q] = !(nr <= thr);
@@ -100,17 +130,16 @@ __global__ void __launch_bounds__(KBLOCK) k_bicg_p(Op A, KrySys<NS, T> K, int it
                 if (!act[q]) { sc.done = 1; sc.final_iters = 0; }
             }
         } else {
-            const int pq = (it - 1) & 1, cq = it & 1;
-            const double r0r = tot[2 * q + 1];
-            const int iters = sc.iters[pq] + 1;
-            const double rho_p = sc.rho[pq], r0n_p = sc.r0n[pq], al = sc.alpha[pq], omp = sc.omega[pq];
+            const double r0r = uni(tot[2 * q + 1]);
+            const int iters = uni(siter[q]) + 1;
+            const double rho_p = uni(srho[q]), r0n_p = uni(sr0n[q]), al = uni(salp[q]), omp = uni(somg[q]);
             double rho = rho_p, r0n = r0n_p;
-            if (omp == 0.0 || nr <= sc.thr || iters >= kmax) {
+            if (omp == 0.0 || nr <= uni(sthr[q]) || iters >= kmax) {
                 act[q] = false;
             } else if (fabs(r0r) <= 1e-12 * nr * r0n_p) {
                 rst[q] = 1; rho = rr; r0n = nr; beta[q] = 0.0; act[q] = true;
             } else {
-                beta[q] = (r0r / rho_p) * (al / omp); rho = r0r; act[q] = true;
+                beta[q] = uni((r0r / rho_p) * (al / omp)); rho = r0r; act[q] = true;
             }
             om[q] = omp;
             if (lead()) {
@@ -122,18 +151,18 @@ __global__ void __launch_bounds__(KBLOCK) k_bicg_p(Op A, KrySys<NS, T> K, int it
         }
         any = any || act[q];
     }
-    if (fin_only || !any) return;
-    A.each([&](const Idx &x_) {
-        const int c = x_.c;
+    if (!any) return;
+    if (!PRE && ok) load();
+    while (ok) {
 #pragma unroll
         for (int q = 0; q < NS; q++) {
             if (!act[q]) continue;
-            const T r = K.r[q][c];
-            if (rst[q]) K.r0[q][c] = r;
-            // the first iteration starts from p = r (p and v of an earlier solve are not read)
-            K.p[q][c] = it == 0 ? r : r + (T)beta[q] * (K.p[q][c] - (T)om[q] * K.v[q][c]);
+            if (rst[q]) K.r0[q][x.c] = r[q];
+            K.p[q][x.c] = it == 0 ? r[q] : r[q] + (T)beta[q] * (p[q] - (T)om[q] * v[q]);
         }
-    });
+        ok = w.next(x);
+        if (ok) load();
+    }
 }
 
 // MODE 1: v = A M^-1 p, partials r0.v.  MODE 2: t = A M^-1 s (s held in r),
@@ -141,34 +170,55 @@ __global__ void __launch_bounds__(KBLOCK) k_bicg_p(Op A, KrySys<NS, T> K, int it
 template <class Op, int NS, int MODE, int PREC = 0, class T = double>
 __global__ void __launch_bounds__(KBLOCK) k_bicg_spmv(Op A, KrySys<NS, T> K) {
     static_assert(PREC == 0 || NS == 1, "explicit preconditioner: one system");
-    if (kdone(K)) return;
     constexpr int NV = MODE == 1 ? NS : 2 * NS;
     double red[NV];
 #pragma unroll
     for (int q = 0; q < NV; q++) red[q] = 0.0;
     bool act[NS];
+    bool any = false;
+    auto w = A.walk();
+    Idx x;
+    T y[NS], m[NS];                       // A z and the vector of its product r0 or s
+    const T *xv[NS], *dinv[NS];
 #pragma unroll
-    for (int q = 0; q < NS; q++) act[q] = !K.sc[q].done;
-    A.each([&](const Idx &x) {
-        const int c = x.c;
+    for (int q = 0; q < NS; q++) {
+        xv[q] = MODE == 1 ? K.p[q] : K.r[q];
+        dinv[q] = K.dinv_w[q];
+    }
+    auto row = [&]() {
+        if constexpr (PREC == 1) y[0] = A.apply_z(MODE == 1 ? K.zp : K.zs, K.ap_w[0], x);
+        else A.apply_n(xv, dinv, x, y);
+#pragma unroll
+        for (int q = 0; q < NS; q++) m[q] = MODE == 1 ? K.r0[q][x.c] : xv[q][x.c];
+    };
+    int done[NS];
+#pragma unroll
+    for (int q = 0; q < NS; q++) done[q] = K.sc[q].done;
+    bool ok = w.first(x);
+    if (ok) row();
+#pragma unroll
+    for (int q = 0; q < NS; q++) {
+        act[q] = !uni(done[q]);
+        any = any || act[q];
+    }
+    if (!any) return;
+    while (ok) {
 #pragma unroll
         for (int q = 0; q < NS; q++) {
             if (!act[q]) continue;
-            const T *xv = MODE == 1 ? K.p[q] : K.r[q];
-            T y;
-            if constexpr (PREC == 1) y = A.apply_z(MODE == 1 ? K.zp : K.zs, K.ap_w[q], x);
-            else y = A.apply(xv, K.dinv_w[q], x);
-            const double yd = y;
+            const double yd = y[q];
             if (MODE == 1) {
-                K.v[q][c] = y;
-                red[q] += (double)K.r0[q][c] * yd;
+                K.v[q][x.c] = y[q];
+                red[q] += (double)m[q] * yd;
             } else {
-                K.t[q][c] = y;
-                red[2 * q] += yd * (double)xv[c];
+                K.t[q][x.c] = y[q];
+                red[2 * q] += yd * (double)m[q];
                 red[2 * q + 1] += yd * yd;
             }
         }
-    });
+        ok = w.next(x);
+        if (ok) row();
+    }
     double *dst[NV];
 #pragma unroll
     for (int q = 0; q < NS; q++) {
@@ -182,7 +232,22 @@ __global__ void __launch_bounds__(KBLOCK) k_bicg_spmv(Op A, KrySys<NS, T> K) {
 // PREC 1 defers the x update to k_bicg_r.
 template <class Op, int NS, int PREC = 0, class T = double>
 __global__ void __launch_bounds__(KBLOCK) k_bicg_s(Op A, KrySys<NS, T> K, int it, int nb) {
-    if (kdone(K)) return;
+    auto w = A.walk();
+    Idx x;
+    T r[NS], v[NS], p[NS], d[NS], xs[NS];
+    auto load = [&](int q) {
+        r[q] = K.r[q][x.c];
+        v[q] = K.v[q][x.c];
+        if constexpr (PREC == 0) { p[q] = K.p[q][x.c]; d[q] = K.dinv_w[q][x.c]; xs[q] = K.x[q][x.c]; }
+    };
+    bool ok = w.first(x);
+    if (ok)
+#pragma unroll
+        for (int q = 0; q < NS; q++) load(q);
+    const int cq = it & 1;
+    struct { int done, iters; double rho; } pre[NS];
+#pragma unroll
+    for (int q = 0; q < NS; q++) pre[q] = {K.sc[q].done, K.sc[q].iters[cq], K.sc[q].rho[cq]};
     double tot[NS];
     const double *src[NS];
 #pragma unroll
@@ -191,39 +256,61 @@ __global__ void __launch_bounds__(KBLOCK) k_bicg_s(Op A, KrySys<NS, T> K, int it
     bool act[NS];
     double al[NS];
     bool any = false;
-    const int cq = it & 1;
 #pragma unroll
     for (int q = 0; q < NS; q++) {
         KryScal &sc = K.sc[q];
-        act[q] = !sc.done;
+        act[q] = !uni(pre[q].done);
         al[q] = 0.0;
         if (!act[q]) continue;
-        if (tot[q] == 0.0) {                       // r0.v = 0: stop before the update
+        if (uni(tot[q]) == 0.0) {                       // r0.v = 0: stop before the update
             act[q] = false;
-            if (lead()) { sc.done = 1; sc.final_iters = sc.iters[cq]; }
+            if (lead()) { sc.done = 1; sc.final_iters = pre[q].iters; }
             continue;
         }
-        al[q] = sc.rho[cq] / tot[q];
+        al[q] = uni(pre[q].rho / tot[q]);
         if (lead()) sc.alpha[cq] = al[q];
         any = true;
     }
     if (!any) return;
-    A.each([&](const Idx &x_) {
-        const int c = x_.c;
+    while (ok) {
 #pragma unroll
         for (int q = 0; q < NS; q++) {
             if (!act[q]) continue;
-            if constexpr (PREC == 0) K.x[q][c] = K.x[q][c] + al[q] * (K.p[q][c] * K.dinv_w[q][c]);
-            K.r[q][c] = K.r[q][c] - (T)al[q] * K.v[q][c];
+            if constexpr (PREC == 0) K.x[q][x.c] = xs[q] + al[q] * (p[q] * d[q]);
+            K.r[q][x.c] = r[q] - (T)al[q] * v[q];
         }
-    });
+        ok = w.next(x);
+        if (ok)
+#pragma unroll
+            for (int q = 0; q < NS; q++)
+                if (act[q]) load(q);
+    }
 }
 
 // omega = t.s / t.t ; x += omega M^-1 s ; r = s - omega t ; partials r.r, r0.r
 // PREC 1: x += alpha zp + omega zs.
 template <class Op, int NS, int PREC = 0, class T = double>
 __global__ void __launch_bounds__(KBLOCK) k_bicg_r(Op A, KrySys<NS, T> K, int it, int nb) {
-    if (kdone(K)) return;
+    auto w = A.walk();
+    Idx x;
+    T sv[NS], t[NS], d[NS], xs[NS], r0[NS];
+    float zp = 0.0f, zs = 0.0f;
+    auto load = [&](int q) {
+        sv[q] = K.r[q][x.c];
+        t[q] = K.t[q][x.c];
+        xs[q] = K.x[q][x.c];
+        r0[q] = K.r0[q][x.c];
+        if constexpr (PREC == 1) { zp = K.zp[x.c]; zs = K.zs[x.c]; }
+        else d[q] = K.dinv_w[q][x.c];
+    };
+    bool ok = w.first(x);
+    if (ok)
+#pragma unroll
+        for (int q = 0; q < NS; q++) load(q);
+    const int cq = it & 1;
+    struct { int done; double alpha; } pre[NS];
+#pragma unroll
+    for (int q = 0; q < NS; q++) pre[q] = {K.sc[q].done, K.sc[q].alpha[cq]};
     double tot[2 * NS];
     const double *src[2 * NS];
 #pragma unroll
@@ -231,47 +318,50 @@ __global__ void __launch_bounds__(KBLOCK) k_bicg_r(Op A, KrySys<NS, T> K, int it
     sum_partials<2 * NS>(src, nb, tot);
     bool act[NS];
     double om[NS], al[NS];
-    const int cq = it & 1;
+    bool any = false;
 #pragma unroll
     for (int q = 0; q < NS; q++) {
-        act[q] = !K.sc[q].done;
+        act[q] = !uni(pre[q].done);
         const double ts = tot[2 * q], tt = tot[2 * q + 1];
-        om[q] = tt > 0.0 ? ts / tt : 0.0;
-        al[q] = K.sc[q].alpha[cq];
+        om[q] = uni(tt > 0.0 ? ts / tt : 0.0);
+        al[q] = uni(pre[q].alpha);
         if (act[q] && lead()) K.sc[q].omega[cq] = om[q];
+        any = any || act[q];
     }
+    if (!any) return;
     double red[2 * NS];
 #pragma unroll
     for (int q = 0; q < 2 * NS; q++) red[q] = 0.0;
-    A.each([&](const Idx &x_) {
-        const int c = x_.c;
+    while (ok) {
 #pragma unroll
         for (int q = 0; q < NS; q++) {
             if (!act[q]) continue;
-            const T sv = K.r[q][c];
-            if constexpr (PREC == 1)
-                K.x[q][c] = K.x[q][c] + ((T)al[q] * (T)K.zp[c] + (T)om[q] * (T)K.zs[c]);
-            else
-                K.x[q][c] = K.x[q][c] + om[q] * (sv * K.dinv_w[q][c]);
-            const T r = sv - (T)om[q] * K.t[q][c];
-            K.r[q][c] = r;
+            if constexpr (PREC == 1) K.x[q][x.c] = xs[q] + ((T)al[q] * (T)zp + (T)om[q] * (T)zs);
+            else K.x[q][x.c] = xs[q] + om[q] * (sv[q] * d[q]);
+            const T r = sv[q] - (T)om[q] * t[q];
+            K.r[q][x.c] = r;
             red[2 * q] += (double)r * (double)r;
-            red[2 * q + 1] += (double)K.r0[q][c] * (double)r;
+            red[2 * q + 1] += (double)r0[q] * (double)r;
         }
-    });
+        ok = w.next(x);
+        if (ok)
+#pragma unroll
+            for (int q = 0; q < NS; q++)
+                if (act[q]) load(q);
+    }
     double *dst[2 * NS];
 #pragma unroll
     for (int q = 0; q < NS; q++) { dst[2 * q] = K.red.pr[q]; dst[2 * q + 1] = K.red.pr[q] + gridDim.x; }
     put_partials<2 * NS>(red, dst);
 }
 
-// solve() prologue on the reference's general cell list (solvers.f90:232-240)
-// and the BiCGStab start, for the drop-in cms2d_solve.
 // Clears n 32-bit words with vector stores (used instead of a memset node).
 __global__ void k_zero_words(unsigned int *p, int n) {
     for (int i = threadIdx.x; i < n; i += blockDim.x) p[i] = 0u;
 }
 
+// solve() prologue on the reference's general cell list (solvers.f90:232-240)
+// and the BiCGStab start, for the drop-in cms2d_solve.
 // bias: the reference's small number added to the starting residual
 // (pbicgstab.f90), 0 for the transposed solve of the adjoint, which must stay
 // linear in its right-hand side.

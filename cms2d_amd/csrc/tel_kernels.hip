@@ -602,41 +602,85 @@ struct TelOpT {
     const uint64_t *meta;
     const CA *a;                 // [TF*nd]
     __device__ __forceinline__ int n() const { return nc; }
-    __device__ __forceinline__ Idx at(int t) const {
-        Idx x;
-        x.c = t;
-        x.i = x.j = 0;
-        return x;
-    }
     // Passes over the list in order: in pass p the blocks take consecutive
     // runs of KBLOCK cells from p * gridDim.x * KBLOCK on, consecutive blocks
     // on one XCD (xcd_block), so the cells a row above and below (a few
     // thousand entries away) are read by that XCD's blocks in the same pass.
+    struct Walk {
+        int t, nc;
+        __device__ __forceinline__ bool first(Idx &x) const {
+            x.c = t;
+            x.i = x.j = 0;
+            return t < nc;
+        }
+        __device__ __forceinline__ bool next(Idx &x) {
+            t += (int)gridDim.x * KBLOCK;
+            return first(x);
+        }
+    };
+    __device__ __forceinline__ Walk walk() const {
+        return Walk{xcd_block(blockIdx.x, gridDim.x) * KBLOCK + (int)threadIdx.x, nc};
+    }
     template <class F>
     __device__ __forceinline__ void each(F &&f) const {
-        const int b = xcd_block(blockIdx.x, gridDim.x);
-        for (int t = b * KBLOCK + (int)threadIdx.x; t < nc; t += (int)gridDim.x * KBLOCK) f(at(t));
+        Walk w = walk();
+        Idx x;
+        for (bool ok = w.first(x); ok; ok = w.next(x)) f(x);
+    }
+    // sum_k a_k z_nb of NS vectors, get(q, nb) the value of vector q at an
+    // active neighbour: the neighbour indices and coefficients are loaded once
+    // for all of them, four slots at a time without a branch between (slots
+    // past the last face and ghosts read cell c with coefficient 0), the slots
+    // of joint cells after them.
+    template <int NS, class V, class Get>
+    __device__ __forceinline__ void sums(int c, Get &&get, V (&sum)[NS]) const {
+        const int nf = m_ncf(meta[c]);
+        int nb[4];
+        V w[4];
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            nb[k] = c2c[k * nd + c];
+            w[k] = (V)a[k * nd + c];
+        }
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            const bool in = k < nf && nb[k] < nc;
+            nb[k] = in ? nb[k] : c;
+            w[k] = in ? w[k] : V(0);
+        }
+        V z[NS][4];
+#pragma unroll
+        for (int q = 0; q < NS; q++)
+#pragma unroll
+            for (int k = 0; k < 4; k++) z[q][k] = get(q, nb[k]);
+#pragma unroll
+        for (int q = 0; q < NS; q++) {
+            sum[q] = w[0] * z[q][0];
+#pragma unroll
+            for (int k = 1; k < 4; k++) sum[q] += w[k] * z[q][k];
+        }
+        for (int k = 4; k < nf; k++) {
+            const int j = c2c[k * nd + c];
+            if (j >= nc) continue;
+            const V wk = (V)a[k * nd + c];
+#pragma unroll
+            for (int q = 0; q < NS; q++) sum[q] += wk * get(q, j);
+        }
     }
     // V: the vectors' type (double; float in the inner solves of the FP32 form)
-    template <class V>
-    __device__ __forceinline__ V apply(const V *xv, const V *dinv, const Idx &x) const {
-        const int c = x.c, nf = m_ncf(meta[c]);
-        V sum = V(0);
-        for (int k = 0; k < nf; k++) {
-            const int nb = c2c[k * nd + c];
-            if (nb < nc) sum += (V)a[k * nd + c] * (xv[nb] * dinv[nb]);
-        }
-        return xv[c] - sum;
+    template <int NS, class V>
+    __device__ __forceinline__ void apply_n(const V *const (&xv)[NS], const V *const (&dinv)[NS], const Idx &x,
+                                            V (&y)[NS]) const {
+        V sum[NS];
+        sums<NS, V>(x.c, [&](int q, int nb) { return xv[q][nb] * dinv[q][nb]; }, sum);
+#pragma unroll
+        for (int q = 0; q < NS; q++) y[q] = xv[q][x.c] - sum[q];
     }
     template <class C>
     __device__ __forceinline__ C apply_z(const float *z, const C *ap, const Idx &x) const {
-        const int c = x.c, nf = m_ncf(meta[c]);
-        C sum = C(0);
-        for (int k = 0; k < nf; k++) {
-            const int nb = c2c[k * nd + c];
-            if (nb < nc) sum += (C)a[k * nd + c] * (C)z[nb];
-        }
-        return ap[c] * (C)z[c] - sum;
+        C sum[1];
+        sums<1, C>(x.c, [&](int, int nb) { return (C)z[nb]; }, sum);
+        return ap[x.c] * (C)z[x.c] - sum[0];
     }
 };
 using TelOp = TelOpT<double>;
