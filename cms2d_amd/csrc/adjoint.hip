@@ -176,16 +176,33 @@ static int adj_solved(cms2d_flow *F, int sc0, int ns, const char *what) {
     return 0;
 }
 
-static KryCtx adj_ctx(cms2d_flow *F) {
+// The transposed solves of one adjoint call: their iteration pairs, captured at
+// the first reverse iteration (the operators' and solutions' arrays are those of
+// the call), and the counts they took (as prev_iters of the flow).
+struct RevSolves {
+    hipGraphExec_t graph[6]{};
+    int prev[PREV_OUTER][6]{};
+    int last[6]{8, 4, 4, 8, 4, 4};
+    RevSolves() = default;
+    RevSolves(const RevSolves &) = delete;
+    RevSolves &operator=(const RevSolves &) = delete;
+    ~RevSolves() {
+        for (auto &ge : graph)
+            if (ge) (void)hipGraphExecDestroy(ge);
+    }
+};
+static KryCtx adj_ctx(cms2d_flow *F, RevSolves &R, int it) {
     KryCtx X = flow_ctx(F, false);
-    X.graph = nullptr;
+    X.graph = F->use_graphs ? R.graph : nullptr;
+    X.prev_iters = R.prev[std::min(it, PREV_OUTER - 1)];
+    X.last_iters = R.last;
     X.atol = 0.0;    // relative stop only: the adjoint right-hand sides can be small
     return X;
 }
 
 // Reverse of one outer iteration: T the state at its start, E at its end, M
 // its recorded intermediate values.
-static int rev_iter(cms2d_flow *F, Ad &A, const St &T, const St &E, const Mid &M) {
+static int rev_iter(cms2d_flow *F, Ad &A, RevSolves &R, int it, const St &T, const St &E, const Mid &M) {
     const Geo &g = F->g;
     const Par &P = F->P;
     const int nbp = F->nblk_pad, nba = F->nblk_act;
@@ -199,7 +216,7 @@ static int rev_iter(cms2d_flow *F, Ad &A, const St &T, const St &E, const Mid &M
     LAUNCH(k_r_pvfc2, nbp, g, T, (const double *)M.ppv, P, A);
     LAUNCH(k_r_pvfc1, nba, g, T, M, A);
     // pp: A^T lambda = dL/dpp
-    KryCtx X = adj_ctx(F);
+    KryCtx X = adj_ctx(F, R, it);
     {
         LAUNCH(k_r_transpose, nba, g, (const double *)M.ap[0], (const double *)M.ap[1], (const double *)M.ap[2],
                (const double *)M.ap[3], A);
@@ -209,6 +226,8 @@ static int rev_iter(cms2d_flow *F, Ad &A, const St &T, const St &E, const Mid &M
         hipLaunchKernelGGL(k_r_start<1>, dim3(F->nblk_kry), dim3(KBLOCK), 0, F->st, g, K, S);
         mg_setup_from(F, A.tN, A.tE, A.tS, A.tW, K.ap_w[0]);
         const StencilOp At{g, A.tN, A.tE, A.tS, A.tW};
+        if (X.graph && !R.graph[0])
+            if (int rc = capture_bicg_pair<StencilOp, 1, 1, double>(X, K, At, R.graph[0], PpPre{F})) return rc;
         if (int rc = run_bicg<StencilOp, 1, 1, double>(X, K, At, 0, PpPre{F})) return rc;
         if (int rc = adj_solved(F, 0, 1, "pp")) return rc;
     }
@@ -226,6 +245,8 @@ static int rev_iter(cms2d_flow *F, Ad &A, const St &T, const St &E, const Mid &M
         AdjStart<2> S{M.au[0], M.au[1], M.au[2], M.au[3], {M.spu, M.spv}, {A.u, A.v}, 1.0 / F4(0.8)};
         hipLaunchKernelGGL(k_r_start<2>, dim3(F->nblk_kry), dim3(KBLOCK), 0, F->st, g, K, S);
         const StencilOp At{g, A.tN, A.tE, A.tS, A.tW};
+        if (X.graph && !R.graph[1])
+            if (int rc = capture_bicg_pair<StencilOp, 2, 0, double>(X, K, At, R.graph[1])) return rc;
         if (int rc = run_bicg<StencilOp, 2, 0, double>(X, K, At, 1)) return rc;
         if (int rc = adj_solved(F, 1, 2, "u/v")) return rc;
     }
@@ -236,7 +257,7 @@ static int rev_iter(cms2d_flow *F, Ad &A, const St &T, const St &E, const Mid &M
 
 // Reverse of one time step recorded in the tape; geta: dL/deta of the gauges
 // after this step (device, ng values).
-static int rev_step(cms2d_flow *F, Ad &A, Tape &tp, const int *cells, int ng, const double *geta) {
+static int rev_step(cms2d_flow *F, Ad &A, RevSolves &R, Tape &tp, const int *cells, int ng, const double *geta) {
     const Geo &g = F->g;
     const Par &P = F->P;
     const int nbp = F->nblk_pad, nba = F->nblk_act;
@@ -246,7 +267,7 @@ static int rev_step(cms2d_flow *F, Ad &A, Tape &tp, const int *cells, int ng, co
     LAUNCH(k_r_velface, nba, g, S, P, A);
     for (int it = tp.niter - 1; it >= 0; it--) {
         const St T = snap_view(F, tp.snap[it]), E = snap_view(F, tp.snap[it + 1]);
-        if (int rc = rev_iter(F, A, T, E, mid_view(F, tp.mid[it]))) return rc;
+        if (int rc = rev_iter(F, A, R, it, T, E, mid_view(F, tp.mid[it]))) return rc;
     }
     const St T0 = snap_view(F, tp.snap[0]);
     LAUNCH(k_r_srcsnk, nba, g, T0, P, A);
@@ -348,6 +369,7 @@ extern "C" int cms2d_flow_adjoint(cms2d_flow *F, int nsteps, int every, int ngau
     HIPCHK(hipMalloc((void **)&mem.ad, (size_t)AD_NARRAYS * F->npad * sizeof(double)));
     HIPCHK(hipMemsetAsync(mem.ad, 0, (size_t)AD_NARRAYS * F->npad * sizeof(double), F->st));
     Ad A = ad_view(F, mem.ad);
+    RevSolves rev;
     mem.ss.resize(std::min(every, nsteps));
     for (int s = ncp - 1; s >= 0; s--) {
         const int n0 = s * every, n1 = std::min(nsteps, n0 + every);
@@ -363,7 +385,7 @@ extern "C" int cms2d_flow_adjoint(cms2d_flow *F, int nsteps, int every, int ngau
             const int rc = step_once(F);
             F->tape = nullptr;
             if (rc) { restore0(); return rc; }
-            if (int r2 = rev_step(F, A, mem.tape, mem.cells, ngauge, mem.geta + (size_t)n * ng)) {
+            if (int r2 = rev_step(F, A, rev, mem.tape, mem.cells, ngauge, mem.geta + (size_t)n * ng)) {
                 restore0();
                 return r2;
             }

@@ -129,6 +129,9 @@ namespace cms {
 struct Tape;
 }
 
+// Outer iterations told apart by prev_iters (later ones share the last entry).
+static constexpr int PREV_OUTER = 16;
+
 struct cms2d_flow {
     cms::TelHost *tel = nullptr;   // telescoping grid (cell-list step), or null
     int dev = 0;
@@ -161,7 +164,12 @@ struct cms2d_flow {
     double dtimebeg = 0.0, deltime = 0.0;
     int ntime = 0, maxit = 0, niter = 0, iconv = 1;
     double rmom[3]{}, rmom0[3]{}, rmom1[3]{};
-    int kry[3]{}, prev_iters[6]{4, 2, 2, 4, 2, 2};
+    int kry[3]{};
+    // iterations that each system's last solve at an outer iteration took, by
+    // the outer iteration (the counts fall over a step's outer iterations and
+    // repeat from step to step)
+    int prev_iters[PREV_OUTER][6]{};
+    int last_iters[6]{4, 2, 2, 4, 2, 2};   // of its last solve (where there is none yet)
     // timing of the pp-system SpMV launches (events bracket each launch)
     bool stats = true;
     KTimer tm;                 // live timing of the pp solve's main kernels
@@ -358,7 +366,7 @@ struct KryCtx {
     int kmax;
     double rtol, atol;
     KryScal *d_sc, *h_sc;
-    int *prev_iters;
+    int *prev_iters, *last_iters;  // expected counts (0: unknown), and the last solve's
     KTimer *tm;                    // timed launches (or null)
     hipGraphExec_t *graph = nullptr;   // per-system graph slots (or null: direct launches)
 };
@@ -430,11 +438,13 @@ static int run_bicg(KryCtx &X, KrySys<NS, T> &K, Op A, int sc0, Pre pre = Pre())
         for (int q = 0; q < NS; q++) d &= X.h_sc[sc0 + q].done;
         return d;
     };
-    // batches: the last solve's count, then 2, 2, 4, 8, ... so that few
+    // batches: the expected count, then 2, 2, 4, 8, ... so that few
     // launches follow convergence (each costs a few microseconds even when it
     // returns at once) and few host round trips are needed
     int it = 0, nbatch = 0, grow = 2;
-    int batch = std::max(1, X.prev_iters[sc0]);
+    int batch = 1;
+    for (int q = sc0; q < sc0 + NS; q++)
+        batch = std::max(batch, X.prev_iters[q] > 0 ? X.prev_iters[q] : X.last_iters[q]);
     const hipGraphExec_t ge = X.graph ? X.graph[sc0] : nullptr;
     for (bool first = true; first || (!all_done() && it < X.kmax); first = false) {
         const int nb = std::min(batch, X.kmax - it);
@@ -466,7 +476,8 @@ static int run_bicg(KryCtx &X, KrySys<NS, T> &K, Op A, int sc0, Pre pre = Pre())
         batch = grow;
         if (++nbatch >= 2) grow = std::min(2 * grow, 64);
     }
-    for (int q = 0; q < NS; q++) X.prev_iters[sc0 + q] = std::max(1, X.h_sc[sc0 + q].final_iters);
+    for (int q = 0; q < NS; q++)
+        X.prev_iters[sc0 + q] = X.last_iters[sc0 + q] = std::max(1, X.h_sc[sc0 + q].final_iters);
     return 0;
 }
 
@@ -656,6 +667,7 @@ static int pp_solve_refine(cms2d_flow *F, KryCtx &X, StencilOp A) {
     InnerPre pre{F};
     int total = 0;
     for (int sw = 0; sw < REF_SWEEPS && !F->h_sc[0].done; sw++) {
+        Xi.prev_iters = F->prev_iters[std::min(sw, PREV_OUTER - 1)];   // the sweeps' counts repeat, sweep by sweep
         hipLaunchKernelGGL(k_ref_start<StencilOp32>, dim3(nb), dim3(KBLOCK), 0, F->st, A32, Ki, (const double *)K.r[0]);
         if (int rc = run_bicg<StencilOp32, 1, 1, float>(Xi, Ki, A32, 3, pre)) return rc;
         total += F->h_sc[3].final_iters;
@@ -686,6 +698,7 @@ static int uv_solve_refine(cms2d_flow *F, KryCtx &X, StencilOp A) {
     Xi.rtol = REF_RTOL_UV;
     int total[2] = {0, 0};
     for (int sw = 0; sw < REF_SWEEPS && !(F->h_sc[1].done && F->h_sc[2].done); sw++) {
+        Xi.prev_iters = F->prev_iters[std::min(sw, PREV_OUTER - 1)];
         hipLaunchKernelGGL(k_ref_start2<StencilOp32>, dim3(nb), dim3(KBLOCK), 0, F->st, A32, Ki, K);
         if (int rc = run_bicg<StencilOp32, 2, 0, float>(Xi, Ki, A32, 4)) return rc;
         for (int q = 0; q < 2; q++) total[q] += F->h_sc[4 + q].final_iters;
@@ -758,7 +771,8 @@ static KryCtx flow_ctx(cms2d_flow *F, bool timed) {
     KryCtx X;
     X.st = F->st; X.nblk = F->nblk_kry; X.kmax = F->P.kmax;
     X.rtol = F->P.rtol; X.atol = F->P.atol;
-    X.d_sc = F->d_sc; X.h_sc = F->h_sc; X.prev_iters = F->prev_iters;
+    X.d_sc = F->d_sc; X.h_sc = F->h_sc; X.prev_iters = F->prev_iters[std::min(std::max(F->niter, 1), PREV_OUTER) - 1];
+    X.last_iters = F->last_iters;
     X.tm = (timed && F->stats) ? &F->tm : nullptr;
     X.graph = F->use_graphs ? F->kgraph : nullptr;
     return X;
@@ -1890,7 +1904,7 @@ static void ck_host_get(const cms2d_flow *F, CkHost &c) {
     for (int n = 0; n < 3; n++) { c.rmom[n] = F->rmom[n]; c.rmom0[n] = F->rmom0[n]; c.rmom1[n] = F->rmom1[n]; c.kry[n] = F->kry[n]; }
     c.dtvar = F->dtvar; c.jtime = F->jtime; c.mtime = F->mtime; c.ntime = F->ntime; c.maxit = F->maxit;
     c.niter = F->niter; c.iconv = F->iconv; c.prev_gm = F->prev_gm;
-    for (int n = 0; n < 6; n++) c.prev_iters[n] = F->prev_iters[n];
+    for (int n = 0; n < 6; n++) c.prev_iters[n] = F->last_iters[n];
     c.windconst = F->windconst; c.wndx = F->wndx; c.wndy = F->wndy;
     c.wse_inc = F->wse_inc;
     c.q_inc = F->q_inc;
@@ -1901,7 +1915,7 @@ static void ck_host_set(cms2d_flow *F, const CkHost &c) {
     for (int n = 0; n < 3; n++) { F->rmom[n] = c.rmom[n]; F->rmom0[n] = c.rmom0[n]; F->rmom1[n] = c.rmom1[n]; F->kry[n] = c.kry[n]; }
     F->dtvar = c.dtvar; F->jtime = c.jtime; F->mtime = c.mtime; F->ntime = c.ntime; F->maxit = c.maxit;
     F->niter = c.niter; F->iconv = c.iconv; F->prev_gm = c.prev_gm;
-    for (int n = 0; n < 6; n++) F->prev_iters[n] = c.prev_iters[n];
+    for (int n = 0; n < 6; n++) F->last_iters[n] = c.prev_iters[n];
     F->windconst = c.windconst; F->wndx = c.wndx; F->wndy = c.wndy;
     F->wse_inc = c.wse_inc;
     F->q_inc = c.q_inc;
@@ -2136,9 +2150,9 @@ static int solve_device(const SolveBufs &B, hipStream_t st, int ncells, int nmax
     EllOp A{ncells, nmaxfaces, B.c2c, B.a};
     hipLaunchKernelGGL(k_ell_prologue, dim3(nblk), dim3(KBLOCK), 0, st, A, (const int *)B.w, B.ss,
                        (const double *)B.sp, B.res, (const double *)B.phi, relax, K, bias);
-    int prev = 8;
+    int prev = 0, last = 8;
     KryCtx X{st, nblk, kmax > 0 ? kmax : 4000, rtol > 0 ? rtol : 1e-10, atol >= 0 ? atol : 1e-12,
-             B.sc, &h_sc, &prev, nullptr};
+             B.sc, &h_sc, &prev, &last, nullptr};
     if (int rc = run_bicg(X, K, A, 0)) return rc;
     HIPCHK(hipStreamSynchronize(st));
     return 0;

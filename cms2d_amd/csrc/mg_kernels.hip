@@ -121,6 +121,9 @@ struct MTile {
     static constexpr int NS = (SX * SY + NT - 1) / NT;                        // staged per thread (down)
     static constexpr int HX = SX / 2, NH = (HX * SY + NT - 1) / NT;           // staged black cells (up)
     static constexpr int NR = (TX + TY + NT - 1) / NT;                        // halo cells per thread
+    // the stop flag is tested first on the large tiles (a launch after the stop
+    // must not stream a large level), after the loads are issued on the others
+    static constexpr bool EARLY = TX * TY >= 1024;
     static_assert(NB * NT * 4 == TX * TY && TX % 2 == 0 && TY % 2 == 0, "whole blocks per thread");
 };
 
@@ -165,6 +168,7 @@ __global__ void __launch_bounds__(NT) k_mg_down(MgLevel f, const TB *b, MgLevel 
     using T = MTile<TX, TY, NT>;
     __shared__ float q[T::SY][T::SX];     // b/ap, then the black cells' z in place
     const bool done = sc->done;
+    if (T::EARLY && done) return;
     int X0, Y0;
     mg_tile_origin<TX, TY>(X0, Y0);
     float4 a[T::NB][4], ha[T::NR];
@@ -244,6 +248,7 @@ __global__ void __launch_bounds__(NT) k_mg_up(MgLevel L, const TB *b, MgLevel C,
     using T = MTile<TX, TY, NT>;
     __shared__ float w[T::SY][T::SX];     // black cells: w; red cells: the new z
     const bool done = sc->done;
+    if (T::EARLY && done) return;
     int X0, Y0;
     mg_tile_origin<TX, TY>(X0, Y0);
     float4 a[T::NB][4], ha[T::NR];

@@ -515,6 +515,7 @@ static int tel_uv_solve_refine(cms2d_flow *F, KryCtx &X, const TelOp &A) {
     Xi.rtol = REF_RTOL_UV;
     int total[2] = {0, 0};
     for (int sw = 0; sw < REF_SWEEPS && !(F->h_sc[1].done && F->h_sc[2].done); sw++) {
+        Xi.prev_iters = F->prev_iters[std::min(sw, PREV_OUTER - 1)];
         hipLaunchKernelGGL(k_ref_start2<TelOp32>, dim3(nb), dim3(KBLOCK), 0, F->st, A32, Ki, K);
         if (int rc = run_bicg<TelOp32, 2, 0, float>(Xi, Ki, A32, 4)) return rc;
         for (int q = 0; q < 2; q++) total[q] += F->h_sc[4 + q].final_iters;
@@ -546,6 +547,7 @@ static int tel_pp_solve_refine(cms2d_flow *F, KryCtx &X, const TelOp &A) {
     TelInnerPre pre{F};
     int total = 0;
     for (int sw = 0; sw < REF_SWEEPS && !F->h_sc[0].done; sw++) {
+        Xi.prev_iters = F->prev_iters[std::min(sw, PREV_OUTER - 1)];
         hipLaunchKernelGGL(k_ref_start<TelOp32>, dim3(nb), dim3(KBLOCK), 0, F->st, A32, Ki, (const double *)K.r[0]);
         if (int rc = run_bicg<TelOp32, 1, 1, float>(Xi, Ki, A32, 3, pre)) return rc;
         total += F->h_sc[3].final_iters;
