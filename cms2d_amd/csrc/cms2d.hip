@@ -2211,9 +2211,12 @@ extern "C" int cms2d_solve(int ncells, int ncellsD, int nmaxfaces, const double 
 // i, so the transposed solve runs the same kernels on a system written by
 // k_adj_setup (relax 1, sp chosen so that its diagonal is ap).
 
-__global__ void k_adj_setup(EllOp A, const int *back, const double *sp, double relax, const double *gphi,
+// lam starts from 0 on the ghosts too: the solve prologue multiplies them by
+// their zero coefficients, and fresh memory can hold a NaN.
+__global__ void k_adj_setup(EllOp A, int nd, const int *back, const double *sp, double relax, const double *gphi,
                             double *at, double *spt, double *sst, double *lam) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < nd) lam[i] = 0.0;
     if (i >= A.ncells) return;
     const int nf = A.nf;
     double asum = 0.0, tsum = 0.0;
@@ -2228,7 +2231,6 @@ __global__ void k_adj_setup(EllOp A, const int *back, const double *sp, double r
     const double ap = (asum - sp[i]) / relax;
     spt[i] = tsum - ap;
     sst[i] = gphi[i];
-    lam[i] = 0.0;
 }
 // Gradients of the active cells' inputs from lambda.
 __global__ void k_adj_grads(EllOp A, const double *sp, const double *phi_old, const double *phi, double relax,
@@ -2339,7 +2341,7 @@ extern "C" int cms2d_solve_adjoint(int ncells, int ncellsD, int nmaxfaces, const
         HIPCHK(hipMemcpyAsync(gp, gphi, n * sizeof(double), hipMemcpyHostToDevice, st));
         const EllOp A{ncells, nmaxfaces, c2c, a};
         const unsigned nb = (unsigned)((n + BLOCK - 1) / BLOCK);
-        hipLaunchKernelGGL(k_adj_setup, dim3(nb), dim3(BLOCK), 0, st, A, (const int *)bk, (const double *)spd, relax,
+        hipLaunchKernelGGL(k_adj_setup, dim3((unsigned)((nD + BLOCK - 1) / BLOCK)), dim3(BLOCK), 0, st, A, ncellsD, (const int *)bk, (const double *)spd, relax,
                            (const double *)gp, B.a, B.sp, B.ss, B.phi);
         hipLaunchKernelGGL(k_set_int, dim3(nb), dim3(BLOCK), 0, st, B.w, ncells, 1);
         KryScal h_sc{};
