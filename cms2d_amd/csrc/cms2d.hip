@@ -407,6 +407,12 @@ template <class Op, int NS, int PREC, class T, class Pre>
 static void bicg_iter(const KryCtx &X, KrySys<NS, T> &K, Op A, Pre &pre, int i) {
     const dim3 grid(X.nblk), blk(KBLOCK);
     if (X.tm) X.tm->it = i;
+    if constexpr (PREC == 0 && Op::FUSED > 0) if (A.n() <= Op::FUSED) {
+        hipLaunchKernelGGL((k_bicg_f1<Op, NS, T>), grid, blk, 0, X.st, A, K, i, X.nblk, X.kmax, X.rtol, X.atol);
+        hipLaunchKernelGGL((k_bicg_f2<Op, NS, T>), grid, blk, 0, X.st, A, K, i, X.nblk);
+        hipLaunchKernelGGL((k_bicg_f3<Op, NS, T>), grid, blk, 0, X.st, A, K, i, X.nblk);
+        return;
+    }
     hipLaunchKernelGGL((k_bicg_p<Op, NS, T>), grid, blk, 0, X.st, A, K, i, X.nblk, X.kmax, X.rtol, X.atol, 0);
     if (PREC) pre(0);
     tlaunch(X.tm, TG_SPMV_PP, k_bicg_spmv<Op, NS, 1, PREC, T>, grid, blk, 0, X.st, A, K);
@@ -1486,6 +1492,9 @@ static int create_impl(const cms2d_flow_desc *d, cms2d_flow *F) {
             F->Kuv.dinv_w[q] = kv[q + 1][6];
         }
         F->Kuv.sc = F->d_sc + 1;
+        for (int q = 0; q < 2; q++)
+            if (int rc = dalloc(F, &F->Kuv.p2[q], N)) return rc;
+        F->Kpp.p2[0] = F->Kuv.p2[0];       // (pp without a multigrid; solves do not overlap)
     }
     // multigrid hierarchy: level 0 shares the padded layout of the flow arrays
     F->precond = d->precond;
@@ -1522,7 +1531,8 @@ static int create_impl(const cms2d_flow_desc *d, cms2d_flow *F) {
         if (F->precision == CMS2D_PREC_FP32_REFINE) {
             KrySys<2, float> &K2 = F->Kin2;
             for (int q = 0; q < 2; q++) {
-                float **vec[] = {&K2.x[q], &K2.r[q], &K2.r0[q], &K2.p[q], &K2.v[q], &K2.t[q], &K2.ap_w[q], &K2.dinv_w[q]};
+                float **vec[] = {&K2.x[q], &K2.r[q], &K2.r0[q], &K2.p[q], &K2.p2[q],
+                                 &K2.v[q], &K2.t[q], &K2.ap_w[q], &K2.dinv_w[q]};
                 for (float **v : vec)
                     if (int rc = dalloc(F, v, N)) return rc;
             }
@@ -2143,7 +2153,7 @@ static int solve_device(const SolveBufs &B, hipStream_t st, int ncells, int nmax
     KrySys<1> K{};
     K.x[0] = B.phi;
     K.r[0] = B.vec; K.r0[0] = B.vec + n; K.p[0] = B.vec + 2 * n; K.v[0] = B.vec + 3 * n; K.t[0] = B.vec + 4 * n;
-    K.ap_w[0] = B.vec + 5 * n;
+    K.p2[0] = B.vec + 5 * n;
     K.dinv_w[0] = B.vec + 6 * n;
     K.sc = B.sc;
     K.red.pr[0] = B.partials; K.red.pv[0] = B.partials + 2 * nblk; K.red.pt[0] = B.partials + 3 * nblk;

@@ -131,6 +131,13 @@ __device__ __forceinline__ void grid_walk(const Geo &g, F &&f) {
     for (bool ok = w.first(x); ok; ok = w.next(x)) f(x);
 }
 
+// Systems of up to this many cells take the Jacobi iteration in three launches
+// (k_bicg_f1): at 20 000 cells 24 us against 26 for two systems and 13 % of a
+// whole cms2d_solve call; equal at 120 000; at 3 M cells 349 against 275 us,
+// where forming p and s at every neighbour costs more loads than the sweeps
+// save.
+constexpr int KRY_FUSED = 65536;
+
 // Matrix operators: y_i = ap_i z_i - sum_k a_k(i) z_nb(k).  apply() is the
 // Jacobi-preconditioned form, z = M^-1 x = x/ap with 1/ap stored (dinv), so
 // y_i = x_i - sum_k a_k(i) x_nb dinv_nb; z = 0 on ghost cells, where the
@@ -138,10 +145,11 @@ __device__ __forceinline__ void grid_walk(const Geo &g, F &&f) {
 // neighbours are read without a bounds test, whose branches would each wait
 // for their own load.
 struct StencilOp {
+    static constexpr int FUSED = KRY_FUSED;
     using C = double;
     Geo g;
     const C *aN, *aE, *aS, *aW;
-    __device__ __forceinline__ int n() const { return g.nact; }
+    __host__ __device__ __forceinline__ int n() const { return g.nact; }
     __device__ __forceinline__ GridWalk walk() const { return GridWalk(g); }
     template <class F>
     __device__ __forceinline__ void each(F &&f) const { grid_walk(g, f); }
@@ -151,6 +159,16 @@ struct StencilOp {
         x.i = t - x.j * g.nx;
         x.c = cidx(g, x.i, x.j);
         return x;
+    }
+    // sum_k a_k z_nb of NS vectors, get(q, nb) the value of vector q at cell nb
+    // (V: their type)
+    template <int NS, class V, class Get>
+    __device__ __forceinline__ void sums(const Idx &x, Get &&get, V (&sum)[NS]) const {
+        const int c = x.c, cN = c + g.nxp, cE = c + 1, cS = c - g.nxp, cW = c - 1;
+        const V wN = (V)aN[c], wE = (V)aE[c], wS = (V)aS[c], wW = (V)aW[c];
+#pragma unroll
+        for (int q = 0; q < NS; q++)
+            sum[q] = ((wN * get(q, cN) + wE * get(q, cE)) + wS * get(q, cS)) + wW * get(q, cW);
     }
     // of NS vectors at once (V: their type)
     template <int NS, class V>
@@ -178,12 +196,21 @@ struct StencilOp {
 };
 // The same operator in FP32, the four coefficients of a cell side by side (N, E, S, W).
 struct StencilOp32 {
+    static constexpr int FUSED = KRY_FUSED;
     Geo g;
     const float4 *a;
-    __device__ __forceinline__ int n() const { return g.nact; }
+    __host__ __device__ __forceinline__ int n() const { return g.nact; }
     __device__ __forceinline__ GridWalk walk() const { return GridWalk(g); }
     template <class F>
     __device__ __forceinline__ void each(F &&f) const { grid_walk(g, f); }
+    template <int NS, class V, class Get>
+    __device__ __forceinline__ void sums(const Idx &x, Get &&get, V (&sum)[NS]) const {
+        const int c = x.c;
+        const float4 w = a[c];
+#pragma unroll
+        for (int q = 0; q < NS; q++)
+            sum[q] = ((w.x * get(q, c + g.nxp) + w.y * get(q, c + 1)) + w.z * get(q, c - g.nxp)) + w.w * get(q, c - 1);
+    }
     __device__ __forceinline__ float sum(const float *z, const float *dinv, const Idx &x) const {
         const int c = x.c;
         const int nb[4] = {c + g.nxp, c + 1, c - g.nxp, c - 1};
@@ -208,11 +235,26 @@ struct StencilOp32 {
 // (0-based, ghosts numbered from ncells, -1 for no face).
 constexpr int ELL_MAX_FACES = 8;   // nmaxfaces: 4 Cartesian, 6 telescoping (read_tel, geospatial.F90:433)
 struct EllOp {
+    static constexpr int FUSED = KRY_FUSED;
     int ncells, nf;      // cells, faces per cell (row stride of c2c and a)
     const int *c2c;
     const double *a;
-    __device__ __forceinline__ int n() const { return ncells; }
+    __host__ __device__ __forceinline__ int n() const { return ncells; }
     __device__ __forceinline__ ChunkWalk walk() const { return ChunkWalk(ncells); }
+    template <int NS, class V, class Get>
+    __device__ __forceinline__ void sums(const Idx &x, Get &&get, V (&sum)[NS]) const {
+        const int c = x.c;
+#pragma unroll
+        for (int q = 0; q < NS; q++) sum[q] = V(0);
+#pragma unroll
+        for (int k = 0; k < ELL_MAX_FACES; k++) {
+            if (k >= nf) break;
+            const int nb = c2c[nf * c + k];
+            if (nb < 0 || nb >= ncells) continue;
+#pragma unroll
+            for (int q = 0; q < NS; q++) sum[q] += a[nf * c + k] * get(q, nb);
+        }
+    }
     template <int NS>
     __device__ __forceinline__ void apply_n(const double *const (&xv)[NS], const double *const (&dinv)[NS],
                                             const Idx &x, double (&y)[NS]) const {
@@ -237,6 +279,7 @@ struct EllOp {
 template <int NS, class T = double>
 struct KrySys {
     T *x[NS], *r[NS], *r0[NS], *p[NS], *v[NS], *t[NS];
+    T *p2[NS];         // second buffer of p in the fused form (k_bicg_f1)
     T *ap_w[NS];       // diagonal ap of each system (written by the prologue)
     T *dinv_w[NS];     // 1/ap (Jacobi form)
     float *zp, *zs;    // M^-1 p and M^-1 s of system 0 (explicit preconditioner only)

@@ -63,6 +63,74 @@ __global__ void __launch_bounds__(KBLOCK) k_uv_prologue(Geo g, St s, KrySys<2> K
 // partials and before it tests a flag; only the stores wait for those (in
 // turn, flag, partials, scalars and operands took 1.5-2 us more per launch).
 
+// The start of iteration it (or of the solve, it == 0): which systems go on,
+// their beta and omega, and whether r0 restarts; block 0 publishes the scalars.
+template <int NS>
+struct KryStart {
+    int sdone[NS], siter[NS];
+    double sthr[NS], srho[NS], sr0n[NS], salp[NS], somg[NS];
+    bool act[NS];
+    int rst[NS];
+    double beta[NS], om[NS];
+    // the scalars of system q as iteration it - 1 left them (slot pq)
+    template <class Sys>
+    __device__ __forceinline__ void scalars(const Sys &K, int q, int pq) {
+        const KryScal &sc = K.sc[q];
+        sdone[q] = sc.done; siter[q] = sc.iters[pq]; sthr[q] = sc.thr; srho[q] = sc.rho[pq];
+        sr0n[q] = sc.r0n[pq]; salp[q] = sc.alpha[pq]; somg[q] = sc.omega[pq];
+    }
+    // tot: r.r and r0.r of each system (r.r and res.res when it == 0), n cells;
+    // false: every system has stopped
+    template <class Sys>
+    __device__ __forceinline__ bool finish(const Sys &K, const double (&tot)[2 * NS], int it, int kmax, double rtol,
+                                           double atol, int n, bool load) {
+        const int pq = (it - 1) & 1, cq = it & 1;
+        bool any = false;
+#pragma unroll
+        for (int q = 0; q < NS; q++) {
+            KryScal &sc = K.sc[q];
+            act[q] = false; rst[q] = 0; beta[q] = 0.0; om[q] = 1.0;
+            if (load) scalars(K, q, pq);
+            if (uni(sdone[q])) continue;
+            const double rr = uni(tot[2 * q]), nr = uni(sqrt(rr));
+            if (it == 0) {
+                const double thr = fmax(rtol * nr, atol * sqrt((double)n));
+                act[q] = !(nr <= thr);
+                if (lead()) {
+                    sc.rmom = sqrt(tot[2 * q + 1] / (double)(float)n);   // sqrt(adak/real(ncells))
+                    sc.thr = thr;
+                    sc.rho[0] = rr;
+                    sc.r0n[0] = nr;
+                    sc.iters[0] = 0;
+                    sc.rnorm = nr;
+                    if (!act[q]) { sc.done = 1; sc.final_iters = 0; }
+                }
+            } else {
+                const double r0r = uni(tot[2 * q + 1]);
+                const int iters = uni(siter[q]) + 1;
+                const double rho_p = uni(srho[q]), r0n_p = uni(sr0n[q]), al = uni(salp[q]), omp = uni(somg[q]);
+                double rho = rho_p, r0n = r0n_p;
+                if (omp == 0.0 || nr <= uni(sthr[q]) || iters >= kmax) {
+                    act[q] = false;
+                } else if (fabs(r0r) <= 1e-12 * nr * r0n_p) {
+                    rst[q] = 1; rho = rr; r0n = nr; beta[q] = 0.0; act[q] = true;
+                } else {
+                    beta[q] = uni((r0r / rho_p) * (al / omp)); rho = r0r; act[q] = true;
+                }
+                om[q] = omp;
+                if (lead()) {
+                    sc.rnorm = nr;
+                    sc.iters[cq] = iters;
+                    if (act[q]) { sc.rho[cq] = rho; sc.r0n[cq] = r0n; }
+                    else { sc.done = 1; sc.final_iters = iters; }
+                }
+            }
+            any = any || act[q];
+        }
+        return any;
+    }
+};
+
 // Finishes iteration it-1 (or starts the solve when it == 0) and, unless
 // fin_only, updates p.  Launched with fin_only on one block at the end of a
 // batch so the host can read the state; the next batch repeats the same
@@ -92,73 +160,22 @@ __global__ void __launch_bounds__(KBLOCK, NS == 2 ? 8 : 1) k_bicg_p(Op A, KrySys
     constexpr bool PRE = NS == 1;
     bool ok = !fin_only && w.first(x);
     if (PRE && ok) load();
-    const int pq = (it - 1) & 1, cq = it & 1;
-    int sdone[NS], siter[NS];
-    double sthr[NS], srho[NS], sr0n[NS], salp[NS], somg[NS];
-    auto scalars = [&](int q) {
-        const KryScal &sc = K.sc[q];
-        sdone[q] = sc.done; siter[q] = sc.iters[pq]; sthr[q] = sc.thr; srho[q] = sc.rho[pq];
-        sr0n[q] = sc.r0n[pq]; salp[q] = sc.alpha[pq]; somg[q] = sc.omega[pq];
-    };
-    if (PRE) scalars(0);
+    const int pq = (it - 1) & 1;
+    KryStart<NS> f;
+    if (PRE) f.scalars(K, 0, pq);
     double tot[2 * NS];
     const double *src[2 * NS];
 #pragma unroll
     for (int q = 0; q < NS; q++) { src[2 * q] = K.red.pr[q]; src[2 * q + 1] = K.red.pr[q] + nb; }
     sum_partials<2 * NS>(src, nb, tot);
-    bool act[NS];
-    int rst[NS];
-    double beta[NS], om[NS];
-    bool any = false;
-#pragma unroll
-    for (int q = 0; q < NS; q++) {
-        KryScal &sc = K.sc[q];
-        act[q] = false; rst[q] = 0; beta[q] = 0.0; om[q] = 1.0;
-        if (!PRE) scalars(q);
-        if (uni(sdone[q])) continue;
-        const double rr = uni(tot[2 * q]), nr = uni(sqrt(rr));
-        if (it == 0) {
-            const double thr = fmax(rtol * nr, atol * sqrt((double)A.n()));
-            act[q] = !(nr <= thr);
-            if (lead()) {
-                sc.rmom = sqrt(tot[2 * q + 1] / (double)(float)A.n());   // sqrt(adak/real(ncells))
-                sc.thr = thr;
-                sc.rho[0] = rr;
-                sc.r0n[0] = nr;
-                sc.iters[0] = 0;
-                sc.rnorm = nr;
-                if (!act[q]) { sc.done = 1; sc.final_iters = 0; }
-            }
-        } else {
-            const double r0r = uni(tot[2 * q + 1]);
-            const int iters = uni(siter[q]) + 1;
-            const double rho_p = uni(srho[q]), r0n_p = uni(sr0n[q]), al = uni(salp[q]), omp = uni(somg[q]);
-            double rho = rho_p, r0n = r0n_p;
-            if (omp == 0.0 || nr <= uni(sthr[q]) || iters >= kmax) {
-                act[q] = false;
-            } else if (fabs(r0r) <= 1e-12 * nr * r0n_p) {
-                rst[q] = 1; rho = rr; r0n = nr; beta[q] = 0.0; act[q] = true;
-            } else {
-                beta[q] = uni((r0r / rho_p) * (al / omp)); rho = r0r; act[q] = true;
-            }
-            om[q] = omp;
-            if (lead()) {
-                sc.rnorm = nr;
-                sc.iters[cq] = iters;
-                if (act[q]) { sc.rho[cq] = rho; sc.r0n[cq] = r0n; }
-                else { sc.done = 1; sc.final_iters = iters; }
-            }
-        }
-        any = any || act[q];
-    }
-    if (!any) return;
+    if (!f.finish(K, tot, it, kmax, rtol, atol, A.n(), !PRE)) return;
     if (!PRE && ok) load();
     while (ok) {
 #pragma unroll
         for (int q = 0; q < NS; q++) {
-            if (!act[q]) continue;
-            if (rst[q]) K.r0[q][x.c] = r[q];
-            K.p[q][x.c] = it == 0 ? r[q] : r[q] + (T)beta[q] * (p[q] - (T)om[q] * v[q]);
+            if (!f.act[q]) continue;
+            if (f.rst[q]) K.r0[q][x.c] = r[q];
+            K.p[q][x.c] = it == 0 ? r[q] : r[q] + (T)f.beta[q] * (p[q] - (T)f.om[q] * v[q]);
         }
         ok = w.next(x);
         if (ok) load();
@@ -355,6 +372,196 @@ __global__ void __launch_bounds__(KBLOCK) k_bicg_r(Op A, KrySys<NS, T> K, int it
     put_partials<2 * NS>(red, dst);
 }
 
+// The Jacobi iteration in three launches (systems of up to KRY_FUSED cells,
+// where a launch costs more than its loads): p and s are formed where they are
+// read, at a cell and at its neighbours, instead of in sweeps of their own
+// (f1: k_bicg_p and v = A M^-1 p; f2: alpha and t = A M^-1 s; f3: both updates of x
+// and r).  A neighbour's p needs r, p and v of the launches before, so p
+// goes to the buffer that it was not read from, and v to the one that held t
+// (K.p and K.p2, K.v and K.t in turn by the parity of it; t takes the place of
+// the v that f1 read).  The values are those of the five sweeps.
+template <int NS, class T>
+struct KryBuf {
+    T *pin[NS], *pout[NS], *vin[NS], *vout[NS];
+    __device__ __forceinline__ KryBuf(const KrySys<NS, T> &K, int it) {
+#pragma unroll
+        for (int q = 0; q < NS; q++) {
+            const bool o = it & 1;
+            pin[q] = o ? K.p[q] : K.p2[q];
+            pout[q] = o ? K.p2[q] : K.p[q];
+            vin[q] = o ? K.v[q] : K.t[q];
+            vout[q] = o ? K.t[q] : K.v[q];
+        }
+    }
+};
+template <class Op, int NS, class T = double>
+__global__ void __launch_bounds__(KBLOCK) k_bicg_f1(Op A, KrySys<NS, T> K, int it, int nb, int kmax, double rtol,
+                                                   double atol) {
+    const KryBuf<NS, T> B(K, it);
+    auto w = A.walk();
+    Idx x;
+    bool ok = w.first(x);
+    double tot[2 * NS];
+    const double *src[2 * NS];
+#pragma unroll
+    for (int q = 0; q < NS; q++) { src[2 * q] = K.red.pr[q]; src[2 * q + 1] = K.red.pr[q] + nb; }
+    sum_partials<2 * NS>(src, nb, tot);
+    KryStart<NS> f;
+    if (!f.finish(K, tot, it, kmax, rtol, atol, A.n(), true)) return;
+    double red[NS];
+#pragma unroll
+    for (int q = 0; q < NS; q++) red[q] = 0.0;
+    for (; ok; ok = w.next(x)) {
+        T sum[NS];
+        auto pnew = [&](int q, int c) {
+            const T r = K.r[q][c];
+            return it == 0 ? r : r + (T)f.beta[q] * (B.pin[q][c] - (T)f.om[q] * B.vin[q][c]);
+        };
+        A.template sums<NS, T>(x, [&](int q, int c) { return f.act[q] ? pnew(q, c) * K.dinv_w[q][c] : T(0); }, sum);
+#pragma unroll
+        for (int q = 0; q < NS; q++) {
+            if (!f.act[q]) continue;
+            const int c = x.c;
+            const T p = pnew(q, c), y = p - sum[q];
+            T r0 = K.r0[q][c];
+            if (f.rst[q]) K.r0[q][c] = r0 = K.r[q][c];
+            B.pout[q][c] = p;
+            B.vout[q][c] = y;
+            red[q] += (double)r0 * (double)y;
+        }
+    }
+    double *dst[NS];
+#pragma unroll
+    for (int q = 0; q < NS; q++) dst[q] = K.red.pv[q];
+    put_partials<NS>(red, dst);
+}
+template <class Op, int NS, class T = double>
+__global__ void __launch_bounds__(KBLOCK) k_bicg_f2(Op A, KrySys<NS, T> K, int it, int nb) {
+    const KryBuf<NS, T> B(K, it);
+    auto w = A.walk();
+    Idx x;
+    bool ok = w.first(x);
+    const int cq = it & 1;
+    int sdone[NS], siter[NS];
+    double srho[NS];
+#pragma unroll
+    for (int q = 0; q < NS; q++) { sdone[q] = K.sc[q].done; siter[q] = K.sc[q].iters[cq]; srho[q] = K.sc[q].rho[cq]; }
+    double tot[NS];
+    const double *src[NS];
+#pragma unroll
+    for (int q = 0; q < NS; q++) src[q] = K.red.pv[q];
+    sum_partials<NS>(src, nb, tot);
+    bool act[NS];
+    double al[NS];
+    bool any = false;
+#pragma unroll
+    for (int q = 0; q < NS; q++) {
+        act[q] = !uni(sdone[q]);
+        al[q] = 0.0;
+        if (!act[q]) continue;
+        if (uni(tot[q]) == 0.0) {                  // r0.v = 0: stop before the update
+            act[q] = false;
+            if (lead()) { K.sc[q].done = 1; K.sc[q].final_iters = siter[q]; }
+            continue;
+        }
+        al[q] = uni(srho[q] / tot[q]);
+        if (lead()) K.sc[q].alpha[cq] = al[q];
+        any = true;
+    }
+    if (!any) return;
+    double red[2 * NS];
+#pragma unroll
+    for (int q = 0; q < 2 * NS; q++) red[q] = 0.0;
+    for (; ok; ok = w.next(x)) {
+        T sum[NS];
+        auto snew = [&](int q, int c) { return K.r[q][c] - (T)al[q] * B.vout[q][c]; };
+        A.template sums<NS, T>(x, [&](int q, int c) { return act[q] ? snew(q, c) * K.dinv_w[q][c] : T(0); }, sum);
+#pragma unroll
+        for (int q = 0; q < NS; q++) {
+            if (!act[q]) continue;
+            const T s = snew(q, x.c), y = s - sum[q];
+            const double yd = y;
+            B.vin[q][x.c] = y;
+            red[2 * q] += yd * (double)s;
+            red[2 * q + 1] += yd * yd;
+        }
+    }
+    double *dst[2 * NS];
+#pragma unroll
+    for (int q = 0; q < NS; q++) { dst[2 * q] = K.red.pt[q]; dst[2 * q + 1] = K.red.pt[q] + gridDim.x; }
+    put_partials<2 * NS>(red, dst);
+}
+template <class Op, int NS, class T = double>
+__global__ void __launch_bounds__(KBLOCK) k_bicg_f3(Op A, KrySys<NS, T> K, int it, int nb) {
+    const KryBuf<NS, T> B(K, it);
+    auto w = A.walk();
+    Idx x;
+    T r[NS], v[NS], t[NS], d[NS], xs[NS], p[NS], r0[NS];
+    auto load = [&](int q) {
+        r[q] = K.r[q][x.c];
+        v[q] = B.vout[q][x.c];
+        t[q] = B.vin[q][x.c];
+        d[q] = K.dinv_w[q][x.c];
+        xs[q] = K.x[q][x.c];
+        p[q] = B.pout[q][x.c];
+        r0[q] = K.r0[q][x.c];
+    };
+    bool ok = w.first(x);
+    constexpr bool PRE = NS == 1;         // (k_bicg_p)
+    if (PRE && ok) load(0);
+    const int cq = it & 1;
+    int sdone[NS];
+    double salp[NS];
+#pragma unroll
+    for (int q = 0; q < NS; q++) { sdone[q] = K.sc[q].done; salp[q] = K.sc[q].alpha[cq]; }
+    double tot[2 * NS];
+    const double *src[2 * NS];
+#pragma unroll
+    for (int q = 0; q < NS; q++) { src[2 * q] = K.red.pt[q]; src[2 * q + 1] = K.red.pt[q] + nb; }
+    sum_partials<2 * NS>(src, nb, tot);
+    bool act[NS];
+    double om[NS], al[NS];
+    bool any = false;
+#pragma unroll
+    for (int q = 0; q < NS; q++) {
+        act[q] = !uni(sdone[q]);
+        const double ts = tot[2 * q], tt = tot[2 * q + 1];
+        om[q] = uni(tt > 0.0 ? ts / tt : 0.0);
+        al[q] = uni(salp[q]);
+        if (act[q] && lead()) K.sc[q].omega[cq] = om[q];
+        any = any || act[q];
+    }
+    if (!any) return;
+    double red[2 * NS];
+#pragma unroll
+    for (int q = 0; q < 2 * NS; q++) red[q] = 0.0;
+    if (!PRE && ok)
+#pragma unroll
+        for (int q = 0; q < NS; q++) load(q);
+    while (ok) {
+#pragma unroll
+        for (int q = 0; q < NS; q++) {
+            if (!act[q]) continue;
+            const T s = r[q] - (T)al[q] * v[q];
+            const T x1 = xs[q] + al[q] * (p[q] * d[q]);
+            K.x[q][x.c] = x1 + om[q] * (s * d[q]);
+            const T rn = s - (T)om[q] * t[q];
+            K.r[q][x.c] = rn;
+            red[2 * q] += (double)rn * (double)rn;
+            red[2 * q + 1] += (double)r0[q] * (double)rn;
+        }
+        ok = w.next(x);
+        if (ok)
+#pragma unroll
+            for (int q = 0; q < NS; q++)
+                if (act[q]) load(q);
+    }
+    double *dst[2 * NS];
+#pragma unroll
+    for (int q = 0; q < NS; q++) { dst[2 * q] = K.red.pr[q]; dst[2 * q + 1] = K.red.pr[q] + gridDim.x; }
+    put_partials<2 * NS>(red, dst);
+}
+
 // Clears n 32-bit words with vector stores (used instead of a memset node).
 __global__ void k_zero_words(unsigned int *p, int n) {
     for (int i = threadIdx.x; i < n; i += blockDim.x) p[i] = 0u;
@@ -388,7 +595,6 @@ __global__ void __launch_bounds__(KBLOCK) k_ell_prologue(EllOp A, const int *iwe
         double rs = iwet[c] * (anb + ssv - ap * ph) / ap;
         res[c] = rs;
         double r = anb + ssv - ap * ph + bias;
-        K.ap_w[0][c] = ap;
         K.dinv_w[0][c] = 1.0 / ap;
         K.r[0][c] = r; K.r0[0][c] = r;
         red[0] += r * r;

@@ -597,11 +597,12 @@ __global__ void k_tl_bound_uv(TelG T, TelS s, Par P) {
 // over active neighbours (z = 0 on ghost cells, pbicgstab.f90:55,76).
 template <class CA>
 struct TelOpT {
+    static constexpr int FUSED = 0;       // (six faces a cell: not measured to gain)
     int nc, nd;
     const int *c2c;
     const uint64_t *meta;
     const CA *a;                 // [TF*nd]
-    __device__ __forceinline__ int n() const { return nc; }
+    __host__ __device__ __forceinline__ int n() const { return nc; }
     // Passes over the list in order: in pass p the blocks take consecutive
     // runs of KBLOCK cells from p * gridDim.x * KBLOCK on, consecutive blocks
     // on one XCD (xcd_block), so the cells a row above and below (a few
@@ -633,7 +634,8 @@ struct TelOpT {
     // past the last face and ghosts read cell c with coefficient 0), the slots
     // of joint cells after them.
     template <int NS, class V, class Get>
-    __device__ __forceinline__ void sums(int c, Get &&get, V (&sum)[NS]) const {
+    __device__ __forceinline__ void sums(const Idx &x, Get &&get, V (&sum)[NS]) const {
+        const int c = x.c;
         const int nf = m_ncf(meta[c]);
         int nb[4];
         V w[4];
@@ -672,14 +674,14 @@ struct TelOpT {
     __device__ __forceinline__ void apply_n(const V *const (&xv)[NS], const V *const (&dinv)[NS], const Idx &x,
                                             V (&y)[NS]) const {
         V sum[NS];
-        sums<NS, V>(x.c, [&](int q, int nb) { return xv[q][nb] * dinv[q][nb]; }, sum);
+        sums<NS, V>(x, [&](int q, int nb) { return xv[q][nb] * dinv[q][nb]; }, sum);
 #pragma unroll
         for (int q = 0; q < NS; q++) y[q] = xv[q][x.c] - sum[q];
     }
     template <class C>
     __device__ __forceinline__ C apply_z(const float *z, const C *ap, const Idx &x) const {
         C sum[1];
-        sums<1, C>(x.c, [&](int, int nb) { return (C)z[nb]; }, sum);
+        sums<1, C>(x, [&](int, int nb) { return (C)z[nb]; }, sum);
         return ap[x.c] * (C)z[x.c] - sum[0];
     }
 };
