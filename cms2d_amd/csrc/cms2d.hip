@@ -1701,13 +1701,11 @@ extern "C" int cms2d_flow_step(cms2d_flow *F, int nsteps, cms2d_step_info *info)
         (void)hipEventElapsedTime(&ms, F->step_ev[0], F->step_ev[1]);
         info->kernel_ms = ms;
         info->dt = F->deltime;
-        std::vector<uint8_t> w(F->npad);
-        HIPCHK(hipMemcpyAsync(w.data(), F->s.iwet, F->npad, hipMemcpyDeviceToHost, F->st));
-        HIPCHK(hipStreamSynchronize(F->st));
-        int nw = 0;
-        for (int j = 0; j < F->g.ny; j++)
-            for (int i = 0; i < F->g.nx; i++) nw += w[(size_t)(j + 1) * F->g.nxp + i + 1];
-        info->nwet = nw;
+        int *count = F->s.flags + 3;
+        LAUNCH(k_set_int, 1, count, 1, 0);
+        LAUNCH(k_count_wet, F->nblk_act, F->g, (const uint8_t *)F->s.iwet, count);
+        if (int rc = sync_flags(F)) return rc;
+        info->nwet = F->h_flags[3];
     }
     return CMS2D_OK;
 }
@@ -2008,20 +2006,16 @@ extern "C" int cms2d_flow_get(cms2d_flow *F, const char *name, double *out) {
     if (!F || !name || !out) return set_err(CMS2D_ERR_ARG, "null argument");
     if (F->tel) return tel_get(F, name, out);
     HIPCHK(hipSetDevice(F->dev));
-    HIPCHK(hipStreamSynchronize(F->st));
-    const Geo &g = F->g;
-    std::vector<double> h(F->npad);
+    // packed on the device in the pp solve's t, which holds nothing between solves
+    double *packed = F->Kpp.t[0];
     if (!strcmp(name, "iwet")) {
-        std::vector<uint8_t> w(F->npad);
-        HIPCHK(hipMemcpyAsync(w.data(), F->s.iwet, F->npad, hipMemcpyDeviceToHost, F->st));
-        HIPCHK(hipStreamSynchronize(F->st));
-        for (int j = 0; j < g.ny; j++)
-            for (int i = 0; i < g.nx; i++) out[(size_t)j * g.nx + i] = w[(size_t)(j + 1) * g.nxp + i + 1];
-        return CMS2D_OK;
+        LAUNCH(k_pack<uint8_t>, F->nblk_act, F->g, (const uint8_t *)F->s.iwet, packed);
+    } else {
+        const double *p = field_ptr(F, name);
+        if (!p) return set_err(CMS2D_ERR_ARG, std::string("unknown field ") + name);
+        LAUNCH(k_pack<double>, F->nblk_act, F->g, p, packed);
     }
-    double *p = field_ptr(F, name);
-    if (!p) return set_err(CMS2D_ERR_ARG, std::string("unknown field ") + name);
-    HIPCHK(hipMemcpyAsync(h.data(), p, F->npad * sizeof(double), hipMemcpyDeviceToHost, F->st));
+    HIPCHK(hipMemcpyAsync(out, packed, (size_t)F->g.nact * sizeof(double), hipMemcpyDeviceToHost, F->st));
     HIPCHK(hipStreamSynchronize(F->st));
     for (int j = 0; j < g.ny; j++)
         for (int i = 0; i < g.nx; i++) out[(size_t)j * g.nx + i] = h[(size_t)(j + 1) * g.nxp + i + 1];

@@ -1432,6 +1432,28 @@ __global__ void k_river_rating(Geo g, St s, int k, int m, double ramp, double *q
     else {
         int i = 1, jj = m;
         while (jj > i + 1) {
+// Active cells of a padded array in row-major order (what cms2d_flow_get hands
+// out, so that one copy of the grid's size crosses to the host and no host
+// loop follows: 7 -> 1.7 ms a field at 3 M cells).
+template <class T>
+__global__ void k_pack(Geo g, const T *src, double *dst) {
+    int i, j, c;
+    if (!act_thread(g, i, j, c)) return;
+    dst[j * g.nx + i] = (double)src[c];
+}
+// Wet active cells, added to *count (a wave at a time).
+__global__ void __launch_bounds__(BLOCK) k_count_wet(Geo g, const uint8_t *iwet, int *count) {
+    int i, j, c;
+    const bool wet = act_thread(g, i, j, c) && iwet[c];
+    const int n = __popcll(__ballot(wet));
+    if ((threadIdx.x & 63) == 0 && n) atomicAdd(count, n);
+}
+__global__ void __launch_bounds__(BLOCK) k_count_wet_list(int n, const uint8_t *iwet, int *count) {
+    const int i = blockIdx.x * BLOCK + threadIdx.x;
+    const int w = __popcll(__ballot(i < n && iwet[i]));
+    if ((threadIdx.x & 63) == 0 && w) atomicAdd(count, w);
+}
+
             const int kk = (i + jj) / 2;
             if (stage < x[kk - 1]) jj = kk;
             else i = kk;

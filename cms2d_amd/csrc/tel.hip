@@ -1449,12 +1449,11 @@ static int tel_step(cms2d_flow *F, int nsteps, cms2d_step_info *info) {
         (void)hipEventElapsedTime(&ms, F->step_ev[0], F->step_ev[1]);
         info->kernel_ms = ms;
         info->dt = F->deltime;
-        std::vector<uint8_t> w(H.T.n);
-        HIPCHK(hipMemcpyAsync(w.data(), H.s.iwet, H.T.n, hipMemcpyDeviceToHost, F->st));
-        HIPCHK(hipStreamSynchronize(F->st));
-        int nw = 0;
-        for (uint8_t x : w) nw += x;
-        info->nwet = nw;
+        int *count = H.s.flags + 3;
+        TLAUNCH(k_set_int, 1, count, 1, 0);
+        TLAUNCH(k_count_wet_list, H.nblk_n, H.T.n, (const uint8_t *)H.s.iwet, count);
+        if (int rc = tel_sync_flags(F)) return rc;
+        info->nwet = F->h_flags[3];
     }
     return CMS2D_OK;
 }
