@@ -2017,8 +2017,6 @@ extern "C" int cms2d_flow_get(cms2d_flow *F, const char *name, double *out) {
     }
     HIPCHK(hipMemcpyAsync(out, packed, (size_t)F->g.nact * sizeof(double), hipMemcpyDeviceToHost, F->st));
     HIPCHK(hipStreamSynchronize(F->st));
-    for (int j = 0; j < g.ny; j++)
-        for (int i = 0; i < g.nx; i++) out[(size_t)j * g.nx + i] = h[(size_t)(j + 1) * g.nxp + i + 1];
     return CMS2D_OK;
 }
 
