@@ -1432,6 +1432,21 @@ __global__ void k_river_rating(Geo g, St s, int k, int m, double ramp, double *q
     else {
         int i = 1, jj = m;
         while (jj > i + 1) {
+            const int kk = (i + jj) / 2;
+            if (stage < x[kk - 1]) jj = kk;
+            else i = kk;
+        }
+        double lb0 = 1.0, lb1 = 1.0;
+        lb0 = lb0 * (stage - x[i]) / (x[i - 1] - x[i]);
+        lb1 = lb1 * (stage - x[i - 1]) / (x[i] - x[i - 1]);
+        const double sum = (0.0 + lb0) + lb1;
+        w = 0.0;
+        w += lb0 / sum * v[i - 1];
+        w += lb1 / sum * v[i];
+    }
+    q[0] = ramp * w;
+}
+
 // Active cells of a padded array in row-major order (what cms2d_flow_get hands
 // out, so that one copy of the grid's size crosses to the host and no host
 // loop follows: 7 -> 1.7 ms a field at 3 M cells).
@@ -1452,21 +1467,6 @@ __global__ void __launch_bounds__(BLOCK) k_count_wet_list(int n, const uint8_t *
     const int i = blockIdx.x * BLOCK + threadIdx.x;
     const int w = __popcll(__ballot(i < n && iwet[i]));
     if ((threadIdx.x & 63) == 0 && w) atomicAdd(count, w);
-}
-
-            const int kk = (i + jj) / 2;
-            if (stage < x[kk - 1]) jj = kk;
-            else i = kk;
-        }
-        double lb0 = 1.0, lb1 = 1.0;
-        lb0 = lb0 * (stage - x[i]) / (x[i - 1] - x[i]);
-        lb1 = lb1 * (stage - x[i - 1]) / (x[i] - x[i - 1]);
-        const double sum = (0.0 + lb0) + lb1;
-        w = 0.0;
-        w += lb0 / sum * v[i - 1];
-        w += lb1 / sum * v[i];
-    }
-    q[0] = ramp * w;
 }
 
 __global__ void k_set_int(int *p, int n, int v) {
