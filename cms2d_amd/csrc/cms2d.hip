@@ -916,7 +916,7 @@ static int flow_recalculate(cms2d_flow *F) {
     LAUNCH(k_recalc, F->nblk_pad, F->g, F->s);
     if (int rc = wetdry(F)) return rc;
     if (F->qside >= 0) LAUNCH(k_bndflux, F->nblk_act, F->g, F->s);   // bndflux
-    LAUNCH(k_grad_fric_vis, F->nblk_act, F->g, F->s, F->P);
+    LAUNCH(k_grad_fric_vis, F->nblk_act, F->g, F->s, F->P, 1, 1);
     return eddyvis_tail(F);
 }
 
@@ -1028,7 +1028,7 @@ static int flow_imp_once(cms2d_flow *F) {
         TAPE(TAPE_PVFC1);
         LAUNCH(k_pvfc2, F->nblk_pad, g, s, F->P);
         LAUNCH(k_ghost_p, (2 * g.nx + 2 * g.ny + BLOCK - 1) / BLOCK, g, s, F->P);
-        LAUNCH(k_grad_fric_vis, F->nblk_act, g, s, F->P);
+        LAUNCH(k_grad_fric_vis, F->nblk_act, g, s, F->P, 0, F->stat_on);
         // bndriver_vel and bndflux after flow_grad_interp (flow_imp.F90:236-237): the
         // weights take the new hk; bndflux then writes the fluxes bndriver_vel wrote
         river_vel(F);
@@ -1064,6 +1064,35 @@ static void fill_geo(Geo &g, int nx, int ny, double dx, double dy, const int *si
         g.dsx[k] = g.fnx[k] * g.ds[k];
         g.dsy[k] = g.fny[k] * g.ds[k];
         g.side[k] = side[k];
+    }
+    // der_grad_cbgg's weights (flow_kernels.hip cbgg_grad): along an axis the other
+    // axis' faces weigh 0; weights below the screen (1e-8) are 0, the others
+    // less their mean
+    auto weights = [&](const double *ds, int plus, int minus, int b, double (&out)[3]) {
+        double w[3] = {0.0, 0.0, 0.0};
+        const int k[2] = {std::min(plus, minus), std::max(plus, minus)};   // faces in order
+        for (int q = 0; q < 2; q++) {
+            const int m = k[q] == plus ? 1 : 2;
+            if (b & m) {
+                w[0] += ds[k[q]] * (1.0 - g.fintp[k[q]]);
+                w[m] = ds[k[q]] * g.fintp[k[q]];
+            } else {
+                w[0] += ds[k[q]];
+            }
+        }
+        const double tolw = F4(1.0e-8);
+        int n = 0;
+        double sum = 0.0;
+        for (double &x : w) {
+            x /= g.area;
+            if (std::fabs(x) > tolw) { n++; sum += x; }
+        }
+        const double mean = n ? sum / (double)n : 0.0;
+        for (int q = 0; q < 3; q++) out[q] = std::fabs(w[q]) > tolw ? w[q] - mean : 0.0;
+    };
+    for (int b = 0; b < 4; b++) {
+        weights(g.dsx, KE, KW, b, g.gx[b]);
+        weights(g.dsy, KN, KS, b, g.gy[b]);
     }
 }
 
@@ -1125,7 +1154,7 @@ static int init_state(cms2d_flow *F) {
     HIPCHK(hipMemcpyAsync(s.h1, s.h, N * sizeof(double), hipMemcpyDeviceToDevice, F->st));
     if (int rc = wetdry(F)) return rc;
     HIPCHK(hipMemcpyAsync(s.iwet1, s.iwet, N, hipMemcpyDeviceToDevice, F->st));
-    LAUNCH(k_grad_fric_vis, F->nblk_act, g, s, F->P);
+    LAUNCH(k_grad_fric_vis, F->nblk_act, g, s, F->P, 1, 1);
     LAUNCH(k_convflux, F->nblk_act, g, s);
     HIPCHK(hipMemcpyAsync(s.fluxE1, s.fluxE, N * sizeof(double), hipMemcpyDeviceToDevice, F->st));
     HIPCHK(hipMemcpyAsync(s.fluxN1, s.fluxN, N * sizeof(double), hipMemcpyDeviceToDevice, F->st));

@@ -27,6 +27,9 @@ struct Geo {
     int nact;                 // nx*ny
     double dx, dy, area;
     double ds[4], dn[4], dsxy[4], fnx[4], fny[4], fintp[4], rx[4], ry[4], dsx[4], dsy[4];
+    // wet-only Green-Gauss weights of (cell, plus, minus neighbour) along x and y by
+    // the wet flags of the plus (1) and minus (2) neighbour
+    double gx[4][3], gy[4][3];
     int side[4];              // boundary type per side (CMS2D_BND_*)
 };
 

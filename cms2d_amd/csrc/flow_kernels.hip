@@ -77,8 +77,9 @@ __device__ __forceinline__ double length2drag(double z0, double h) {
 }
 // The per-law part of fric_eval (friction.F90:638-679): the law's input
 // (cfrict, z0, cbf or coefman) stays, the other coefficients follow from it
-// and the depth; returns the drag coefficient.
-__device__ __forceinline__ double fric_law(const Par &P, const St &s, int c, double h) {
+// and the depth; returns the drag coefficient.  z0: whether the roughness length
+// of Manning friction is wanted (an exponential, a square root and a division).
+__device__ __forceinline__ double fric_law(const Par &P, const St &s, int c, double h, bool z0 = true) {
     double cd;
     switch (P.mbedfric) {
     case 1:
@@ -100,7 +101,7 @@ __device__ __forceinline__ double fric_law(const Par &P, const St &s, int c, dou
     default:
         cd = man2drag(s.coefman[c], h);
         s.cfrict[c] = cd;
-        if (cd != 0.0) s.z0[c] = drag2length(cd, h);
+        if (z0 && cd != 0.0) s.z0[c] = drag2length(cd, h);
     }
     return cd;
 }
@@ -133,51 +134,31 @@ __device__ __forceinline__ void pad_ij(const Geo &g, int t, int &i, int &j) {
 
 // Cell-based Green-Gauss gradient with wet-only stencils (der_grad_cbgg with
 // gow%ibc=1, der_lib.f90:272-378, screened and re-centred as :360-376), then
-// der_grad_eval (:726-839).  Weights are rebuilt from iwet on every call,
-// which is what der_update keeps them equal to (derivatives.f90:204-296).
+// der_grad_eval (:726-839).  On a uniform grid the weights along x depend on
+// the wet flags of E and W alone, along y on N and S: fill_geo evaluates the
+// four cases of each once (Geo::gx, gy), and a cell picks its case instead of
+// rebuilding, dividing and screening ten weights.
+__device__ __forceinline__ double grad_axis(const double (&w)[4][3], int b, double vc, double vp, double vm) {
+    double a = 0.0;
+    const double wc = b & 1 ? (b & 2 ? w[3][0] : w[1][0]) : (b & 2 ? w[2][0] : w[0][0]);
+    const double wp = b & 1 ? (b & 2 ? w[3][1] : w[1][1]) : (b & 2 ? w[2][1] : w[0][1]);
+    const double wm = b & 1 ? (b & 2 ? w[3][2] : w[1][2]) : (b & 2 ? w[2][2] : w[0][2]);
+    if (wc != 0.0) a += wc * vc;
+    if (wp != 0.0) a += wp * vp;
+    if (wm != 0.0) a += wm * vm;
+    return a;
+}
 __device__ __forceinline__ void cbgg_grad(const Geo &g, const uint8_t *iwet, int c, int nv,
                                           const double *const *var, double *gx, double *gy) {
-    if (!iwet[c]) {
-        for (int q = 0; q < nv; q++) { gx[q] = 0.0; gy[q] = 0.0; }
-        return;
-    }
-    double wx[5] = {0, 0, 0, 0, 0}, wy[5] = {0, 0, 0, 0, 0};
-    int ix[5];
-    ix[0] = c;
-#pragma unroll
-    for (int k = 0; k < 4; k++) {
-        int nb = nbr(g, c, k);
-        ix[k + 1] = nb;
-        if (iwet[nb] == 1) {
-            wx[0] += g.dsx[k] * (1.0 - g.fintp[k]);
-            wx[k + 1] = g.dsx[k] * g.fintp[k];
-            wy[0] += g.dsy[k] * (1.0 - g.fintp[k]);
-            wy[k + 1] = g.dsy[k] * g.fintp[k];
-        } else {
-            wx[0] += g.dsx[k];
-            wy[0] += g.dsy[k];
-        }
-    }
-#pragma unroll
-    for (int k = 0; k < 5; k++) { wx[k] /= g.area; wy[k] /= g.area; }
-    const double tolw = F4(1.0e-8);
-    int nx_ = 0, ny_ = 0;
-    double sx = 0.0, sy = 0.0;
-#pragma unroll
-    for (int k = 0; k < 5; k++) {
-        if (fabs(wx[k]) > tolw) { nx_++; sx += wx[k]; }
-        if (fabs(wy[k]) > tolw) { ny_++; sy += wy[k]; }
-    }
-    double mx = nx_ ? sx / (double)nx_ : 0.0, my = ny_ ? sy / (double)ny_ : 0.0;
+    const int cN = c + g.nxp, cE = c + 1, cS = c - g.nxp, cW = c - 1;
+    const int bx = (iwet[cE] == 1) | (iwet[cW] == 1) << 1, by = (iwet[cN] == 1) | (iwet[cS] == 1) << 1;
+    const bool wet = iwet[c];
     for (int q = 0; q < nv; q++) {
-        double ax = 0.0, ay = 0.0;
-#pragma unroll
-        for (int k = 0; k < 5; k++) {
-            if (fabs(wx[k]) > tolw) ax += (wx[k] - mx) * var[q][ix[k]];
-            if (fabs(wy[k]) > tolw) ay += (wy[k] - my) * var[q][ix[k]];
-        }
-        gx[q] = ax;
-        gy[q] = ay;
+        const double vc = var[q][c];
+        const double ax = grad_axis(g.gx, bx, vc, var[q][cE], var[q][cW]);
+        const double ay = grad_axis(g.gy, by, vc, var[q][cN], var[q][cS]);
+        gx[q] = wet ? ax : 0.0;
+        gy[q] = wet ? ay : 0.0;
     }
 }
 
@@ -838,8 +819,6 @@ __global__ void k_pvfc1(Geo g, St s) {
     const double *vars[1] = {s.pp};
     double gx, gy;
     cbgg_grad(g, s.iwet, c, 1, vars, &gx, &gy);
-    s.dppx[c] = gx;
-    s.dppy[c] = gy;
     if (s.iwet[c] == 0) return;
     double val = s.h[c] * s.apuareap[c] / (1.0 - s.sumu[c] + SMALL);
     s.u[c] = s.u[c] - val * gx;
@@ -889,21 +868,26 @@ __global__ void k_ghost_p(Geo g, St s, Par P) {
 
 // flow_grad_interp (flow_imp.F90:1106-1127) + fric_eval (friction.F90:615-797,
 // Manning) + flow_eddyvis cell values (flow_eddyvis.f90:128-160, mturbul=5).
-__global__ void k_grad_fric_vis(Geo g, St s, Par P) {
+// all: also what only the initial state needs (k_velface gives a step's final
+// uv, bsvel and z0; between outer iterations z0 is read next to dry cells, by
+// the wall friction).  grads: the gradients are kept (statistics).
+__global__ void k_grad_fric_vis(Geo g, St s, Par P, int all, int grads) {
     int i, j, c;
     if (!act_thread(g, i, j, c)) return;
     const double *vars[2] = {s.u, s.v};
     double gx[2], gy[2];
     cbgg_grad(g, s.iwet, c, 2, vars, gx, gy);
-    s.dux[c] = gx[0]; s.duy[c] = gy[0]; s.dvx[c] = gx[1]; s.dvy[c] = gy[1];
+    if (grads) { s.dux[c] = gx[0]; s.duy[c] = gy[0]; s.dvx[c] = gx[1]; s.dvy[c] = gy[1]; }
     // interp_scal_cell2face(p, ibc=1)
     const double pc = s.p[c];
     const int wc = s.iwet[c];
+    bool wall = false;
     double sx = 0.0, sy = 0.0, hkv[4];
 #pragma unroll
     for (int k = 0; k < 4; k++) {
         int nb = nbr(g, c, k);
         int wn = s.iwet[nb];
+        wall = wall || wn == 0;
         double pk;
         if (wc * wn == 1) pk = g.fintp[k] * s.p[nb] + (1.0 - g.fintp[k]) * pc;
         else if (wc == 1) pk = pc;
@@ -921,7 +905,7 @@ __global__ void k_grad_fric_vis(Geo g, St s, Par P) {
     if (i == 0) s.hkE[c - 1] = hkv[KW];
     // fric_eval
     double h = s.h[c], u = s.u[c], v = s.v[c];
-    double cd = fric_law(P, s, c, h);
+    double cd = fric_law(P, s, c, h, all || wall);
     double Um, Uwc, taum;
     if (P.noptset >= 3) {
         double Um2 = u * u + v * v;
@@ -934,7 +918,8 @@ __global__ void k_grad_fric_vis(Geo g, St s, Par P) {
         taum = RHOW * cd * Um * Um;
     }
     double bsvel = sqrt(taum / RHOW + F4(1.0e-15));
-    s.uv[c] = Um; s.uelwc[c] = Uwc; s.bsvel[c] = bsvel;
+    s.uelwc[c] = Uwc;
+    if (all) { s.uv[c] = Um; s.bsvel[c] = bsvel; }
     // eddy viscosity, cell value (flow_eddyvis.f90:23-160): TURBULENCE_MODEL
     // CONSTANT (0), FALCONER (1), PARABOLIC (2), SUBGRID-WU (3), SUBGRID (5);
     // the coefficients keep their mturbul-5 defaults (flow.F90:81-92)
@@ -1299,7 +1284,7 @@ __global__ void k_update(Geo g, St s) {
     s.iwet1[t] = s.iwet[t];
     s.u1[t] = s.u[t]; s.v1[t] = s.v[t]; s.p1[t] = s.p[t]; s.h1[t] = s.h[t];
     s.fluxE1[t] = s.fluxE[t]; s.fluxN1[t] = s.fluxN[t];
-    s.pp[t] = 0.0; s.dppx[t] = 0.0; s.dppy[t] = 0.0;
+    s.pp[t] = 0.0;
     s.maxeta[t] = fmax(s.eta[t], s.maxeta[t]);   // maximum water level, CMS_Flow.f90:352-355
 }
 
@@ -1308,7 +1293,7 @@ __global__ void k_recalc(Geo g, St s) {
     int t = blockIdx.x * blockDim.x + threadIdx.x;
     if (t >= g.nxp * g.nyp) return;
     s.u[t] = s.u1[t]; s.v[t] = s.v1[t]; s.p[t] = s.p1[t]; s.h[t] = s.h1[t];
-    s.pp[t] = 0.0; s.dppx[t] = 0.0; s.dppy[t] = 0.0;
+    s.pp[t] = 0.0;
     s.iwet[t] = s.iwet1[t];
     s.fluxE[t] = s.fluxE1[t]; s.fluxN[t] = s.fluxN1[t];
 }
