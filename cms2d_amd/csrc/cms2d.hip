@@ -1001,7 +1001,7 @@ static int flow_imp_once(cms2d_flow *F) {
             const bool curve = F->side_type[sd] == CMS2D_BND_WSE_CURVE;
             hipLaunchKernelGGL(k_wse_adjust, dim3(1), dim3(1024), n * sizeof(double), F->st, g, s, F->P, sd,
                                curve ? wsecurve : w, ramp, curve ? F->wse_gx : 0.0, curve ? F->wse_gy : 0.0,
-                               (int)(curve && F->wse_adjust_off));
+                               (int)((curve && F->wse_adjust_off) || !wse_forced(F->P)));
         }
         hipLaunchKernelGGL(k_pp_src, dim3(F->nblk_kry), dim3(KBLOCK), 0, F->st, g, s, F->P, F->Kpp);
         TAPE(TAPE_PPSRC);

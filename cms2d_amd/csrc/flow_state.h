@@ -33,5 +33,10 @@ struct Par {
     int mturbul;               // turbulence model (flow_eddyvis.f90:23-160)
     int mbedfric;              // bottom friction law (fric_eval, friction.F90:638-688)
 };
+// Whether wave or wind stress sets the water level up along a string
+// (bnd_wse_adjust): without either every term of its sums is 0.
+__host__ __device__ inline bool wse_forced(const Par &P) {
+    return P.noptset >= 3 || P.tauwx != 0.0 || P.tauwy != 0.0;
+}
 
 }  // namespace cms

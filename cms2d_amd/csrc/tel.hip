@@ -94,27 +94,37 @@ __global__ void __launch_bounds__(BLOCK) k_tl_mg_setup0(TelG T, const int *blk, 
 }
 
 // The residual r - A Z of cell i for a correction Z that is nonzero on
-// refined cells only (so only cells next to them see it); the face loads
-// are issued together (every slot, predicated) and summed in face order.
+// refined cells only (so only cells next to them see it), summed in face order.
+// The refined region is small and these sweeps wait for memory, not for
+// bandwidth: everything that cell i itself selects is fetched at once (the
+// slots past the last face hold -1), then Z at the neighbours.  (Slots fetched
+// after the cell's bits: 19 us a restriction of 120 thousand refined cells.)
 template <class TB>
 __device__ __forceinline__ double tl_res(const TelG &T, const TB *r, const double *ap, const double *apc,
-                                         const float *Z, int i, uint64_t m) {
-    double ri = (double)r[i];
-    if (m_near(m)) {
-        const int nf = m_ncf(m);
-        int nbk[TF];
-        float zk[TF];
+                                         const float *Z, int i) {
+    const uint64_t m = T.meta[i];
+    const double ri = (double)r[i];
+    int nbk[TF];
+    double a[TF];
+    float zk[TF];
 #pragma unroll
-        for (int k = 0; k < TF; k++) nbk[k] = k < nf ? tnb(T, i, k) : T.n;
+    for (int k = 0; k < TF; k++) nbk[k] = tnb(T, i, k);
 #pragma unroll
-        for (int k = 0; k < TF; k++) zk[k] = nbk[k] < T.n ? Z[nbk[k]] : 0.0f;
-        double az = ap[i] * (double)Z[i];
+    for (int k = 0; k < TF; k++) a[k] = apc[k * T.nd + i];
+    const double api = ap[i];
+    const float zi = Z[i];
+    if (!m_near(m)) return ri;
 #pragma unroll
-        for (int k = 0; k < TF; k++)
-            if (nbk[k] < T.n) az -= apc[k * T.nd + i] * (double)zk[k];
-        ri -= az;
+    for (int k = 0; k < TF; k++) {
+        const bool in = nbk[k] >= 0 && nbk[k] < T.n;
+        nbk[k] = in ? nbk[k] : -1;
+        zk[k] = Z[in ? nbk[k] : i];
     }
-    return ri;
+    double az = api * (double)zi;
+#pragma unroll
+    for (int k = 0; k < TF; k++)
+        if (nbk[k] >= 0) az -= a[k] * (double)zk[k];
+    return ri - az;
 }
 
 // Coefficients of level k from the cell list's pp system (once per outer iteration).
@@ -152,26 +162,35 @@ __global__ void k_tl_cs_pre2(TelG T, const int *ref, int nref, const uint8_t *le
     const int t = blockIdx.x * blockDim.x + threadIdx.x;
     if (t >= nref) return;
     const int i = ref[t];
-    if (lev[i] != top) {
+    const bool on = lev[i] == top;
+    int nbk[TF];
+    double a[TF], rk[TF], dk[TF];
+#pragma unroll
+    for (int k = 0; k < TF; k++) nbk[k] = tnb(T, i, k);
+#pragma unroll
+    for (int k = 0; k < TF; k++) a[k] = apc[k * T.nd + i];
+    const double ri = (double)r[i], api = ap[i];
+    if (!on) {
         Z[i] = 0.0f;
         return;
     }
-    auto z1 = [&](int x) { return lev[x] == top ? TEL_OMEGA * (float)((double)r[x] / ap[x]) : 0.0f; };
-    const uint64_t m = T.meta[i];
-    const int nf = m_ncf(m);
-    int nbk[TF];
-    float zk[TF];
+    uint8_t lk[TF];
 #pragma unroll
-    for (int k = 0; k < TF; k++) nbk[k] = k < nf ? tnb(T, i, k) : T.n;
-#pragma unroll
-    for (int k = 0; k < TF; k++) zk[k] = nbk[k] < T.n ? z1(nbk[k]) : 0.0f;
-    const float zi = z1(i);
-    double az = ap[i] * (double)zi;
+    for (int k = 0; k < TF; k++) {
+        const bool in = nbk[k] >= 0 && nbk[k] < T.n;
+        nbk[k] = in ? nbk[k] : -1;
+        const int x = in ? nbk[k] : i;
+        rk[k] = (double)r[x];
+        dk[k] = ap[x];
+        lk[k] = lev[x];
+    }
+    const float zi = TEL_OMEGA * (float)(ri / api);
+    double az = api * (double)zi;
 #pragma unroll
     for (int k = 0; k < TF; k++)
-        if (nbk[k] < T.n) az -= apc[k * T.nd + i] * (double)zk[k];
-    const double res = (double)r[i] - az;
-    Z[i] = zi + TEL_OMEGA * (float)(res / ap[i]);
+        if (nbk[k] >= 0) az -= a[k] * (double)(lk[k] == top ? TEL_OMEGA * (float)(rk[k] / dk[k]) : 0.0f);
+    const double res = ri - az;
+    Z[i] = zi + TEL_OMEGA * (float)(res / api);
 }
 // A damped Jacobi sweep on the finest cells: zout = zin + omega D^-1 (r - A zin)
 template <class TB>
@@ -181,7 +200,7 @@ __global__ void k_tl_cs_fjac(TelG T, const int *top, int ntop, const TB *r, cons
     const int t = blockIdx.x * blockDim.x + threadIdx.x;
     if (t >= ntop) return;
     const int i = top[t];
-    const double res = tl_res(T, r, ap, apc, zin, i, T.meta[i]);
+    const double res = tl_res(T, r, ap, apc, zin, i);
     zout[i] = zin[i] + TEL_OMEGA * (float)(res / ap[i]);
 }
 // Residual r - A Z summed into the level-k squares, and the first sweep from
@@ -194,19 +213,23 @@ __global__ void __launch_bounds__(BLOCK) k_tl_cs_restrict(TelG T, TelLev V, cons
     __shared__ double sr[BLOCK];
     const int q0 = V.blk[blockIdx.x], q1 = V.blk[blockIdx.x + 1], q = q0 + threadIdx.x;
     double ri = 0.0;
-    int c = 0;
+    int c = 0, first = -1, last = 0;
+    float dinv = 0.0f;
     if (q < q1) {
         const int i = V.kcell[q];
-        ri = tl_res(T, r, ap, apc, Z, i, T.meta[i]);
         c = V.kseg[q];
+        first = V.kstart[c];
+        last = V.kstart[c + 1];
+        dinv = V.dinv[c];
+        ri = tl_res(T, r, ap, apc, Z, i);
     }
     sr[threadIdx.x] = ri;
     __syncthreads();
-    if (q >= q1 || V.kstart[c] != q) return;
+    if (first != q) return;
     double acc = 0.0;
-    for (int p = q; p < V.kstart[c + 1]; p++) acc += sr[p - q0];
+    for (int p = q; p < last; p++) acc += sr[p - q0];
     V.r[c] = (float)acc;
-    V.z[c] = TEL_OMEGA * (float)acc * V.dinv[c];
+    V.z[c] = TEL_OMEGA * (float)acc * dinv;
 }
 // The second sweep on level k (from the first, z0) and its correction added
 // to the cells inside each square (Z1, and Z2 if given).
@@ -254,19 +277,20 @@ __global__ void __launch_bounds__(BLOCK) k_tl_mg_restrict(TelG T, const int *blk
         }
         return;
     }
-    int i = 0;
+    int b = 0, first = -1, last = 0;
     double ri = 0.0;
     if (q < q1) {
-        i = bcells[q];
-        ri = tl_res(T, r, ap, apc, Z, i, T.meta[i]);
+        const int i = bcells[q];
+        b = T.base[i];
+        first = T.bstart[b];
+        last = T.bstart[b + 1];
+        ri = tl_res(T, r, ap, apc, Z, i);
     }
     sr[threadIdx.x] = ri;
     __syncthreads();
-    if (q >= q1) return;
-    const int b = T.base[i];
-    if (T.bstart[b] != q) return;
+    if (first != q) return;
     double acc = 0.0;
-    for (int p = q; p < T.bstart[b + 1]; p++) acc += sr[p - q0];
+    for (int p = q; p < last; p++) acc += sr[p - q0];
     b0[L.idx(b % T.nbx, b / T.nbx)] = (float)acc;
 }
 // z = Z + P zb on every cell, into both buffers of the up sweeps (a block of
@@ -305,6 +329,7 @@ struct TelHost {
     float *zp = nullptr;                  // correction of the down sweeps (0 on unrefined cells)
     float *zq = nullptr;                  // second buffer of the up sweeps
     float *apc32 = nullptr;               // FP32 coefficients of the FP32 form's current inner solve (u/v, then pp)
+    int4 *run = nullptr;                  // neighbour offsets of the operator's chunks (TelOpT)
     int *bcells = nullptr;
     int *blkb = nullptr, nblkb = 0;       // blocks of the base restriction (whole base cells)
     int *plainb = nullptr, *plainc = nullptr;   // first base cell of a plain block (see k_tl_mg_restrict), or -1
@@ -452,7 +477,7 @@ struct TelInnerPre {
     }
 };
 
-static TelOp tel_op(const TelHost &H, const double *a) { return TelOp{H.T.n, H.T.nd, H.T.c2c, H.T.meta, a}; }
+static TelOp tel_op(const TelHost &H, const double *a) { return TelOp{H.T.n, H.T.nd, H.T.c2c, H.T.meta, H.run, a}; }
 
 // The BiCGStab pairs of the u/v and pp systems, captured once at creation
 // (the pp pair's timed-group launches noted for the launch counts).
@@ -463,7 +488,7 @@ static int tel_capture_graphs(cms2d_flow *F) {
     if (F->precision == CMS2D_PREC_FP32_REFINE) {
         // the inner FP32 pairs of the refinement form (u and v; pp), on the
         // FP32 coefficients converted before each of their solves
-        const TelOp32 A32{H.T.n, H.T.nd, H.T.c2c, H.T.meta, H.apc32};
+        const TelOp32 A32{H.T.n, H.T.nd, H.T.c2c, H.T.meta, H.run, H.apc32};
         if (int rc = capture_bicg_pair<TelOp32, 2, 0, float>(inner_ctx(X), F->Kin2, A32, F->kgraph[4])) return rc;
         return capture_bicg_pair<TelOp32, 1, 1, float>(inner_ctx(X), F->Kin, A32, F->kgraph[3], TelInnerPre{F});
     }
@@ -510,7 +535,7 @@ static int tel_uv_solve_refine(cms2d_flow *F, KryCtx &X, const TelOp &A) {
     TLAUNCH(k_tl_uv_to32, H.nblk_nd, H.T, (const double *)H.s.am, K, H.apc32, Ki);
     HIPCHK(hipMemcpyAsync(F->h_sc + 1, F->d_sc + 1, 2 * sizeof(KryScal), hipMemcpyDeviceToHost, F->st));
     HIPCHK(hipStreamSynchronize(F->st));
-    const TelOp32 A32{H.T.n, H.T.nd, H.T.c2c, H.T.meta, H.apc32};
+    const TelOp32 A32{H.T.n, H.T.nd, H.T.c2c, H.T.meta, H.run, H.apc32};
     KryCtx Xi = inner_ctx(X);
     Xi.rtol = REF_RTOL_UV;
     int total[2] = {0, 0};
@@ -542,7 +567,7 @@ static int tel_pp_solve_refine(cms2d_flow *F, KryCtx &X, const TelOp &A) {
     TLAUNCH(k_tl_to32, H.nblk_nd, H.T, (const double *)H.s.apc, (const double *)K.ap_w[0], H.apc32, Ki.ap_w[0]);
     HIPCHK(hipMemcpyAsync(F->h_sc, F->d_sc, sizeof(KryScal), hipMemcpyDeviceToHost, F->st));
     HIPCHK(hipStreamSynchronize(F->st));
-    const TelOp32 A32{H.T.n, H.T.nd, H.T.c2c, H.T.meta, H.apc32};
+    const TelOp32 A32{H.T.n, H.T.nd, H.T.c2c, H.T.meta, H.run, H.apc32};
     KryCtx Xi = inner_ctx(X);
     TelInnerPre pre{F};
     int total = 0;
@@ -622,7 +647,7 @@ static int tel_flow_imp(cms2d_flow *F) {
                 (const double *)H.gap[0][H.cap], (const double *)H.gap[1][H.cap]);
         if (T.nstr > 0)
             hipLaunchKernelGGL(k_tl_wse_adjust, dim3(1), dim3(1024), T.nstr * sizeof(double), F->st, T, s, F->P, w,
-                               F->ramp, (int)!(F->wse_adjust_off && !F->wse_t.empty()));
+                               F->ramp, (int)(!(F->wse_adjust_off && !F->wse_t.empty()) && wse_forced(F->P)));
         hipLaunchKernelGGL(k_tl_pp_src, dim3(F->nblk_kry), dim3(KBLOCK), 0, F->st, T, s, F->P, H.Kpp, Ap,
                            (const double *)H.gpp[0][H.cpp], (const double *)H.gpp[1][H.cpp]);
         {
@@ -1092,6 +1117,18 @@ static int tel_create(const cms2d_flow_desc *d, const cms2d_tel_grid *tg, cms2d_
         if (near) m |= 1ull << 41;
         m |= (uint64_t)strmask[i] << 42;
         m |= (uint64_t)qmask[i] << 48;
+        bool plain = t.ncf[i] == 4;
+        for (int k = 0; k < t.ncf[i]; k++) {
+            const size_t f = (size_t)k * nd + i;
+            const int nb = t.c2c[f], dr = t.dir[f];
+            const bool ns = dr == KN || dr == KS;
+            const bool even = t.dx[nb] == t.dx[i] && t.dy[nb] == t.dy[i] &&
+                              (ns ? t.x[nb] == t.x[i] && std::fabs(t.y[nb] - t.y[i]) == t.dy[i]
+                                  : t.y[nb] == t.y[i] && std::fabs(t.x[nb] - t.x[i]) == t.dx[i]);
+            if (even) m |= 1ull << (54 + k);
+            plain = plain && even && dr == k;
+        }
+        if (plain) m |= 1ull << 60;
         meta[i] = m;
     }
 
@@ -1120,6 +1157,26 @@ static int tel_create(const cms2d_flow_desc *d, const cms2d_tel_grid *tg, cms2d_
     uint8_t *gw;
     if (int rc = tel_upload(F, &c2c, t.c2c.data(), t.c2c.size())) return rc;
     if (int rc = tel_upload(F, &met, meta.data(), meta.size())) return rc;
+    {
+        // chunks of 64 cells of four faces whose neighbours, all cells, lie at
+        // the same four offsets in the list from each (x = 0: not such a chunk)
+        std::vector<int4> run((n + 63) / 64, make_int4(0, 0, 0, 0));
+        for (int q = 0; (q + 1) * 64 <= n; q++) {
+            const int i0 = q * 64;
+            int off[4];
+            for (int k = 0; k < 4; k++) off[k] = t.c2c[(size_t)k * nd + i0] - i0;
+            bool same = true;
+            for (int i = i0; same && i < i0 + 64; i++) {
+                same = t.ncf[i] == 4;
+                for (int k = 0; same && k < 4; k++) {
+                    const int nb = t.c2c[(size_t)k * nd + i];
+                    same = nb < n && nb - i == off[k];
+                }
+            }
+            if (same) run[q] = make_int4(off[0], off[1], off[2], off[3]);
+        }
+        if (int rc = tel_upload(F, &H.run, run.data(), run.size())) return rc;
+    }
     if (int rc = tel_upload(F, &xx, t.x.data(), (size_t)nd)) return rc;
     if (int rc = tel_upload(F, &yy, t.y.data(), (size_t)nd)) return rc;
     if (int rc = tel_upload(F, &ddx, t.dx.data(), (size_t)nd)) return rc;

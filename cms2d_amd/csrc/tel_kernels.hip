@@ -21,8 +21,14 @@ namespace cms {
 
 constexpr int TF = 6;   // nmaxfaces of a telescoping grid (geospatial.F90:433)
 
-// Per-cell bits: ncface, the face directions (0..3 = N,E,S,W), llec2llec, the
-// faces the cell owns, joint, and the multigrid smoothing flags.
+// Per-cell bits: ncface (4 to 6), the face directions (0..3 = N,E,S,W),
+// llec2llec, the faces the cell owns, joint, the multigrid smoothing flags,
+// the cellstring faces, the even faces (bit 54+k: the neighbour has this cell's
+// size and lies on its axis at that distance, each to the last bit) and the
+// plain cells (bit 60: four even faces in slots N,E,S,W).  An even face's
+// geometry is a function of the cell's own size, so it takes no load of the
+// neighbour's centre and size; a grid whose centres are rounded keeps the
+// general form for the faces where they do not compare equal.
 __device__ __forceinline__ int m_ncf(uint64_t m) { return (int)(m & 7u); }
 __device__ __forceinline__ int m_dir(uint64_t m, int k) { return (int)((m >> (3 + 2 * k)) & 3u); }
 __device__ __forceinline__ int m_llec(uint64_t m, int k) { return (int)((m >> (15 + 3 * k)) & 7u); }
@@ -32,6 +38,9 @@ __device__ __forceinline__ bool m_smooth(uint64_t m) { return (m >> 40) & 1u; }
 __device__ __forceinline__ bool m_near(uint64_t m) { return (m >> 41) & 1u; }
 __device__ __forceinline__ bool m_str(uint64_t m, int k) { return (m >> (42 + k)) & 1u; }
 __device__ __forceinline__ bool m_qstr(uint64_t m, int k) { return (m >> (48 + k)) & 1u; }   // flux string
+__device__ __forceinline__ bool m_strs(uint64_t m) { return (m >> 42) & 0xfffu; }             // any string face
+__device__ __forceinline__ bool m_even(uint64_t m, int k) { return (m >> (54 + k)) & 1u; }
+__device__ __forceinline__ bool m_plain(uint64_t m) { return (m >> 60) & 1u; }
 
 // Topology and geometry (device pointers).
 struct TelG {
@@ -81,9 +90,58 @@ __device__ __forceinline__ FGeo fgeo(const TelG &T, int i, int nb, int d) {
     else f.fintp = dxi / (dxi + dxn);
     return f;
 }
+// The same of face k of a cell with bits m, from the cell's own size where the
+// face is even.
+__device__ __forceinline__ FGeo fgeo(const TelG &T, int i, int nb, uint64_t m, int k) {
+    const int d = m_dir(m, k);
+    if (!m_even(m, k)) return fgeo(T, i, nb, d);
+    FGeo f;
+    const double dxi = T.dx[i], dyi = T.dy[i];
+    const bool ns = d == KN || d == KS;
+    f.ds = ns ? dxi : dyi;
+    f.dn = ns ? dyi : dxi;
+    f.fnx = d == KE ? 1 : d == KW ? -1 : 0;
+    f.fny = d == KN ? 1 : d == KS ? -1 : 0;
+    f.rx = f.fnx * (dxi / 2.0);
+    f.ry = f.fny * (dyi / 2.0);
+    f.rpx = f.rx - f.fnx * fabs(f.rx);
+    f.rpy = f.ry - f.fny * fabs(f.ry);
+    f.dsx = f.fnx * f.ds;
+    f.dsy = f.fny * f.ds;
+    f.dsxy = f.ds / f.dn;
+    f.fintp = 0.5;
+    return f;
+}
 // The perpendicular offset rp used by the skewness terms of face (i, k):
 // rpy on x faces, rpx on y faces.  Ghost faces carry none.
 __device__ __forceinline__ double rp_of(const FGeo &f, int d) { return (d == KE || d == KW) ? f.rpy : f.rpx; }
+
+// v(k) of the faces of a cell.  Every cell has at least four (a ghost on a side
+// without a neighbour), so the first four are fetched together, without a
+// branch between, before any of them is used: a loop over the faces waits for
+// each in turn.  The last two are those of a joint cell.
+template <class V, class F>
+__device__ __forceinline__ void tel_fetch(int nf, V (&a)[TF], F &&v) {
+#pragma unroll
+    for (int k = 0; k < 4; k++) a[k] = v(k);
+#pragma unroll
+    for (int k = 4; k < TF; k++) a[k] = V(0);
+    if (nf > 4) {
+#pragma unroll
+        for (int k = 4; k < TF; k++)
+            if (k < nf) a[k] = v(k);
+    }
+}
+template <class F>
+__device__ __forceinline__ void tel_faces(int nf, F &&f) {
+#pragma unroll
+    for (int k = 0; k < 4; k++) f(k);
+    if (nf > 4) {
+#pragma unroll
+        for (int k = 4; k < TF; k++)
+            if (k < nf) f(k);
+    }
+}
 
 // Device state of a telescoping flow.
 struct TelS {
@@ -122,6 +180,37 @@ __device__ __forceinline__ void tel_grad(const TelG &T, const uint8_t *iwet, int
     const int nf = m_ncf(m);
 #pragma unroll
     for (int q = 0; q < NV; q++) { gx[q] = 0.0; gy[q] = 0.0; }
+    if (m_plain(m)) {
+        // Four even faces: between neighbours that all count, the weights are
+        // +-ds/(2 area) across the cell and 0 on the cell itself, and the four
+        // neighbours' values are fetched together with their flags.  (The form
+        // below loads face after face and divides seven times: 500 -> 180 us
+        // for three fields of 2.8 M cells, nearly all of them plain.)
+        int nb[4];
+#pragma unroll
+        for (int k = 0; k < 4; k++) nb[k] = tnb(T, i, k);
+        const int w0 = iwet[i];
+        const double dx = T.dx[i], dy = T.dy[i];
+        int w[4];
+#pragma unroll
+        for (int k = 0; k < 4; k++) w[k] = iwet[nb[k]];
+        double val[NV][4];
+#pragma unroll
+        for (int q = 0; q < NV; q++)
+#pragma unroll
+            for (int k = 0; k < 4; k++) val[q][k] = var[q][nb[k]];
+        if (w0 == 0 && ibc == 1) return;
+        if (ibc == 0 || (w[0] & w[1] & w[2] & w[3]) == 1) {
+            const double area = dx * dy, wx = dy * 0.5 / area, wy = dx * 0.5 / area;
+            const double tolw = F4(1.0e-8);
+#pragma unroll
+            for (int q = 0; q < NV; q++) {
+                if (wx > tolw) gx[q] = wx * val[q][KE] + -wx * val[q][KW];
+                if (wy > tolw) gy[q] = wy * val[q][KN] + -wy * val[q][KS];
+            }
+            return;
+        }
+    }
     if (iwet[i] == 0 && ibc == 1) return;
     const double area = T.dx[i] * T.dy[i];
     double wx[TF + 1], wy[TF + 1];
@@ -132,7 +221,7 @@ __device__ __forceinline__ void tel_grad(const TelG &T, const uint8_t *iwet, int
         wx[k + 1] = 0.0; wy[k + 1] = 0.0; ix[k + 1] = i;
         if (k >= nf) continue;
         const int nb = tnb(T, i, k), d = m_dir(m, k);
-        const FGeo f = fgeo(T, i, nb, d);
+        const FGeo f = fgeo(T, i, nb, m, k);
         ix[k + 1] = nb;
         if (iwet[nb] == 1 || ibc == 0) {
             wx[0] += f.dsx * (1.0 - f.fintp);
@@ -186,7 +275,7 @@ __device__ __forceinline__ void tel_grad(const TelG &T, const uint8_t *iwet, int
         if (nb >= T.n) continue;
         if (xd ? fabs(T.dy[i] / T.dy[nb] - 1.0) < F4(0.1) : fabs(T.dx[i] / T.dx[nb] - 1.0) < F4(0.1)) continue;
         if (iwet[nb] == 0 && ibc == 1) continue;
-        const FGeo f = fgeo(T, i, nb, d);
+        const FGeo f = fgeo(T, i, nb, m, k);
         const FGeo b = fgeo(T, nb, i, (d + 2) & 3);
         if (xd) {
             wxy[0] += f.dsx * (1.0 - f.fintp) * f.rpy / area;
@@ -469,12 +558,16 @@ __global__ void k_tl_mom(TelG T, TelS s, Par P) {
     const double cb = 1.0 * s.cfrict[i] * s.uelwc[i] * area;
     s.sp[i] = s.spuv0[i] - cb;
     const uint64_t m = T.meta[i];
-    for (int k = 0; k < m_ncf(m); k++) {
-        const int f = k * T.nd + i, nb = tnb(T, i, k);
-        const FGeo g = fgeo(T, i, nb, m_dir(m, k));
-        const double ddk = s.visk[f] * s.hk[f] * g.dsxy;
-        s.am[f] = schmcoef(P.ndsch, ddk, s.flux[f]);
-    }
+    const int nf = m_ncf(m);
+    double vk[TF], hk[TF], fl[TF];
+    tel_fetch(nf, vk, [&](int k) { return s.visk[k * T.nd + i]; });
+    tel_fetch(nf, hk, [&](int k) { return s.hk[k * T.nd + i]; });
+    tel_fetch(nf, fl, [&](int k) { return s.flux[k * T.nd + i]; });
+    tel_faces(nf, [&](int k) {
+        const FGeo g = fgeo(T, i, tnb(T, i, k), m, k);
+        const double ddk = vk[k] * hk[k] * g.dsxy;
+        s.am[k * T.nd + i] = schmcoef(P.ndsch, ddk, fl[k]);
+    });
 }
 
 // defcorparagradvec (computational.F90:149-264) on joint cells: the deferred
@@ -487,7 +580,7 @@ __device__ __forceinline__ bool tl_skew_face(const TelG &T, const TelS &s, const
     if (!m_joint(m) || s.iwet[o] == 0) return false;
     const int nb = tnb(T, o, k), d = m_dir(m, k);
     if (nb >= T.n || s.iwet[nb] == 0) return false;
-    const FGeo f = fgeo(T, o, nb, d), b = fgeo(T, nb, o, (d + 2) & 3);
+    const FGeo f = fgeo(T, o, nb, m, k), b = fgeo(T, nb, o, (d + 2) & 3);
     const bool xd = d == KE || d == KW;
     const double rpi = rp_of(f, d), rpn = rp_of(b, d);
     const int fo = k * T.nd + o;
@@ -534,21 +627,22 @@ __global__ void k_tl_bound_uv(TelG T, TelS s, Par P) {
     const uint64_t m = T.meta[i];
     const int nf = m_ncf(m);
     double sp = s.sp[i];
+    const bool strs = m_strs(m);
     // flux string first (bound_uv's order): bnd_vel_flux (bnd_vel.f90:2-32)
-    for (int k = 0; k < nf; k++) {
+    for (int k = 0; strs && k < nf; k++) {
         if (!m_qstr(m, k)) continue;
         const int f = k * T.nd + i, nb = tnb(T, i, k);
-        const FGeo g = fgeo(T, i, nb, m_dir(m, k));
+        const FGeo g = fgeo(T, i, nb, m, k);
         const double a = schmcoef(1, s.visk[f] * s.hk[f] * g.dsxy, s.flux[f]);
         s.su[i] = s.su[i] + a * s.u[nb];
         s.sv[i] = s.sv[i] + a * s.v[nb];
         sp = sp - a;
         s.am[f] = 0.0;
     }
-    for (int k = 0; k < nf; k++) {
+    for (int k = 0; strs && k < nf; k++) {
         if (!m_str(m, k)) continue;
         const int f = k * T.nd + i, nb = tnb(T, i, k);
-        const FGeo g = fgeo(T, i, nb, m_dir(m, k));
+        const FGeo g = fgeo(T, i, nb, m, k);
         const double ddk = s.visk[f] * s.hk[f] * g.dsxy;
         const double a = schmcoef(1, ddk, s.flux[f]);
         if (fabs(g.fny) > F4(0.9999)) {
@@ -569,10 +663,16 @@ __global__ void k_tl_bound_uv(TelG T, TelS s, Par P) {
     if (P.wallfric) {
         if (w == 1) {
             double spu = sp, spv = sp;
-            for (int k = 0; k < nf; k++) {
+            int nbs[TF], wn[TF];
+            tel_fetch(nf, nbs, [&](int k) { return tnb(T, i, k); });
+            tel_fetch(nf, wn, [&](int k) { return (int)s.iwet[nbs[k]]; });
+            bool dry = false;
+#pragma unroll
+            for (int k = 0; k < TF; k++) dry = dry || (k < nf && wn[k] == 0);
+            for (int k = 0; dry && k < nf; k++) {
                 const int f = k * T.nd + i, nb = tnb(T, i, k);
                 if (s.iwet[nb] != 0) continue;
-                const FGeo g = fgeo(T, i, nb, m_dir(m, k));
+                const FGeo g = fgeo(T, i, nb, m, k);
                 const double z0w = s.z0[i] * 1.0;
                 if (fabs(g.fny) > F4(0.999)) spu -= g.ds * s.hk[f] * wall_coef(fabs(g.ry), z0w) * fabs(s.u[i]);
                 else spv -= g.ds * s.hk[f] * wall_coef(fabs(g.rx), z0w) * fabs(s.v[i]);
@@ -601,6 +701,10 @@ struct TelOpT {
     int nc, nd;
     const int *c2c;
     const uint64_t *meta;
+    // [ceil(n/64)] offsets of the four neighbours from each cell of a chunk of
+    // 64 (x = 0: they differ): one wave's cells, in place of 24 B a cell of
+    // slots and bits (84 -> 60 B a cell in the sweeps of the pp solve).
+    const int4 *run;
     const CA *a;                 // [TF*nd]
     __host__ __device__ __forceinline__ int n() const { return nc; }
     // Passes over the list in order: in pass p the blocks take consecutive
@@ -636,19 +740,26 @@ struct TelOpT {
     template <int NS, class V, class Get>
     __device__ __forceinline__ void sums(const Idx &x, Get &&get, V (&sum)[NS]) const {
         const int c = x.c;
-        const int nf = m_ncf(meta[c]);
-        int nb[4];
+        const int4 o = run[__builtin_amdgcn_readfirstlane(c >> 6)];
+        int nb[4], nf = 4;
         V w[4];
+        if (o.x) {
+            nb[0] = c + o.x; nb[1] = c + o.y; nb[2] = c + o.z; nb[3] = c + o.w;
 #pragma unroll
-        for (int k = 0; k < 4; k++) {
-            nb[k] = c2c[k * nd + c];
-            w[k] = (V)a[k * nd + c];
-        }
+            for (int k = 0; k < 4; k++) w[k] = (V)a[k * nd + c];
+        } else {
+            nf = m_ncf(meta[c]);
 #pragma unroll
-        for (int k = 0; k < 4; k++) {
-            const bool in = k < nf && nb[k] < nc;
-            nb[k] = in ? nb[k] : c;
-            w[k] = in ? w[k] : V(0);
+            for (int k = 0; k < 4; k++) {
+                nb[k] = c2c[k * nd + c];
+                w[k] = (V)a[k * nd + c];
+            }
+#pragma unroll
+            for (int k = 0; k < 4; k++) {
+                const bool in = nb[k] < nc;
+                nb[k] = in ? nb[k] : c;
+                w[k] = in ? w[k] : V(0);
+            }
         }
         V z[NS][4];
 #pragma unroll
@@ -696,8 +807,13 @@ __global__ void __launch_bounds__(KBLOCK) k_tl_uv_prologue(TelG T, TelS s, KrySy
         const int c = x_.c;
         const uint64_t m = T.meta[c];
         const int nf = m_ncf(m);
-        double asum = 0.0;
-        for (int k = 0; k < nf; k++) asum += s.am[k * T.nd + c];
+        int nb[TF];
+        double a[TF], un[TF], vn[TF], asum = 0.0;
+        tel_fetch(nf, nb, [&](int k) { return tnb(T, c, k); });
+        tel_fetch(nf, a, [&](int k) { return s.am[k * T.nd + c]; });
+        tel_fetch(nf, un, [&](int k) { return s.u[nb[k]]; });
+        tel_fetch(nf, vn, [&](int k) { return s.v[nb[k]]; });
+        tel_faces(nf, [&](int k) { asum += a[k]; });
         const double rinv = 1.0 / F4(0.8), relaxm = 1.0 - F4(0.8);
         const int w = s.iwet[c];
 #pragma unroll
@@ -710,7 +826,7 @@ __global__ void __launch_bounds__(KBLOCK) k_tl_uv_prologue(TelG T, TelS s, KrySy
             const double ssv = ss[c] + relaxm * ph * ap;
             ss[c] = ssv;
             double anb = 0.0;
-            for (int k = 0; k < nf; k++) anb += s.am[k * T.nd + c] * phi[tnb(T, c, k)];
+            tel_faces(nf, [&](int k) { anb += a[k] * (q ? vn : un)[k]; });
             const double res = w * (anb + ssv - ap * ph) / ap;
             const double r = anb + ssv - ap * ph + SMALL;
             (q ? s.resv : s.resu)[c] = res;
@@ -733,8 +849,10 @@ __global__ void k_tl_pp_prep(TelG T, TelS s) {
     int i;
     if (!tel_thread(T.n, i)) return;
     const uint64_t m = T.meta[i];
-    double asum = 0.0;
-    for (int k = 0; k < m_ncf(m); k++) asum += s.am[k * T.nd + i];
+    const int nf = m_ncf(m);
+    double a[TF], asum = 0.0;
+    tel_fetch(nf, a, [&](int k) { return s.am[k * T.nd + i]; });
+    tel_faces(nf, [&](int k) { asum += a[k]; });
     const int w = s.iwet[i];
     const double apu = w * RELAX_UV / fmax(asum - s.sp[i], F4(1.0e-6));
     const double apa = apu * (T.dx[i] * T.dy[i]);
@@ -756,7 +874,7 @@ __global__ void k_tl_pp_coef_flux(TelG T, TelS s, const double *dHuy, const doub
     for (int k = 0; k < m_ncf(m); k++) {
         if (!m_own(m, k)) continue;
         const int f = k * T.nd + i, nb = tnb(T, i, k), d = m_dir(m, k);
-        const FGeo g = fgeo(T, i, nb, d);
+        const FGeo g = fgeo(T, i, nb, m, k);
         const int b = nb < T.n ? m_llec(m, k) * T.nd + nb : -1;
         const double hk = s.hk[f];
         double a, fl;
@@ -816,7 +934,7 @@ __device__ __forceinline__ double tl_fcorr(const TelG &T, const TelS &s, const d
     if (!m_joint(m) || s.iwet[o] == 0) return 0.0;
     const int nb = tnb(T, o, k), d = m_dir(m, k);
     if (s.iwet[nb] == 0 || nb >= T.n) return 0.0;
-    const FGeo f = fgeo(T, o, nb, d), b = fgeo(T, nb, o, (d + 2) & 3);
+    const FGeo f = fgeo(T, o, nb, m, k), b = fgeo(T, nb, o, (d + 2) & 3);
     const bool xd = d == KE || d == KW;
     const double rpi = rp_of(f, d), rpn = rp_of(b, d);
     const double *dpp = xd ? dppy : dppx;
@@ -836,8 +954,9 @@ __global__ void __launch_bounds__(KBLOCK) k_tl_pp_src(TelG T, TelS s, Par P, Kry
         const uint64_t m = T.meta[c];
         const int nf = m_ncf(m);
         double sp = s.sppp0[c];
-        double fs = 0.0;
-        for (int k = 0; k < nf; k++) fs += s.flux[k * T.nd + c];
+        double fl[TF], fs = 0.0;
+        tel_fetch(nf, fl, [&](int k) { return s.flux[k * T.nd + c]; });
+        tel_faces(nf, [&](int k) { fs += fl[k]; });
         double su = s.sspp0[c] - fs + s.p[c] * sp;
         if (T.skewcor && m_joint(m)) {
             double fc = 0.0;
@@ -850,9 +969,11 @@ __global__ void __launch_bounds__(KBLOCK) k_tl_pp_src(TelG T, TelS s, Par P, Kry
             }
             su = su + F4(0.2) * fc;
         }
-        double a[TF];
-#pragma unroll
-        for (int k = 0; k < TF; k++) a[k] = k < nf ? s.apc[k * T.nd + c] : 0.0;
+        int nbs[TF];
+        double a[TF], ppn[TF];
+        tel_fetch(nf, nbs, [&](int k) { return tnb(T, c, k); });
+        tel_fetch(nf, a, [&](int k) { return s.apc[k * T.nd + c]; });
+        tel_fetch(nf, ppn, [&](int k) { return s.pp[nbs[k]]; });
         const int wet = s.iwet[c];
         if (wet == 0) {
             int sumwet = 0;
@@ -873,7 +994,7 @@ __global__ void __launch_bounds__(KBLOCK) k_tl_pp_src(TelG T, TelS s, Par P, Kry
                 } else if (nb >= T.n) {
                     a[k] = 0.0;
                 } else {
-                    a[k] = fgeo(T, c, nb, m_dir(m, k)).dsxy;
+                    a[k] = fgeo(T, c, nb, m, k).dsxy;
                     aploc += a[k];
                     su += a[k] * s.p[nb];
                 }
@@ -882,19 +1003,22 @@ __global__ void __launch_bounds__(KBLOCK) k_tl_pp_src(TelG T, TelS s, Par P, Kry
             sp = 0.0;
         }
         bool changed = wet == 0;
+        if (m_strs(m)) {
 #pragma unroll
-        for (int k = 0; k < TF; k++)      // flux string: closed faces (boundaries.F90:3544-3551)
-            if (k < nf && m_qstr(m, k)) { a[k] = 0.0; changed = true; }
+            for (int k = 0; k < TF; k++)      // flux string: closed faces (boundaries.F90:3544-3551)
+                if (k < nf && m_qstr(m, k)) { a[k] = 0.0; changed = true; }
 #pragma unroll
-        for (int k = 0; k < TF; k++) {
-            if (k >= nf || !m_str(m, k)) continue;
-            const int gc = tnb(T, c, k);
-            const double ppg = s.wseadj[gc - T.n] * GRAV - s.p[gc];
-            s.pp[gc] = ppg;
-            su += a[k] * ppg;
-            sp -= a[k];
-            a[k] = 0.0;
-            changed = true;
+            for (int k = 0; k < TF; k++) {
+                if (k >= nf || !m_str(m, k)) continue;
+                const int gc = nbs[k];
+                const double ppg = s.wseadj[gc - T.n] * GRAV - s.p[gc];
+                s.pp[gc] = ppg;
+                ppn[k] = ppg;
+                su += a[k] * ppg;
+                sp -= a[k];
+                a[k] = 0.0;
+                changed = true;
+            }
         }
         // the coefficients change only on dry cells and cellstring faces
         if (changed) {
@@ -914,7 +1038,7 @@ __global__ void __launch_bounds__(KBLOCK) k_tl_pp_src(TelG T, TelS s, Par P, Kry
         double anb = 0.0;
 #pragma unroll
         for (int k = 0; k < TF; k++)
-            if (k < nf) anb += a[k] * s.pp[tnb(T, c, k)];
+            if (k < nf) anb += a[k] * ppn[k];
         const double res = wet * (anb + ss - ap * phi) / ap;
         s.resp[c] = res;
         const double r = anb + ss - ap * phi + SMALL;
@@ -957,13 +1081,7 @@ __global__ void __launch_bounds__(1024) k_tl_wse_adjust(TelG T, TelS s, Par P, d
         term[im] = tv;
     }
     __syncthreads();
-    if (threadIdx.x == 0 && adj) {
-        term[im0] = 0.0;
-        double acc = 0.0;
-        for (int im = im0 + 1; im < n; im++) { acc = acc + term[im]; term[im] = acc; }
-        acc = 0.0;
-        for (int im = im0 - 1; im >= 0; im--) { acc = acc + term[im]; term[im] = acc; }
-    }
+    if (adj) wse_prefix(term, n, im0);
     __syncthreads();
     const double base = (1.0 - ramp) * 0.0 + ramp * (w + 0.0);
     for (int im = threadIdx.x; im < n; im += blockDim.x) {
@@ -998,7 +1116,7 @@ __global__ void k_tl_pvfc1(TelG T, TelS s, const double *dppx, const double *dpp
         double fl = s.flux[f] - s.apc[f] * (s.pp[nb] - ppi);
         if (joint && nb < T.n) {
             const int d = m_dir(m, k);
-            const FGeo g = fgeo(T, i, nb, d), gb = fgeo(T, nb, i, (d + 2) & 3);
+            const FGeo g = fgeo(T, i, nb, m, k), gb = fgeo(T, nb, i, (d + 2) & 3);
             const bool xd = d == KE || d == KW;
             const double rpi = rp_of(g, d), rpn = rp_of(gb, d);
             const double *dpp = xd ? dppy : dppx;
@@ -1071,7 +1189,7 @@ __global__ void k_tl_pk(TelG T, TelS s) {
     for (int k = 0; k < m_ncf(m); k++) {
         if (!m_own(m, k)) continue;
         const int nb = tnb(T, i, k);
-        const FGeo g = fgeo(T, i, nb, m_dir(m, k));
+        const FGeo g = fgeo(T, i, nb, m, k);
         const double v = tl_interp<1>(T, s.iwet, s.p, i, k, nb, g, skew, s.dpx, s.dpy);
         s.pk[k * T.nd + i] = v;
         s.pk[m_llec(m, k) * T.nd + nb] = v;
@@ -1086,7 +1204,7 @@ __global__ void k_tl_zbk(TelG T, TelS s, const double *gx, const double *gy) {
     for (int k = 0; k < m_ncf(m); k++) {
         if (!m_own(m, k)) continue;
         const int nb = tnb(T, i, k);
-        const FGeo g = fgeo(T, i, nb, m_dir(m, k));
+        const FGeo g = fgeo(T, i, nb, m, k);
         const double v = tl_interp<0>(T, s.iwet, s.zb, i, k, nb, g, skew, gx, gy);
         s.zbk[k * T.nd + i] = v;
         s.zbk[m_llec(m, k) * T.nd + nb] = v;
@@ -1098,14 +1216,16 @@ __global__ void k_tl_dphk(TelG T, TelS s, Par P) {
     if (!tel_thread(T.n, i)) return;
     const uint64_t m = T.meta[i];
     double sx = 0.0, sy = 0.0;
-    for (int k = 0; k < m_ncf(m); k++) {
-        const int f = k * T.nd + i, nb = tnb(T, i, k);
-        const FGeo g = fgeo(T, i, nb, m_dir(m, k));
-        const double pk = s.pk[f];
-        sx += g.dsx * pk;
-        sy += g.dsy * pk;
-        s.hk[f] = fmax(P.hmin, pk * GRAVINV - s.zbk[f]);
-    }
+    const int nf = m_ncf(m);
+    double pk[TF], zk[TF];
+    tel_fetch(nf, pk, [&](int k) { return s.pk[k * T.nd + i]; });
+    tel_fetch(nf, zk, [&](int k) { return s.zbk[k * T.nd + i]; });
+    tel_faces(nf, [&](int k) {
+        const FGeo g = fgeo(T, i, tnb(T, i, k), m, k);
+        sx += g.dsx * pk[k];
+        sy += g.dsy * pk[k];
+        s.hk[k * T.nd + i] = fmax(P.hmin, pk[k] * GRAVINV - zk[k]);
+    });
     const double area = T.dx[i] * T.dy[i];
     s.dpx[i] = sx / area;
     s.dpy[i] = sy / area;
@@ -1200,10 +1320,14 @@ __global__ void k_tl_vis_fix(TelG T, TelS s) {
         const uint64_t m = T.meta[t];
         const int nf = m_ncf(m);
         if (w[t] == 1) {
-            for (int k = 0; k < nf; k++) {
-                const int nb = tnb(T, t, k);
-                if (w[nb] == 0 || nb >= T.n) val = tl_vis_from(T, vb, t, k);
-            }
+            int nbs[TF], wn[TF];
+            tel_fetch(nf, nbs, [&](int k) { return tnb(T, t, k); });
+            tel_fetch(nf, wn, [&](int k) { return (int)w[nbs[k]]; });
+            int edge = -1;                   // the last such face decides
+#pragma unroll
+            for (int k = 0; k < TF; k++)
+                if (k < nf && (wn[k] == 0 || nbs[k] >= T.n)) edge = k;
+            if (edge >= 0) val = tl_vis_from(T, vb, t, edge);
         } else {
             int best = -1, bk = 0;
             for (int k = 0; k < nf; k++) {
@@ -1244,7 +1368,7 @@ __global__ void k_tl_visk(TelG T, TelS s) {
     for (int k = 0; k < m_ncf(m); k++) {
         if (!m_own(m, k)) continue;
         const int nb = tnb(T, i, k);
-        const FGeo g = fgeo(T, i, nb, m_dir(m, k));
+        const FGeo g = fgeo(T, i, nb, m, k);
         const double v = s.iwet[i] * s.iwet[nb] == 1 ? g.fintp * tl_vis_final(T, s, nb) + (1.0 - g.fintp) * vc : 0.0;
         s.visk[k * T.nd + i] = v;
         s.visk[m_llec(m, k) * T.nd + nb] = v;
@@ -1268,7 +1392,7 @@ __global__ void k_tl_velface(TelG T, TelS s, Par P) {
         const uint64_t m = T.meta[c];
         for (int k = 0; k < m_ncf(m); k++) {
             const int f = k * T.nd + c, nb = tnb(T, c, k);
-            const FGeo g = fgeo(T, c, nb, m_dir(m, k));
+            const FGeo g = fgeo(T, c, nb, m, k);
             const double vel = s.flux[f] / (s.hk[f] * g.ds);
             const double uf = g.fnx * vel, vf = g.fny * vel;
             umin = fmin(umin, uf); umax = fmax(umax, uf);
@@ -1315,7 +1439,7 @@ __global__ void k_tl_convflux(TelG T, TelS s) {
     for (int k = 0; k < m_ncf(m); k++) {
         if (!m_own(m, k)) continue;
         const int f = k * T.nd + i, nb = tnb(T, i, k);
-        const FGeo g = fgeo(T, i, nb, m_dir(m, k));
+        const FGeo g = fgeo(T, i, nb, m, k);
         const double uni = g.fnx * s.u[i] + g.fny * s.v[i];
         const double unk = g.fnx * s.u[nb] + g.fny * s.v[nb];
         double fl = (double)(s.iwet[i] * s.iwet[nb]) * g.ds * s.hk[f] * (g.fintp * unk + (1.0 - g.fintp) * uni);
