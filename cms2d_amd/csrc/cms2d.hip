@@ -975,14 +975,15 @@ static int flow_imp_once(cms2d_flow *F) {
     LAUNCH(k_srcsnk, F->nblk_act, g, s, F->P);
     StencilOp A{g, s.aN, s.aE, s.aS, s.aW};
     for (int n = 0; n < 3; n++) F->kry[n] = 0;
+    const int keep = (F->tape ? MOM_TAPE : 0) | (F->precision == CMS2D_PREC_FP32_REFINE ? MOM_DIAG : 0) |
+                     (F->stat_on ? MOM_RES : 0);
     for (F->niter = 1; F->niter <= F->maxit; F->niter++) {
         if (F->tape)
             if (int rc = tape_snap(F, F->niter - 1)) return rc;
         river_vel(F);
         if (F->P.ndsch >= 5 && F->P.ndsch <= 9) LAUNCH(k_defcor, F->nblk_act, g, s, F->P);
-        LAUNCH(k_mom, F->nblk_act, g, s, F->P);
+        hipLaunchKernelGGL(F->P.ndsch == 4 ? k_mom<4> : k_mom<-1>, dim3(F->nblk_kry), dim3(KBLOCK), 0, F->st, g, s, F->P, F->Kuv, keep);
         TAPE(TAPE_MOM);
-        hipLaunchKernelGGL(k_uv_prologue, dim3(F->nblk_kry), dim3(KBLOCK), 0, F->st, g, s, F->Kuv);
         {
             KryCtx X = flow_ctx(F, false);
             if (F->precision == CMS2D_PREC_FP32_REFINE) {
@@ -1003,7 +1004,7 @@ static int flow_imp_once(cms2d_flow *F) {
                                curve ? wsecurve : w, ramp, curve ? F->wse_gx : 0.0, curve ? F->wse_gy : 0.0,
                                (int)((curve && F->wse_adjust_off) || !wse_forced(F->P)));
         }
-        hipLaunchKernelGGL(k_pp_src, dim3(F->nblk_kry), dim3(KBLOCK), 0, F->st, g, s, F->P, F->Kpp);
+        hipLaunchKernelGGL(k_pp_src, dim3(F->nblk_kry), dim3(KBLOCK), 0, F->st, g, s, F->P, F->Kpp, keep);
         TAPE(TAPE_PPSRC);
         {
             KryCtx X = flow_ctx(F, true);
@@ -1732,7 +1733,7 @@ extern "C" int cms2d_flow_step(cms2d_flow *F, int nsteps, cms2d_step_info *info)
         info->dt = F->deltime;
         int *count = F->s.flags + 3;
         LAUNCH(k_set_int, 1, count, 1, 0);
-        LAUNCH(k_count_wet, F->nblk_act, F->g, (const uint8_t *)F->s.iwet, count);
+        LAUNCH(k_count_wet, std::min(F->nblk_act, WET_BLOCKS), F->g, (const uint8_t *)F->s.iwet, count);
         if (int rc = sync_flags(F)) return rc;
         info->nwet = F->h_flags[3];
     }

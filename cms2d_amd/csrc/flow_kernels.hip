@@ -493,7 +493,7 @@ __device__ __forceinline__ void nvd_face(const Geo &g, const St &s, int ndsch, i
     }
 }
 // Sums over each cell's faces (N, E, S, W, the reference's face order) into
-// tu, tv; k_mom subtracts them from su, sv.
+// tu, tv; k_mom subtracts them from the sources.
 __global__ void k_defcor(Geo g, St s, Par P) {
     int i, j, c;
     if (!act_thread(g, i, j, c)) return;
@@ -506,90 +506,135 @@ __global__ void k_defcor(Geo g, St s, Par P) {
     s.tv[c] = ((nv + ev) + sv_) + wv;
 }
 
-__global__ void k_mom(Geo g, St s, Par P) {
-    int i, j, c;
-    if (!act_thread(g, i, j, c)) return;
-    const double A = g.area, fc = s.fc[c];
-    double u = s.u[c], v = s.v[c], h = s.h[c];
-    double su = s.ssu0[c] + (fc * v - s.dpx[c]) * h * A;
-    double sv = s.ssv0[c] + (-fc * u - s.dpy[c]) * h * A;
-    if (P.ndsch >= 5 && P.ndsch <= 9) {   // deferred corrections of k_defcor
-        su = su - s.tu[c];
-        sv = sv - s.tv[c];
-    }
-    double cbc = 1.0 * s.cfrict[c] * s.uelwc[c] * A;          // cmb=1 (no bed-slope factor)
-    double sp = s.spuv0[c] - cbc;
-    double a[4], hk[4], fl[4], vk[4];
-#pragma unroll
-    for (int k = 0; k < 4; k++) {
-        hk[k] = fsym(s.hkE, s.hkN, g, c, k);
-        vk[k] = fsym(s.viskE, s.viskN, g, c, k);
-        fl[k] = fdir(s.fluxE, s.fluxN, g, c, k);
-        double ddk = vk[k] * hk[k] * g.dsxy[k];
-        a[k] = schmcoef(P.ndsch, ddk, fl[k]);
-    }
-    const int wet = s.iwet[c];
-    // flux sides first (bound_uv's order): bnd_vel_flux (bnd_vel.f90:2-32), the
-    // upwind coefficient times the ghost velocity moves into the sources
-#pragma unroll
-    for (int k = 0; k < 4; k++) {
-        if (!(nb_ghost(g, i, j, k) && g.side[k] == 2)) continue;
-        const int gc = nbr(g, c, k);
-        const double ab = schmcoef(1, vk[k] * hk[k] * g.dsxy[k], fl[k]);
-        su += ab * s.u[gc];
-        sv += ab * s.v[gc];
-        sp -= ab;
-        a[k] = 0.0;
-    }
-    // harmonic water-level sides: fold the boundary face into su/sv/sp
-#pragma unroll
-    for (int k = 0; k < 4; k++) {
-        if (!(nb_ghost(g, i, j, k) && g.side[k] == 1)) continue;
-        int gc = nbr(g, c, k);
-        double ddk = vk[k] * hk[k] * g.dsxy[k];
-        double ab = schmcoef(1, ddk, fl[k]);
-        if (fabs(g.fny[k]) > F4(0.9999)) {
-            s.u[gc] = wet * u * h / s.h[gc];
-            double vg = g.fny[k] * fl[k] / (g.ds[k] * hk[k]);
-            s.v[gc] = vg;
-            sv += ab * vg;
-        } else {
-            double ug = g.fnx[k] * fl[k] / (g.ds[k] * hk[k]);
-            s.u[gc] = ug;
-            s.v[gc] = wet * v * h / s.h[gc];
-            su += ab * ug;
+// With solve()'s prologue for u (n=2) and v (n=3), relax(2) = relax(3) = 0.8
+// (solvers.f90:232-240), and the BiCGStab start (pbicgstab.f90:21-31) of the
+// same cell.  Bound by memory: a cell reads some 140 B and leaves 90 to the
+// solves; the sources stay in registers, and what only some callers read is
+// written for them alone (keep).  As two kernels, with the sources and their
+// sums through memory, 152 + 125 us at 2000 x 1500; now 172.
+// A dry cell's velocity becomes 0 here: its neighbours take it as 0 by its
+// flag, whichever comes first.
+enum { MOM_TAPE = 1, MOM_DIAG = 2, MOM_RES = 4 };   // spu, spv; ap; the residual fields
+template <int SCH>
+__global__ void __launch_bounds__(KBLOCK) k_mom(Geo g, St s, Par P, KrySys<2> K, int keep) {
+    double red[4] = {0.0, 0.0, 0.0, 0.0};
+    grid_walk(g, [&](const Idx &x_) {
+        const int i = x_.i, j = x_.j, c = x_.c;
+        const double A = g.area, fc = s.fc[c];
+        double u = s.u[c], v = s.v[c], h = s.h[c];
+        double su = s.ssu0[c] + (fc * v - s.dpx[c]) * h * A;
+        double sv = s.ssv0[c] + (-fc * u - s.dpy[c]) * h * A;
+        if (P.ndsch >= 5 && P.ndsch <= 9) {   // deferred corrections of k_defcor
+            su = su - s.tu[c];
+            sv = sv - s.tv[c];
         }
-        sp -= ab;
-        a[k] = 0.0;
-    }
-    double spu, spv;
-    if (P.wallfric) {
-        if (wet == 1) {
-            spu = sp;
-            spv = sp;
-            double z0w = s.z0[c] * 1.0;
+        double cbc = 1.0 * s.cfrict[c] * s.uelwc[c] * A;          // cmb=1 (no bed-slope factor)
+        double sp = s.spuv0[c] - cbc;
+        int wn[4];
 #pragma unroll
-            for (int k = 0; k < 4; k++) {
-                if (s.iwet[nbr(g, c, k)] != 0) continue;
-                if (fabs(g.fny[k]) > F4(0.999))
-                    spu = spu - g.ds[k] * hk[k] * wall_coef(fabs(g.ry[k]), z0w) * fabs(u);
-                else
-                    spv = spv - g.ds[k] * hk[k] * wall_coef(fabs(g.rx[k]), z0w) * fabs(v);
+        for (int k = 0; k < 4; k++) wn[k] = s.iwet[nbr(g, c, k)];
+        double a[4], hk[4], fl[4], vk[4];
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            hk[k] = fsym(s.hkE, s.hkN, g, c, k);
+            vk[k] = fsym(s.viskE, s.viskN, g, c, k);
+            fl[k] = fdir(s.fluxE, s.fluxN, g, c, k);
+            double ddk = vk[k] * hk[k] * g.dsxy[k];
+            a[k] = schmcoef(SCH < 0 ? P.ndsch : SCH, ddk, fl[k]);
+        }
+        const int wet = s.iwet[c];
+        // flux sides first (bound_uv's order): bnd_vel_flux (bnd_vel.f90:2-32), the
+        // upwind coefficient times the ghost velocity moves into the sources
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            if (!(nb_ghost(g, i, j, k) && g.side[k] == 2)) continue;
+            const int gc = nbr(g, c, k);
+            const double ab = schmcoef(1, vk[k] * hk[k] * g.dsxy[k], fl[k]);
+            su += ab * s.u[gc];
+            sv += ab * s.v[gc];
+            sp -= ab;
+            a[k] = 0.0;
+        }
+        // harmonic water-level sides: fold the boundary face into su/sv/sp
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            if (!(nb_ghost(g, i, j, k) && g.side[k] == 1)) continue;
+            int gc = nbr(g, c, k);
+            double ddk = vk[k] * hk[k] * g.dsxy[k];
+            double ab = schmcoef(1, ddk, fl[k]);
+            if (fabs(g.fny[k]) > F4(0.9999)) {
+                s.u[gc] = wet * u * h / s.h[gc];
+                double vg = g.fny[k] * fl[k] / (g.ds[k] * hk[k]);
+                s.v[gc] = vg;
+                sv += ab * vg;
+            } else {
+                double ug = g.fnx[k] * fl[k] / (g.ds[k] * hk[k]);
+                s.u[gc] = ug;
+                s.v[gc] = wet * v * h / s.h[gc];
+                su += ab * ug;
+            }
+            sp -= ab;
+            a[k] = 0.0;
+        }
+        double spu, spv;
+        if (P.wallfric) {
+            if (wet == 1) {
+                spu = sp;
+                spv = sp;
+                if ((wn[0] & wn[1] & wn[2] & wn[3]) == 0) {     // beside a dry cell or a wall
+                    const double z0w = s.z0[c] * 1.0;
+                    // the same on both faces across an axis
+                    const double cy = wall_coef(fabs(g.ry[KN]), z0w), cx = wall_coef(fabs(g.rx[KE]), z0w);
+#pragma unroll
+                    for (int k = 0; k < 4; k++) {
+                        if (wn[k] != 0) continue;
+                        if (fabs(g.fny[k]) > F4(0.999)) spu = spu - g.ds[k] * hk[k] * cy * fabs(u);
+                        else spv = spv - g.ds[k] * hk[k] * cx * fabs(v);
+                    }
+                }
+            } else {
+                s.u[c] = u = 0.0; s.v[c] = v = 0.0;
+                spu = -1.0; spv = -1.0; sp = -1.0;
+                su = 0.0; sv = 0.0;
             }
         } else {
-            s.u[c] = 0.0; s.v[c] = 0.0;
-            spu = -1.0; spv = -1.0; sp = -1.0;
-            su = 0.0; sv = 0.0;
+            s.u[c] = u = wet * u;
+            s.v[c] = v = wet * v;
+            sp = wet * sp + (double)(wet - 1);
+            spu = sp; spv = sp;
+            su = wet * su; sv = wet * sv;
         }
-    } else {
-        s.u[c] = wet * u;
-        s.v[c] = wet * v;
-        sp = wet * sp + (double)(wet - 1);
-        spu = sp; spv = sp;
-        su = wet * su; sv = wet * sv;
-    }
-    s.su[c] = su; s.sv[c] = sv; s.sp[c] = sp; s.spu[c] = spu; s.spv[c] = spv;
-    s.aN[c] = a[KN]; s.aE[c] = a[KE]; s.aS[c] = a[KS]; s.aW[c] = a[KW];
+        s.sp[c] = sp;
+        s.aN[c] = a[KN]; s.aE[c] = a[KE]; s.aS[c] = a[KS]; s.aW[c] = a[KW];
+        if (keep & MOM_TAPE) { s.spu[c] = spu; s.spv[c] = spv; }
+        const double asum = ((a[0] + a[1]) + a[2]) + a[3];
+        const double rinv = 1.0 / F4(0.8), relaxm = 1.0 - F4(0.8);
+#pragma unroll
+        for (int q = 0; q < 2; q++) {
+            const double *phi = q ? s.v : s.u;
+            const double ap = (asum - (q ? spv : spu)) * rinv;
+            const double ph = q ? v : u;
+            const double ss = (q ? sv : su) + relaxm * ph * ap;
+            double anb = 0.0;
+#pragma unroll
+            for (int k = 0; k < 4; k++) {
+                const double pn = phi[nbr(g, c, k)];
+                anb += a[k] * (wn[k] ? pn : 0.0);
+            }
+            const double res = wet * (anb + ss - ap * ph) / ap;
+            const double r = anb + ss - ap * ph + SMALL;
+            if (keep & MOM_RES) (q ? s.resv : s.resu)[c] = res;
+            if (keep & MOM_DIAG) K.ap_w[q][c] = ap;
+            K.dinv_w[q][c] = 1.0 / ap;
+            K.r[q][c] = r; K.r0[q][c] = r;
+            red[2 * q] += r * r;
+            red[2 * q + 1] += res * res;
+        }
+    });
+    double *const dst[4] = {K.red.pr[0], K.red.pr[0] + gridDim.x, K.red.pr[1], K.red.pr[1] + gridDim.x};
+    put_partials<4>(red, dst);
+    kry_reset(K.sc[0]);
+    kry_reset(K.sc[1]);
 }
 
 // ------------------------------------------------------- pressure correction
@@ -730,7 +775,7 @@ __global__ void __launch_bounds__(1024) k_wse_adjust(Geo g, St s, Par P, int sid
 // pp sources (flow_imp.F90:700-712) + bound_pp (boundaries.F90:3493-3646) +
 // solve prologue for n=1 (solvers.f90:232-240, relax(1)=1) + BiCGStab start.
 // Runs on the fixed Krylov grid and leaves r.r / res.res partials.
-__global__ void __launch_bounds__(KBLOCK) k_pp_src(Geo g, St s, Par P, KrySys<1> K) {
+__global__ void __launch_bounds__(KBLOCK) k_pp_src(Geo g, St s, Par P, KrySys<1> K, int keep) {
     double red[2] = {0.0, 0.0};
     grid_walk(g, [&](const Idx &x_) {
         const int i = x_.i, j = x_.j, c = x_.c;
@@ -786,12 +831,11 @@ __global__ void __launch_bounds__(KBLOCK) k_pp_src(Geo g, St s, Par P, KrySys<1>
         double ap = (asum - sp) * 1.0;
         double phi = s.pp[c];
         double ss = su + 0.0 * phi * ap;
-        s.su[c] = ss;
         double anb = 0.0;
 #pragma unroll
         for (int k = 0; k < 4; k++) anb += a[k] * s.pp[nbr(g, c, k)];
         double res = wet * (anb + ss - ap * phi) / ap;
-        s.resp[c] = res;
+        if (keep & MOM_RES) s.resp[c] = res;
         double r = anb + ss - ap * phi + SMALL;
         K.ap_w[0][c] = ap;
         K.dinv_w[0][c] = 1.0 / ap;
@@ -1437,17 +1481,31 @@ __global__ void k_pack(Geo g, const T *src, double *dst) {
     if (!act_thread(g, i, j, c)) return;
     dst[j * g.nx + i] = (double)src[c];
 }
-// Wet active cells, added to *count (a wave at a time).
+// Wet active cells, added to *count: one addition a block of a fixed grid (one
+// a wave met at the same word 56 thousand times at 3.6 M cells, 570 us).
+constexpr int WET_BLOCKS = 512;
+template <class F>
+__device__ __forceinline__ void count_wet(int n, int *count, F &&wet) {
+    __shared__ int part[BLOCK / 64];
+    int w = 0;
+    for (int i0 = blockIdx.x * BLOCK; i0 < n; i0 += gridDim.x * BLOCK) {
+        const int i = i0 + threadIdx.x;
+        w += __popcll(__ballot(i < n && wet(i)));
+    }
+    if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = w;
+    __syncthreads();
+    if (threadIdx.x != 0) return;
+    for (int k = 1; k < BLOCK / 64; k++) w += part[k];
+    if (w) atomicAdd(count, w);
+}
 __global__ void __launch_bounds__(BLOCK) k_count_wet(Geo g, const uint8_t *iwet, int *count) {
-    int i, j, c;
-    const bool wet = act_thread(g, i, j, c) && iwet[c];
-    const int n = __popcll(__ballot(wet));
-    if ((threadIdx.x & 63) == 0 && n) atomicAdd(count, n);
+    count_wet(g.nact, count, [&](int t) {
+        const int j = t / g.nx;
+        return iwet[cidx(g, t - j * g.nx, j)] != 0;
+    });
 }
 __global__ void __launch_bounds__(BLOCK) k_count_wet_list(int n, const uint8_t *iwet, int *count) {
-    const int i = blockIdx.x * BLOCK + threadIdx.x;
-    const int w = __popcll(__ballot(i < n && iwet[i]));
-    if ((threadIdx.x & 63) == 0 && w) atomicAdd(count, w);
+    count_wet(n, count, [&](int i) { return iwet[i] != 0; });
 }
 
 __global__ void k_set_int(int *p, int n, int v) {

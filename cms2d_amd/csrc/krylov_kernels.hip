@@ -18,45 +18,6 @@ namespace cms {
 #define SMALL F4(1.0e-15)
 #endif
 
-// solve() prologue for u (n=2) and v (n=3), relax(2)=relax(3)=0.8
-// (solvers.f90:232-240), then the BiCGStab start (pbicgstab.f90:21-31).
-__global__ void __launch_bounds__(KBLOCK) k_uv_prologue(Geo g, St s, KrySys<2> K) {
-    double red[4] = {0.0, 0.0, 0.0, 0.0};
-    grid_walk(g, [&](const Idx &x_) {
-        const int i = x_.i, j = x_.j, c = x_.c;
-        const double a[4] = {s.aN[c], s.aE[c], s.aS[c], s.aW[c]};
-        const int nb[4] = {c + g.nxp, c + 1, c - g.nxp, c - 1};
-        const double asum = ((a[0] + a[1]) + a[2]) + a[3];
-        const double rinv = 1.0 / F4(0.8), relaxm = 1.0 - F4(0.8);
-        const int w = s.iwet[c];
-#pragma unroll
-        for (int q = 0; q < 2; q++) {
-            double *phi = q ? s.v : s.u;
-            double *ss = q ? s.sv : s.su;
-            const double *sp = q ? s.spv : s.spu;
-            double ap = (asum - sp[c]) * rinv;
-            double ph = phi[c];
-            double ssv = ss[c] + relaxm * ph * ap;
-            ss[c] = ssv;
-            double anb = 0.0;
-#pragma unroll
-            for (int k = 0; k < 4; k++) anb += a[k] * phi[nb[k]];
-            double res = w * (anb + ssv - ap * ph) / ap;
-            double r = anb + ssv - ap * ph + SMALL;
-            (q ? s.resv : s.resu)[c] = res;
-            K.ap_w[q][c] = ap;
-            K.dinv_w[q][c] = 1.0 / ap;
-            K.r[q][c] = r; K.r0[q][c] = r;
-            red[2 * q] += r * r;
-            red[2 * q + 1] += res * res;
-        }
-    });
-    double *const dst[4] = {K.red.pr[0], K.red.pr[0] + gridDim.x, K.red.pr[1], K.red.pr[1] + gridDim.x};
-    put_partials<4>(red, dst);
-    kry_reset(K.sc[0]);
-    kry_reset(K.sc[1]);
-}
-
 // The five sweeps.  On a small grid a block makes one pass and a launch lasts
 // as long as its longest chain of loads, so each kernel issues the loads of its
 // first cell, of the stopping flags and of the scalars before it sums the

@@ -1508,7 +1508,7 @@ static int tel_step(cms2d_flow *F, int nsteps, cms2d_step_info *info) {
         info->dt = F->deltime;
         int *count = H.s.flags + 3;
         TLAUNCH(k_set_int, 1, count, 1, 0);
-        TLAUNCH(k_count_wet_list, H.nblk_n, H.T.n, (const uint8_t *)H.s.iwet, count);
+        TLAUNCH(k_count_wet_list, std::min(H.nblk_n, WET_BLOCKS), H.T.n, (const uint8_t *)H.s.iwet, count);
         if (int rc = tel_sync_flags(F)) return rc;
         info->nwet = F->h_flags[3];
     }
