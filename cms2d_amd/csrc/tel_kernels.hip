@@ -147,8 +147,8 @@ __device__ __forceinline__ void tel_faces(int nf, F &&f) {
 struct TelS {
     double *u, *v, *p, *h, *pp, *zb, *vis, *visb, *visc, *u1, *v1, *p1, *h1, *eta, *maxeta;
     double *coefman, *cfrict, *z0, *uv, *uelwc, *bsvel, *cbf, *fc, *wavestrx, *wavestry;
-    double *su, *sv, *sp, *spu, *spv, *ssu0, *ssv0, *spuv0, *sppp0, *sspp0;
-    double *apuareap, *sumu, *Hu, *Hv, *resu, *resv, *resp, *dpx, *dpy, *tu, *tv, *tvis;
+    double *su, *sv, *sp, *ssu0, *ssv0, *spuv0, *sppp0, *sspp0;
+    double *apuareap, *sumu, *Hu, *Hv, *dpx, *dpy, *tu, *tv, *tvis;
     double *flux, *flux1, *hk, *pk, *visk, *zbk, *am, *apc;   // [TF*nd]
     double *wseadj;              // [nstr]
     uint8_t *iwet, *iwet1, *icorner, *ipond;
@@ -184,8 +184,8 @@ __device__ __forceinline__ void tel_grad(const TelG &T, const uint8_t *iwet, int
         // Four even faces: between neighbours that all count, the weights are
         // +-ds/(2 area) across the cell and 0 on the cell itself, and the four
         // neighbours' values are fetched together with their flags.  (The form
-        // below loads face after face and divides seven times: 500 -> 180 us
-        // for three fields of 2.8 M cells, nearly all of them plain.)
+        // below loads face after face and divides seven times: 212 -> 141 us
+        // for three fields of 3.6 M cells, most of them plain.)
         int nb[4];
 #pragma unroll
         for (int k = 0; k < 4; k++) nb[k] = tnb(T, i, k);
@@ -619,80 +619,6 @@ __global__ void k_tl_defcor_skew(TelG T, TelS s, const double *dux, const double
     s.sv[i] = s.sv[i] - sv;
 }
 
-// bound_uv (boundaries.F90:3310-3490) with bnd_vel_openwse (bnd_vel.f90:35-95)
-// on the water-level string faces, wall friction (fric_lib.f90:162-194), dry cells.
-__global__ void k_tl_bound_uv(TelG T, TelS s, Par P) {
-    int i;
-    if (!tel_thread(T.n, i)) return;
-    const uint64_t m = T.meta[i];
-    const int nf = m_ncf(m);
-    double sp = s.sp[i];
-    const bool strs = m_strs(m);
-    // flux string first (bound_uv's order): bnd_vel_flux (bnd_vel.f90:2-32)
-    for (int k = 0; strs && k < nf; k++) {
-        if (!m_qstr(m, k)) continue;
-        const int f = k * T.nd + i, nb = tnb(T, i, k);
-        const FGeo g = fgeo(T, i, nb, m, k);
-        const double a = schmcoef(1, s.visk[f] * s.hk[f] * g.dsxy, s.flux[f]);
-        s.su[i] = s.su[i] + a * s.u[nb];
-        s.sv[i] = s.sv[i] + a * s.v[nb];
-        sp = sp - a;
-        s.am[f] = 0.0;
-    }
-    for (int k = 0; strs && k < nf; k++) {
-        if (!m_str(m, k)) continue;
-        const int f = k * T.nd + i, nb = tnb(T, i, k);
-        const FGeo g = fgeo(T, i, nb, m, k);
-        const double ddk = s.visk[f] * s.hk[f] * g.dsxy;
-        const double a = schmcoef(1, ddk, s.flux[f]);
-        if (fabs(g.fny) > F4(0.9999)) {
-            s.u[nb] = s.iwet[i] * s.u[i] * s.h[i] / s.h[nb];
-            const double vg = g.fny * s.flux[f] / (g.ds * s.hk[f]);
-            s.v[nb] = vg;
-            s.sv[i] = s.sv[i] + a * vg;
-        } else {
-            const double ug = g.fnx * s.flux[f] / (g.ds * s.hk[f]);
-            s.u[nb] = ug;
-            s.v[nb] = s.iwet[i] * s.v[i] * s.h[i] / s.h[nb];
-            s.su[i] = s.su[i] + a * ug;
-        }
-        sp = sp - a;
-        s.am[f] = 0.0;
-    }
-    const int w = s.iwet[i];
-    if (P.wallfric) {
-        if (w == 1) {
-            double spu = sp, spv = sp;
-            int nbs[TF], wn[TF];
-            tel_fetch(nf, nbs, [&](int k) { return tnb(T, i, k); });
-            tel_fetch(nf, wn, [&](int k) { return (int)s.iwet[nbs[k]]; });
-            bool dry = false;
-#pragma unroll
-            for (int k = 0; k < TF; k++) dry = dry || (k < nf && wn[k] == 0);
-            for (int k = 0; dry && k < nf; k++) {
-                const int f = k * T.nd + i, nb = tnb(T, i, k);
-                if (s.iwet[nb] != 0) continue;
-                const FGeo g = fgeo(T, i, nb, m, k);
-                const double z0w = s.z0[i] * 1.0;
-                if (fabs(g.fny) > F4(0.999)) spu -= g.ds * s.hk[f] * wall_coef(fabs(g.ry), z0w) * fabs(s.u[i]);
-                else spv -= g.ds * s.hk[f] * wall_coef(fabs(g.rx), z0w) * fabs(s.v[i]);
-            }
-            s.sp[i] = sp; s.spu[i] = spu; s.spv[i] = spv;
-        } else {
-            s.u[i] = 0.0; s.v[i] = 0.0;
-            s.spu[i] = -1.0; s.spv[i] = -1.0; s.sp[i] = -1.0;
-            s.su[i] = 0.0; s.sv[i] = 0.0;
-        }
-    } else {
-        s.u[i] = w * s.u[i];
-        s.v[i] = w * s.v[i];
-        const double spw = w * sp + (double)(w - 1);
-        s.sp[i] = spw; s.spu[i] = spw; s.spv[i] = spw;
-        s.su[i] = w * s.su[i];
-        s.sv[i] = w * s.sv[i];
-    }
-}
-
 // Cell-list operator for the Krylov kernels: y_i = ap_i z_i - sum_k a_k(i) z_nb
 // over active neighbours (z = 0 on ghost cells, pbicgstab.f90:55,76).
 template <class CA>
@@ -799,40 +725,109 @@ struct TelOpT {
 using TelOp = TelOpT<double>;
 using TelOp32 = TelOpT<float>;   // the inner solve of the FP32 form
 
-// solve prologue for u (n=2) and v (n=3), relax 0.8 (solvers.f90:232-240) and
-// the BiCGStab start (pbicgstab.f90:21-31).
-__global__ void __launch_bounds__(KBLOCK) k_tl_uv_prologue(TelG T, TelS s, KrySys<2> K, TelOp A) {
+// bound_uv (boundaries.F90:3310-3490) with bnd_vel_openwse (bnd_vel.f90:35-95)
+// on the water-level string faces, wall friction (fric_lib.f90:162-194), dry
+// cells; then the solve prologue for u (n=2) and v (n=3), relax 0.8
+// (solvers.f90:232-240), and the BiCGStab start (pbicgstab.f90:21-31) of the
+// same cell, its sources in registers.  Bound by memory (two kernels, with the
+// sources and both diagonals through memory: 59 + 154 us at 3.6 M cells).
+// A dry cell's velocity becomes 0 here: its neighbours take it as 0 by its flag,
+// whichever comes first.  diag: the FP32 form reads the diagonals.
+__global__ void __launch_bounds__(KBLOCK) k_tl_uv_start(TelG T, TelS s, Par P, KrySys<2> K, TelOp A, int diag) {
     double red[4] = {0.0, 0.0, 0.0, 0.0};
     A.each([&](const Idx &x_) {
-        const int c = x_.c;
-        const uint64_t m = T.meta[c];
+        const int i = x_.c;
+        const uint64_t m = T.meta[i];
         const int nf = m_ncf(m);
-        int nb[TF];
+        int nbs[TF], wn[TF];
+        tel_fetch(nf, nbs, [&](int k) { return tnb(T, i, k); });
+        const int w = s.iwet[i];
+        double u = s.u[i], v = s.v[i], su = s.su[i], sv = s.sv[i], sp = s.sp[i];
+        tel_fetch(nf, wn, [&](int k) { return (int)s.iwet[nbs[k]]; });
+        if (m_strs(m)) {
+            // flux string first (bound_uv's order): bnd_vel_flux (bnd_vel.f90:2-32)
+#pragma unroll 1
+            for (int k = 0; k < nf; k++) {
+                if (!m_qstr(m, k)) continue;
+                const int f = k * T.nd + i, nb = tnb(T, i, k);
+                const FGeo g = fgeo(T, i, nb, m, k);
+                const double ab = schmcoef(1, s.visk[f] * s.hk[f] * g.dsxy, s.flux[f]);
+                su = su + ab * s.u[nb];
+                sv = sv + ab * s.v[nb];
+                sp = sp - ab;
+                s.am[f] = 0.0;
+            }
+#pragma unroll 1
+            for (int k = 0; k < nf; k++) {
+                if (!m_str(m, k)) continue;
+                const int f = k * T.nd + i, nb = tnb(T, i, k);
+                const FGeo g = fgeo(T, i, nb, m, k);
+                const double ddk = s.visk[f] * s.hk[f] * g.dsxy;
+                const double ab = schmcoef(1, ddk, s.flux[f]);
+                if (fabs(g.fny) > F4(0.9999)) {
+                    s.u[nb] = w * u * s.h[i] / s.h[nb];
+                    const double vg = g.fny * s.flux[f] / (g.ds * s.hk[f]);
+                    s.v[nb] = vg;
+                    sv = sv + ab * vg;
+                } else {
+                    const double ug = g.fnx * s.flux[f] / (g.ds * s.hk[f]);
+                    s.u[nb] = ug;
+                    s.v[nb] = w * v * s.h[i] / s.h[nb];
+                    su = su + ab * ug;
+                }
+                sp = sp - ab;
+                s.am[f] = 0.0;
+            }
+        }
+        double spu = sp, spv = sp;
+        if (P.wallfric) {
+            if (w == 1) {
+                bool dry = false;
+#pragma unroll
+                for (int k = 0; k < TF; k++) dry = dry || (k < nf && wn[k] == 0);
+#pragma unroll 1
+                for (int k = 0; dry && k < nf; k++) {
+                    const int f = k * T.nd + i, nb = tnb(T, i, k);
+                    if (s.iwet[nb] != 0) continue;
+                    const FGeo g = fgeo(T, i, nb, m, k);
+                    const double z0w = s.z0[i] * 1.0;
+                    const bool ns = fabs(g.fny) > F4(0.999);
+                    const double fr = g.ds * s.hk[f] * wall_coef(fabs(ns ? g.ry : g.rx), z0w) * fabs(ns ? u : v);
+                    if (ns) spu -= fr;
+                    else spv -= fr;
+                }
+            } else {
+                s.u[i] = u = 0.0; s.v[i] = v = 0.0;
+                spu = -1.0; spv = -1.0; sp = -1.0;
+                su = 0.0; sv = 0.0;
+            }
+        } else {
+            s.u[i] = u = w * u;
+            s.v[i] = v = w * v;
+            sp = w * sp + (double)(w - 1);
+            spu = sp; spv = sp;
+            su = w * su;
+            sv = w * sv;
+        }
+        s.sp[i] = sp;
         double a[TF], un[TF], vn[TF], asum = 0.0;
-        tel_fetch(nf, nb, [&](int k) { return tnb(T, c, k); });
-        tel_fetch(nf, a, [&](int k) { return s.am[k * T.nd + c]; });
-        tel_fetch(nf, un, [&](int k) { return s.u[nb[k]]; });
-        tel_fetch(nf, vn, [&](int k) { return s.v[nb[k]]; });
+        tel_fetch(nf, a, [&](int k) { return s.am[k * T.nd + i]; });
+        tel_fetch(nf, un, [&](int k) { return s.u[nbs[k]]; });
+        tel_fetch(nf, vn, [&](int k) { return s.v[nbs[k]]; });
         tel_faces(nf, [&](int k) { asum += a[k]; });
         const double rinv = 1.0 / F4(0.8), relaxm = 1.0 - F4(0.8);
-        const int w = s.iwet[c];
 #pragma unroll
         for (int q = 0; q < 2; q++) {
-            double *phi = q ? s.v : s.u;
-            double *ss = q ? s.sv : s.su;
-            const double *sp = q ? s.spv : s.spu;
-            const double ap = (asum - sp[c]) * rinv;
-            const double ph = phi[c];
-            const double ssv = ss[c] + relaxm * ph * ap;
-            ss[c] = ssv;
+            const double ap = (asum - (q ? spv : spu)) * rinv;
+            const double ph = q ? v : u;
+            const double ss = (q ? sv : su) + relaxm * ph * ap;
             double anb = 0.0;
-            tel_faces(nf, [&](int k) { anb += a[k] * (q ? vn : un)[k]; });
-            const double res = w * (anb + ssv - ap * ph) / ap;
-            const double r = anb + ssv - ap * ph + SMALL;
-            (q ? s.resv : s.resu)[c] = res;
-            K.ap_w[q][c] = ap;
-            K.dinv_w[q][c] = 1.0 / ap;
-            K.r[q][c] = r; K.r0[q][c] = r;
+            tel_faces(nf, [&](int k) { anb += a[k] * (wn[k] ? (q ? vn : un)[k] : 0.0); });
+            const double res = w * (anb + ss - ap * ph) / ap;
+            const double r = anb + ss - ap * ph + SMALL;
+            if (diag) K.ap_w[q][i] = ap;
+            K.dinv_w[q][i] = 1.0 / ap;
+            K.r[q][i] = r; K.r0[q][i] = r;
             red[2 * q] += r * r;
             red[2 * q + 1] += res * res;
         }
@@ -1034,13 +1029,11 @@ __global__ void __launch_bounds__(KBLOCK) k_tl_pp_src(TelG T, TelS s, Par P, Kry
         const double ap = (asum - sp) * 1.0;
         const double phi = s.pp[c];
         const double ss = su + 0.0 * phi * ap;
-        s.su[c] = ss;
         double anb = 0.0;
 #pragma unroll
         for (int k = 0; k < TF; k++)
             if (k < nf) anb += a[k] * ppn[k];
         const double res = wet * (anb + ss - ap * phi) / ap;
-        s.resp[c] = res;
         const double r = anb + ss - ap * phi + SMALL;
         K.ap_w[0][c] = ap;
         K.dinv_w[0][c] = 1.0 / ap;
