@@ -38,22 +38,56 @@ static size_t state_bytes(const cms2d_flow *F) {
     for (auto &a : F->state) n += a.second;
     return n;
 }
+// Copies gathered into launches of k_copy_list on the flow's stream.
+namespace {
+struct Copies {
+    cms2d_flow *F;
+    CopyList L;
+    int n = 0;
+    size_t most = 0;
+    hipError_t err = hipSuccess;
+    explicit Copies(cms2d_flow *f) : F(f) {}
+    void add(void *dst, const void *src, size_t bytes) {
+        if (!bytes) return;
+        L.src[n] = (const char *)src;
+        L.dst[n] = (char *)dst;
+        L.bytes[n] = bytes;
+        most = std::max(most, bytes);
+        if (++n == COPY_MAX) send();
+    }
+    void send() {
+        if (!n) return;
+        const size_t nb = std::min<size_t>((most / 16 + BLOCK) / BLOCK, 256);
+        hipLaunchKernelGGL(k_copy_list, dim3((unsigned)nb, (unsigned)n), dim3(BLOCK), 0, F->st, L);
+        const hipError_t e = hipGetLastError();
+        if (err == hipSuccess) err = e;
+        n = 0;
+        most = 0;
+    }
+};
+}  // namespace
 static int snap_save(cms2d_flow *F, Snap &S) {
     if (!S.dev) HIPCHK(hipMalloc((void **)&S.dev, state_bytes(F)));
+    Copies C(F);
     size_t off = 0;
     for (auto &a : F->state) {
-        HIPCHK(hipMemcpyAsync(S.dev + off, a.first, a.second, hipMemcpyDeviceToDevice, F->st));
+        C.add(S.dev + off, a.first, a.second);
         off += a.second;
     }
+    C.send();
+    HIPCHK(C.err);
     ck_host_get(F, S.host);
     return 0;
 }
 static int snap_load(cms2d_flow *F, const Snap &S) {
+    Copies C(F);
     size_t off = 0;
     for (auto &a : F->state) {
-        HIPCHK(hipMemcpyAsync(a.first, S.dev + off, a.second, hipMemcpyDeviceToDevice, F->st));
+        C.add(a.first, S.dev + off, a.second);
         off += a.second;
     }
+    C.send();
+    HIPCHK(C.err);
     ck_host_set(F, S.host);
     return 0;
 }
@@ -102,36 +136,34 @@ static int tape_mid(cms2d_flow *F, int what) {
     const Mid M = mid_view(F, T.mid[it]);
     const St &s = F->s;
     const size_t nb = (size_t)F->npad * sizeof(double);
-    auto cp = [&](double *dst, const double *src) {
-        return hipMemcpyAsync(dst, src, nb, hipMemcpyDeviceToDevice, F->st);
-    };
-    hipError_t e = hipSuccess;
-    auto chk = [&](hipError_t x) { if (e == hipSuccess) e = x; };
+    Copies C(F);
+    auto cp = [&](double *dst, const double *src) { C.add(dst, src, nb); };
     const double *a4[4] = {s.aN, s.aE, s.aS, s.aW};
     switch (what) {
     case TAPE_MOM:
-        for (int k = 0; k < 4; k++) chk(cp(M.au[k], a4[k]));
-        chk(cp(M.sp, s.sp)); chk(cp(M.spu, s.spu)); chk(cp(M.spv, s.spv));
-        chk(cp(M.u0, s.u)); chk(cp(M.v0, s.v));
+        for (int k = 0; k < 4; k++) cp(M.au[k], a4[k]);
+        cp(M.sp, s.sp); cp(M.spu, s.spu); cp(M.spv, s.spv);
+        cp(M.u0, s.u); cp(M.v0, s.v);
         break;
     case TAPE_UV:
-        chk(cp(M.us, s.u)); chk(cp(M.vs, s.v));
+        cp(M.us, s.u); cp(M.vs, s.v);
         break;
     case TAPE_PPCOEF:
-        for (int k = 0; k < 4; k++) chk(cp(M.a0[k], a4[k]));
-        chk(cp(M.apa, s.apuareap)); chk(cp(M.sumu, s.sumu)); chk(cp(M.Hu, s.Hu)); chk(cp(M.Hv, s.Hv));
+        for (int k = 0; k < 4; k++) cp(M.a0[k], a4[k]);
+        cp(M.apa, s.apuareap); cp(M.sumu, s.sumu); cp(M.Hu, s.Hu); cp(M.Hv, s.Hv);
         break;
     case TAPE_PPSRC:
-        for (int k = 0; k < 4; k++) chk(cp(M.ap[k], a4[k]));
-        chk(cp(M.spp, s.sp));
+        for (int k = 0; k < 4; k++) cp(M.ap[k], a4[k]);
+        cp(M.spp, s.sp);
         break;
     case TAPE_PPSOL:
-        chk(cp(M.pps, s.pp));
+        cp(M.pps, s.pp);
         break;
     default:
-        chk(cp(M.ppv, s.pp));
+        cp(M.ppv, s.pp);
     }
-    if (e != hipSuccess) return set_err(CMS2D_ERR_HIP, std::string("tape copy: ") + hipGetErrorString(e));
+    C.send();
+    if (C.err != hipSuccess) return set_err(CMS2D_ERR_HIP, std::string("tape copy: ") + hipGetErrorString(C.err));
     return 0;
 }
 
