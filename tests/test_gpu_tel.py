@@ -72,6 +72,32 @@ def test_tel_step_matches_reference_vectors(gpu_available, name):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("dx", [16.0, 20.0 / 3.0], ids=["exact", "rounded"])
+@pytest.mark.parametrize("nx,ny", [(200, 5), (131, 9)], ids=lambda v: str(v))
+def test_tel_plain_cells_and_rounded_centres_match_oracle(gpu_available, dx, nx, ny):
+    """Rows long enough for chunks of 64 cells with the same neighbour offsets
+    beside ones without (a refined band, the edges, the last cells of the list),
+    on cell centres that are exact and on ones that are rounded, whose faces
+    then take the general geometry.  dt follows dx, so the systems are alike;
+    bounds as in the other comparisons with the oracle."""
+    c = cases.tidal_tel(nx=nx, ny=ny, dx=dx, dt=1.5 * dx, band=((20, 32), (24, 28)), seed=4)
+    x, y, size = c.tel.geom[:, 0], c.tel.geom[:, 1], c.tel.geom[:, 2]
+    i = np.flatnonzero((size[:-1] == size.max()) & (size[1:] == size.max()) & (y[1:] == y[:-1]))
+    assert len(i) and np.all(x[i + 1] - x[i] == size.max()) == (dx == 16.0)
+    g, o = FlowStep(c), Oracle(c, serial=0)
+    for s in range(4):
+        g.step(1)
+        rc, _ = o.step(1)
+        assert rc == 0
+        assert np.array_equal(g.get("iwet"), o.get("iwet")), s
+        w = o.get("iwet") > 0
+        for f in ("eta", "u", "v"):
+            d = np.abs(g.get(f) - o.get(f))[w if f == "eta" else slice(None)].max()
+            assert d <= 1e-9, (s, f, d)
+    g.close()
+
+
+@pytest.mark.gpu
 def test_tel_uniform_grid_equals_cartesian_flow(gpu_available):
     """A telescoping cell list whose cells are all base cells is the
     rectangle: the cell-list step agrees with the Cartesian step."""
