@@ -31,15 +31,18 @@ HBM_PEAK_GBS = 8000.0
 # V-cycle's levels below level 0) with their algorithmic bytes per launch:
 #   spmv_pp   k_bicg_spmv MODE 1 (v = A z) and MODE 2 (t = A zs): read
 #             aN,aE,aS,aW,ap,r0 (FP64) and z (FP32), write v (FP64): 60 B per
-#             cell; on the cell list the face metadata word, per face the
-#             neighbour index and coefficient, ap, r0, z, v: 36 + 12 F B
+#             cell; on the cell list 28 B of ap, r0, z, v and 8 B a face, and
+#             outside the chunks of equal neighbour offsets the face metadata
+#             word and the neighbour indices, 8 + 4 F B more
 #   mg_down0  k_mg_down on level 0: read b (FP64, FP32 on telescoping grids),
-#             aN..aW, 1/ap (FP32), write z (FP32) and a quarter-size coarse b:
-#             8 + 5*4 + 4 + 1 = 33 B per base cell (29 with FP32 b)
-#   mg_up0    k_mg_up on level 0: read b, aN..aW, 1/ap, z and a quarter-size
-#             coarse z, write z: 8 + 6*4 + 1 + 4 = 37 B per base cell (33)
+#             aN..aW, 1/ap (FP32), write the black cells' z (FP32) and a
+#             quarter-size coarse b: 8 + 5*4 + 2 + 1 = 31 B per base cell (27
+#             with FP32 b)
+#   mg_up0    k_mg_up on level 0: read b, aN..aW, 1/ap, the black z and a
+#             quarter-size coarse z, write z: 8 + 5*4 + 2 + 1 + 4 = 35 B per
+#             base cell (31)
 #   mg_coarse the levels below level 0 of one V-cycle: down and up sweeps of
-#             level l read and write 29 + 33 = 62 B per level-l cell
+#             level l read and write 27 + 31 = 58 B per level-l cell
 #   tel_restrict    residual r - A Z summed into the base cells: per cell the
 #             list entry, metadata, r, base cell and its range (28 B), on cells
 #             next to refined cells also ap, Z and per face index, coefficient
@@ -64,7 +67,7 @@ KERNEL_DESC = {
     "spmv_pp": "k_bicg_spmv MODE 1 and 2 (pp system: v = A z, t = A zs, z from the preconditioner)",
     "mg_down0": "k_mg_down (multigrid level 0: red-black pre-smoothing + restriction)",
     "mg_up0": "k_mg_up (multigrid level 0: correction + red-black post-smoothing)",
-    "mg_coarse": "multigrid levels 1.. of a V-cycle (k_mg_down_pc, k_mg_coarsest, k_mg_up_pc; span)",
+    "mg_coarse": "multigrid levels 1.. of a V-cycle (k_mg_down, k_mg_tail, k_mg_up; span)",
     "tel_restrict": "k_tl_mg_restrict (residual summed into the base cells)",
     "tel_fjac": "k_tl_cs_fjac (damped Jacobi sweep on the 5 m cells)",
     "tel_cs_restrict": "k_tl_cs_restrict (residual summed into the 10 m squares)",
@@ -73,7 +76,8 @@ KERNEL_DESC = {
 
 def mg_level_cells(nx, ny):
     """Cells of the multigrid levels below level 0 (cell-centred 2x2
-    coarsening to at most 4096 cells, at least four levels)."""
+    coarsening to at most 4096 cells, at least four levels: the hierarchy of
+    these workloads)."""
     out = []
     while True:
         nx, ny = (nx + 1) // 2, (ny + 1) // 2
@@ -84,8 +88,8 @@ def mg_level_cells(nx, ny):
 
 def cartesian_groups(case):
     n = case.nx * case.ny
-    coarse = 62 * sum(mg_level_cells(case.nx, case.ny)[:-1])
-    return {"spmv_pp": 60 * n, "mg_down0": 33 * n, "mg_up0": 37 * n, "mg_coarse": coarse}
+    coarse = 58 * sum(mg_level_cells(case.nx, case.ny)[:-1])
+    return {"spmv_pp": 60 * n, "mg_down0": 31 * n, "mg_up0": 35 * n, "mg_coarse": coarse}
 
 
 def tel_groups(case):
@@ -100,15 +104,22 @@ def tel_groups(case):
     nbr = np.where(nb > 0, nb - 1, 0)
     near = refined | (refined[nbr] & (nb > 0)).any(axis=1)
     top = lev == lev.max() if lev.max() > 0 else np.zeros(n, bool)
+    # chunks of 64 cells of four faces whose neighbours, all cells, lie at the
+    # same offsets from each
+    k = n // 64 * 64
+    four = ((nb[:, 0::2] > 0) & (nb[:, 1::2] == 0)).all(axis=1)
+    off = (nb[:, 0::2] - np.arange(n)[:, None])[:k].reshape(-1, 64, 4)
+    chunked = np.zeros(n, bool)
+    chunked[:k] = np.repeat((off == off[:, :1]).all(axis=(1, 2)) & four[:k].reshape(-1, 64).all(axis=1), 64)
     squares = 0
     if lev.max() >= 2:
         g = np.asarray(t.geom)[lev >= 1]
         h = case.dx / 2
         squares = len(np.unique(np.floor(g[:, 1] / h) * (2 * case.nx) + np.floor(g[:, 0] / h)))
     return {
-        "spmv_pp": int((36 + 12 * faces).sum()),
-        "mg_down0": 29 * nbase, "mg_up0": 33 * nbase,
-        "mg_coarse": 62 * sum(mg_level_cells(case.nx, case.ny)[:-1]),
+        "spmv_pp": int((28 + 8 * faces).sum() + (8 + 4 * faces)[~chunked].sum()),
+        "mg_down0": 27 * nbase, "mg_up0": 31 * nbase,
+        "mg_coarse": 58 * sum(mg_level_cells(case.nx, case.ny)[:-1]),
         "tel_restrict": int(28 * n + 4 * nbase + (12 + 16 * faces[near]).sum()),
         "tel_fjac": int((36 + 12 * faces[top]).sum()),
         "tel_cs_restrict": int((36 + 16 * faces[lev >= 1]).sum() + 16 * squares),
@@ -435,7 +446,7 @@ def measure(a, case, label, groups):
                    "bytes_per_launch": nbytes,
                    "achieved_GBs": nbytes / (avg * 1e-3) / 1e9 if avg else None}
     # the roofline kernel: the single kernel with the largest total time
-    # (mg_coarse is a span of nine launches, reported beside it)
+    # (mg_coarse is a span of several launches, reported beside it)
     dom = max((k for k in kern if k != "mg_coarse"), key=lambda k: kern[k]["total_ms"])
     # flow_balance and flow_step_stat as the device keeps them (cms2d_flow_balance):
     # balance = storage + efflux = dV - dt Q_in of a step [m^3]
