@@ -43,10 +43,10 @@ HBM_PEAK_GBS = 8000.0
 #             base cell (31)
 #   mg_coarse the levels below level 0 of one V-cycle: down and up sweeps of
 #             level l read and write 27 + 31 = 58 B per level-l cell
-#   tel_restrict    residual r - A Z summed into the base cells: per cell the
-#             list entry, metadata, r, base cell and its range (28 B), on cells
-#             next to refined cells also ap, Z and per face index, coefficient
-#             and Z (12 + 16 F B), 4 B per base cell written
+#   tel_restrict    residual r - A Z summed into the base cells: per cell r
+#             (8 B), on cells next to refined cells also the list entry,
+#             metadata, base cell and its range, ap, Z and per face index,
+#             coefficient and Z (32 + 16 F B), 4 B per base cell written
 #   tel_fjac  damped Jacobi sweep on the finest cells: list entry, metadata,
 #             r, ap, Z in and out, per face index and coefficient: 36 + 12 F B
 #   tel_cs_restrict residual summed into the 10 m squares: per cell of level
@@ -56,13 +56,13 @@ HBM_PEAK_GBS = 8000.0
 # (FETCH_SIZE x 2.00 + WRITE_SIZE x 1.00, factors from a copy kernel of known
 # size) on the uniform 2000 x 1500 workload; the commands and the table are in
 # profiles/traffic_tidal_2000x1500.md.
-TRAFFIC_PER_CELL = {"spmv_pp": (166.8 + 24.5) * 1e6 / 3.0e6,
-                    "mg_down0": (114.3 + 15.2) * 1e6 / 3.0e6,
-                    "mg_up0": (128.1 + 16.9) * 1e6 / 3.0e6}
+TRAFFIC_PER_CELL = {"spmv_pp": (169.1 + 24.6) * 1e6 / 3.0e6,
+                    "mg_down0": (86.6 + 9.1) * 1e6 / 3.0e6,
+                    "mg_up0": (94.9 + 12.0) * 1e6 / 3.0e6}
 # The same per launch on the telescoping workload at 2000 x 1500
 # (profiles/traffic_tel_2000x1500.md).
-TEL_TRAFFIC = {"spmv_pp": 341.6e6, "mg_down0": 111.8e6, "mg_up0": 128.3e6, "tel_restrict": 174.9e6,
-               "tel_cs_restrict": 74.0e6, "tel_fjac": 58.3e6}
+TEL_TRAFFIC = {"spmv_pp": 244.0e6, "mg_down0": 84.1e6, "mg_up0": 94.6e6, "tel_restrict": 136.6e6,
+               "tel_cs_restrict": 91.4e6, "tel_fjac": 73.9e6}
 KERNEL_DESC = {
     "spmv_pp": "k_bicg_spmv MODE 1 and 2 (pp system: v = A z, t = A zs, z from the preconditioner)",
     "mg_down0": "k_mg_down (multigrid level 0: red-black pre-smoothing + restriction)",
@@ -120,7 +120,7 @@ def tel_groups(case):
         "spmv_pp": int((28 + 8 * faces).sum() + (8 + 4 * faces)[~chunked].sum()),
         "mg_down0": 27 * nbase, "mg_up0": 31 * nbase,
         "mg_coarse": 58 * sum(mg_level_cells(case.nx, case.ny)[:-1]),
-        "tel_restrict": int(28 * n + 4 * nbase + (12 + 16 * faces[near]).sum()),
+        "tel_restrict": int(8 * n + 4 * nbase + (32 + 16 * faces[near]).sum()),
         "tel_fjac": int((36 + 12 * faces[top]).sum()),
         "tel_cs_restrict": int((36 + 16 * faces[lev >= 1]).sum() + 16 * squares),
     }
