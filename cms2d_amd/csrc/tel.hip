@@ -96,8 +96,9 @@ __global__ void __launch_bounds__(BLOCK) k_tl_mg_setup0(TelG T, const int *blk, 
 // The residual r - A Z of cell i for a correction Z that is nonzero on
 // refined cells only (so only cells next to them see it), summed in face order.
 // The refined region is small and these sweeps wait for memory, not for
-// bandwidth: everything that cell i itself selects is fetched at once (the
-// slots past the last face hold -1), then Z at the neighbours.  (Slots fetched
+// bandwidth: everything that cell i itself selects is fetched at once (the last
+// two slots of joint cells, -1 past the last face, after its bits: all six at
+// once moved 1.5 times the bytes), then Z at the neighbours.  (Slots fetched
 // after the cell's bits, on 2000 x 1500 base cells with a refined band:
 // restriction of the refined cells 19.4 -> 15.8 us, to the base grid 30.5 ->
 // 23.5 us.)
@@ -109,13 +110,20 @@ __device__ __forceinline__ double tl_res(const TelG &T, const TB *r, const doubl
     int nbk[TF];
     double a[TF];
     float zk[TF];
+    auto slots = [&](int k0, int k1) {
 #pragma unroll
-    for (int k = 0; k < TF; k++) nbk[k] = tnb(T, i, k);
-#pragma unroll
-    for (int k = 0; k < TF; k++) a[k] = apc[k * T.nd + i];
+        for (int k = k0; k < k1; k++) {
+            nbk[k] = tnb(T, i, k);
+            a[k] = apc[k * T.nd + i];
+        }
+    };
+    slots(0, 4);
     const double api = ap[i];
     const float zi = Z[i];
     if (!m_near(m)) return ri;
+    nbk[4] = nbk[5] = -1;
+    a[4] = a[5] = 0.0;
+    if (m_ncf(m) > 4) slots(4, TF);
 #pragma unroll
     for (int k = 0; k < TF; k++) {
         const bool in = nbk[k] >= 0 && nbk[k] < T.n;
