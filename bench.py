@@ -61,8 +61,8 @@ TRAFFIC_PER_CELL = {"spmv_pp": (169.1 + 24.6) * 1e6 / 3.0e6,
                     "mg_up0": (94.9 + 12.0) * 1e6 / 3.0e6}
 # The same per launch on the telescoping workload at 2000 x 1500
 # (profiles/traffic_tel_2000x1500.md).
-TEL_TRAFFIC = {"spmv_pp": 244.0e6, "mg_down0": 84.1e6, "mg_up0": 94.6e6, "tel_restrict": 136.6e6,
-               "tel_cs_restrict": 91.4e6, "tel_fjac": 73.9e6}
+TEL_TRAFFIC = {"spmv_pp": 244.0e6, "mg_down0": 84.1e6, "mg_up0": 94.6e6, "tel_restrict": 121.3e6,
+               "tel_cs_restrict": 74.8e6, "tel_fjac": 58.6e6}
 KERNEL_DESC = {
     "spmv_pp": "k_bicg_spmv MODE 1 and 2 (pp system: v = A z, t = A zs, z from the preconditioner)",
     "mg_down0": "k_mg_down (multigrid level 0: red-black pre-smoothing + restriction)",

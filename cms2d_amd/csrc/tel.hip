@@ -100,8 +100,9 @@ __global__ void __launch_bounds__(BLOCK) k_tl_mg_setup0(TelG T, const int *blk, 
 // two slots of joint cells, -1 past the last face, after its bits: all six at
 // once moved 1.5 times the bytes), then Z at the neighbours.  (Slots fetched
 // after the cell's bits, on 2000 x 1500 base cells with a refined band:
-// restriction of the refined cells 19.4 -> 15.8 us, to the base grid 30.5 ->
-// 23.5 us.)
+// a sweep of the finest cells 13.0 -> 9.7 us, restriction of the refined cells
+// 19.4 -> 13.4, to the base grid 30.5 ->
+// 22.4.)
 template <class TB>
 __device__ __forceinline__ double tl_res(const TelG &T, const TB *r, const double *ap, const double *apc,
                                          const float *Z, int i) {
