@@ -2036,8 +2036,11 @@ extern "C" int cms2d_flow_get(cms2d_flow *F, const char *name, double *out) {
     if (!F || !name || !out) return set_err(CMS2D_ERR_ARG, "null argument");
     if (F->tel) return tel_get(F, name, out);
     HIPCHK(hipSetDevice(F->dev));
-    // packed on the device in the pp solve's t, which holds nothing between solves
-    double *packed = F->Kpp.t[0];
+    // packed on the device in the pp solve's shadow residual: it holds nothing
+    // between solves, each of which writes it first, and no operator reads it at a
+    // neighbour (the vectors that are read there must keep 0 on the ghost ring, which
+    // the packed values cover: NaN or Inf there would outlive the field)
+    double *packed = F->Kpp.r0[0];
     if (!strcmp(name, "iwet")) {
         LAUNCH(k_pack<uint8_t>, F->nblk_act, F->g, (const uint8_t *)F->s.iwet, packed);
     } else {

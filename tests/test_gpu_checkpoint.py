@@ -63,3 +63,29 @@ def test_restore_rejects_other_grids(gpu_available):
     a.restore(ck)                                      # its own checkpoint is accepted
     a.close()
     b.close()
+
+
+@pytest.mark.gpu
+def test_reading_a_non_finite_field_leaves_the_solves_as_they_were(gpu_available):
+    """cms2d_flow_get of a field that holds NaN changes nothing that a later
+    step reads: the flow, restored from its checkpoint, continues bitwise as one
+    that never held it (Jacobi pp solve on the fused sweeps, whose operator
+    reads every Krylov vector at neighbours, ghost cells included)."""
+    c = cases.tidal(nx=48, ny=32, dx=20.0, seed=9)
+    kw = {"precond": _lib.PRECOND_JACOBI, "kmax": 400}
+    print(f"non-finite get {c.nx}x{c.ny}", flush=True)
+    a = FlowStep(c, **kw)
+    a.step(2)
+    ck = a.checkpoint()
+    a.set("v", np.full(c.ncells, np.nan))
+    assert np.isnan(a.get("v")).any()
+    a.restore(ck)
+    b = FlowStep(c, **kw)
+    b.restore(ck)
+    for _ in range(2):
+        ia, ib = a.step(1), b.step(1)
+        assert (ia["niter"], ia["kry"]) == (ib["niter"], ib["kry"])
+    for name in FIELDS:
+        assert np.array_equal(a.get(name), b.get(name)), name
+    a.close()
+    b.close()
