@@ -2032,23 +2032,47 @@ extern "C" int cms2d_flow_tuning(cms2d_flow *F, int *mg_tile_x, int *graphs) {
     return CMS2D_OK;
 }
 
+// Fields of at least this many cells are packed on the device before the copy;
+// below it the launch costs more than the host loop over the padded copy (us a
+// field, host loop and packed: 15 and 27 at 8000 cells, 21 and 31 at 20 000, 36 and
+// 42 at 50 000, 50 and 50 at 75 000, 73 and 67 at 120 000, 2400 and 1370 at 3 M).
+// Wet flags cross as bytes at every size: packed as doubles they are eight times
+// the bytes (us: 20 and 30 at 20 000 cells, 630 and 1380 at 3 M).
+static constexpr int GET_PACK_CELLS = 75000;
+template <class T>
+static void unpad(const Geo &g, const T *h, double *out) {
+    for (int j = 0; j < g.ny; j++)
+        for (int i = 0; i < g.nx; i++) out[(size_t)j * g.nx + i] = h[(size_t)(j + 1) * g.nxp + i + 1];
+}
+
 extern "C" int cms2d_flow_get(cms2d_flow *F, const char *name, double *out) {
     if (!F || !name || !out) return set_err(CMS2D_ERR_ARG, "null argument");
     if (F->tel) return tel_get(F, name, out);
     HIPCHK(hipSetDevice(F->dev));
+    const Geo &g = F->g;
+    if (!strcmp(name, "iwet")) {
+        std::vector<uint8_t> w(F->npad);
+        HIPCHK(hipMemcpyAsync(w.data(), F->s.iwet, F->npad, hipMemcpyDeviceToHost, F->st));
+        HIPCHK(hipStreamSynchronize(F->st));
+        unpad(g, w.data(), out);
+        return CMS2D_OK;
+    }
+    const double *p = field_ptr(F, name);
+    if (!p) return set_err(CMS2D_ERR_ARG, std::string("unknown field ") + name);
+    if (g.nact < GET_PACK_CELLS) {
+        std::vector<double> h(F->npad);
+        HIPCHK(hipMemcpyAsync(h.data(), p, F->npad * sizeof(double), hipMemcpyDeviceToHost, F->st));
+        HIPCHK(hipStreamSynchronize(F->st));
+        unpad(g, h.data(), out);
+        return CMS2D_OK;
+    }
     // packed on the device in the pp solve's shadow residual: it holds nothing
     // between solves, each of which writes it first, and no operator reads it at a
     // neighbour (the vectors that are read there must keep 0 on the ghost ring, which
     // the packed values cover: NaN or Inf there would outlive the field)
     double *packed = F->Kpp.r0[0];
-    if (!strcmp(name, "iwet")) {
-        LAUNCH(k_pack<uint8_t>, F->nblk_act, F->g, (const uint8_t *)F->s.iwet, packed);
-    } else {
-        const double *p = field_ptr(F, name);
-        if (!p) return set_err(CMS2D_ERR_ARG, std::string("unknown field ") + name);
-        LAUNCH(k_pack<double>, F->nblk_act, F->g, p, packed);
-    }
-    HIPCHK(hipMemcpyAsync(out, packed, (size_t)F->g.nact * sizeof(double), hipMemcpyDeviceToHost, F->st));
+    LAUNCH(k_pack, F->nblk_act, g, p, packed);
+    HIPCHK(hipMemcpyAsync(out, packed, (size_t)g.nact * sizeof(double), hipMemcpyDeviceToHost, F->st));
     HIPCHK(hipStreamSynchronize(F->st));
     return CMS2D_OK;
 }

@@ -1473,13 +1473,12 @@ __global__ void k_river_rating(Geo g, St s, int k, int m, double ramp, double *q
 }
 
 // Active cells of a padded array in row-major order (what cms2d_flow_get hands
-// out, so that one copy of the grid's size crosses to the host and no host
-// loop follows: 7 -> 1.7 ms a field at 3 M cells).
-template <class T>
-__global__ void k_pack(Geo g, const T *src, double *dst) {
+// out of large grids, so that one copy of the grid's size crosses to the host
+// and no host loop follows: 2.4 -> 1.4 ms a field at 3 M cells).
+__global__ void k_pack(Geo g, const double *src, double *dst) {
     int i, j, c;
     if (!act_thread(g, i, j, c)) return;
-    dst[j * g.nx + i] = (double)src[c];
+    dst[j * g.nx + i] = src[c];
 }
 // Wet active cells, added to *count: one addition a block of a fixed grid (one
 // a wave met at the same word 56 thousand times at 3.6 M cells, 570 us).

@@ -270,6 +270,21 @@ def test_multigrid_tile_widths_match(gpu_available, monkeypatch):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("shape", [(3, 3), (250, 299), (250, 300), (251, 300)], ids=lambda s: f"{s[0]}x{s[1]}")
+def test_get_returns_what_was_set(gpu_available, shape):
+    """cms2d_flow_get on both sides of the size from which fields are packed on
+    the device (75 000 cells): the values set, cell by cell, and a wet flag of 1."""
+    c = cases.basin(nx=shape[0], ny=shape[1], dx=10.0, seed=2)
+    g = FlowStep(c)
+    u = np.random.default_rng(5).normal(0.0, 0.1, c.ncells)
+    g.set("u", u)
+    assert np.array_equal(g.get("u"), u)
+    assert np.array_equal(g.get("iwet"), np.ones(c.ncells))
+    assert np.array_equal(g.get("zb"), c.zb)
+    g.close()
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("law", [1, 3, 4])
 def test_friction_laws_match_oracle(gpu_available, law):
     """Drag coefficient, roughness height and linear friction (fric_eval's
