@@ -1039,7 +1039,10 @@ static int flow_imp_once(cms2d_flow *F) {
             F->kry[n] += F->h_sc[n].final_iters;
         }
         check_conv(F);
-        if (F->iconv == 0) return set_err(CMS2D_ERR_DIVERGED, "Model is divergent (check_conv iconv=0)");
+        if (F->iconv == 0) {
+            LAUNCH(k_fric_fields, F->nblk_act, g, s, F->P);
+            return set_err(CMS2D_ERR_DIVERGED, "Model is divergent (check_conv iconv=0)");
+        }
         if (F->iconv == 2) break;
     }
     if (F->niter > F->maxit) F->niter = F->maxit;

@@ -75,6 +75,11 @@ __device__ __forceinline__ double length2drag(double z0, double h) {
     double t = F4(0.4) / (log(h / z0lim) - 1.0);
     return t * t;
 }
+// Roughness length of Manning friction.
+__device__ __forceinline__ void fric_law_z0(const Par &P, const St &s, int c, double h, double cd) {
+    const bool manning = P.mbedfric != 1 && P.mbedfric != 3 && P.mbedfric != 4;
+    if (manning && cd != 0.0) s.z0[c] = drag2length(cd, h);
+}
 // The per-law part of fric_eval (friction.F90:638-679): the law's input
 // (cfrict, z0, cbf or coefman) stays, the other coefficients follow from it
 // and the depth; returns the drag coefficient.  z0: whether the roughness length
@@ -101,7 +106,7 @@ __device__ __forceinline__ double fric_law(const Par &P, const St &s, int c, dou
     default:
         cd = man2drag(s.coefman[c], h);
         s.cfrict[c] = cd;
-        if (z0 && cd != 0.0) s.z0[c] = drag2length(cd, h);
+        if (z0) fric_law_z0(P, s, c, h, cd);
     }
     return cd;
 }
@@ -909,8 +914,8 @@ __global__ void k_ghost_p(Geo g, St s, Par P) {
 // flow_grad_interp (flow_imp.F90:1106-1127) + fric_eval (friction.F90:615-797,
 // Manning) + flow_eddyvis cell values (flow_eddyvis.f90:128-160, mturbul=5).
 // all: also what only the initial state needs (k_velface gives a step's final
-// uv, bsvel and z0; between outer iterations z0 is read next to dry cells, by
-// the wall friction).  grads: the gradients are kept (statistics).
+// uv, bsvel and z0, k_fric_fields those of a step that stops before it; between
+// outer iterations z0 is read next to dry cells, by the wall friction).  grads: the gradients are kept (statistics).
 __global__ void k_grad_fric_vis(Geo g, St s, Par P, int all, int grads) {
     int i, j, c;
     if (!act_thread(g, i, j, c)) return;
@@ -1315,6 +1320,18 @@ __global__ void k_velface(Geo g, St s, Par P) {
     else taum = RHOW * cd * Um * Um;
     s.uv[c] = Um; s.uelwc[c] = Uwc;
     s.bsvel[c] = sqrt(taum / RHOW + F4(1.0e-15));
+}
+
+// uv, bsvel and z0 of the last k_grad_fric_vis, for a step that ends as divergent
+// before k_velface: what cms2d_flow_get then hands out belongs to its u, v and h.
+__global__ void k_fric_fields(Geo g, St s, Par P) {
+    int i, j, c;
+    if (!act_thread(g, i, j, c)) return;
+    const double u = s.u[c], v = s.v[c], cd = s.cfrict[c];
+    const double Um = sqrt(u * u + v * v), taum = RHOW * cd * Um * Um;
+    s.uv[c] = Um;
+    s.bsvel[c] = sqrt(taum / RHOW + F4(1.0e-15));
+    fric_law_z0(P, s, c, s.h[c], cd);
 }
 
 // flow_update, CMS_Flow.f90:312-350

@@ -96,3 +96,32 @@ def test_gpu_initial_condition_matches_oracle(gpu_available):
     for name, tol in (("eta", TOL_ETA), ("u", TOL_VEL), ("v", TOL_VEL)):
         err = np.abs(o.get(name) - g.get(name))[wet].max()
         assert err <= tol, (name, err)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("law", [2, 3])
+def test_friction_fields_of_a_divergent_step(gpu_available, law):
+    """The fields read back after a divergent step belong together: current
+    speed, bed velocity and (Manning friction) roughness length are those of its
+    last velocity, depth and drag coefficient."""
+    c, p = dam_break()
+    if law == 3:
+        c.mbedfric, c.mann = 3, np.full(c.ncells, 1.0 / 512.0)
+    print(f"dam break 48x32 dt 300 friction law {law}", flush=True)
+    g = FlowStep(c)
+    g.set("p", p)
+    with pytest.raises(_lib.Cms2dError) as e:
+        g.step(1)
+    assert e.value.code == -3                        # CMS2D_ERR_DIVERGED
+    u, v, h, cd = (g.get(n) for n in ("u", "v", "h", "cfrict"))
+    speed = np.sqrt(u * u + v * v)
+    assert speed.max() > 0.1
+    assert np.allclose(g.get("uv"), speed, rtol=1e-14, atol=0.0)
+    # tau_m = rho cd U^2, bed velocity sqrt(tau_m / rho + 1e-15) (the reference's literals are single)
+    assert np.allclose(g.get("bsvel"), np.sqrt(cd * speed ** 2 + np.float32(1e-15)), rtol=1e-13, atol=0.0)
+    if law == 2:
+        z0 = np.maximum(h / np.exp(np.float64(np.float32(0.4)) / np.sqrt(cd) + 1.0), np.float32(1e-6))
+        assert np.allclose(g.get("z0"), z0, rtol=1e-12, atol=0.0)
+    else:
+        assert np.array_equal(g.get("z0"), c.mann)
+    g.close()
