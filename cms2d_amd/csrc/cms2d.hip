@@ -1228,7 +1228,7 @@ static bool mg_tail_layout(const Mg &M, int l, MgTail &T) {
 static int mg_alloc(cms2d_flow *F, int nx, int ny, double ratio) {
     Mg &M = F->mg;
     size_t ncoarse = 0;                                // padded cells of levels 1 ..
-    auto levels = [&](bool deep, double &r) -> int {
+    auto levels = [&](bool deep, double &r) -> bool {          // false: more than MG_MAX_LEVELS
         M.nlev = 0;
         M.w0 = deep ? 0.5f : 1.0f;
         M.w1 = deep ? 0.25f : 0.0f;
@@ -1243,16 +1243,16 @@ static int mg_alloc(cms2d_flow *F, int nx, int ny, double ratio) {
             M.nlev++;
             MgTail T;
             const bool end = deep ? r <= MG_DEEP_RATIO : M.nlev >= MG_SHORT_LEVELS;
-            if (mg_tail_layout(M, M.nlev - 1, T) && (end || (mx == 1 && my == 1))) return 0;
-            if (M.nlev == MG_MAX_LEVELS) return set_err(CMS2D_ERR_ARG, "grid too large for the multigrid hierarchy");
+            if (mg_tail_layout(M, M.nlev - 1, T) && (end || (mx == 1 && my == 1))) return true;
+            if (M.nlev == MG_MAX_LEVELS) return false;
             mx = (mx + 1) / 2;
             my = (my + 1) / 2;
         }
     };
     double r;                                          // of the coarsest level
-    if (int rc = levels(false, r)) return rc;
-    if (r > MG_SHORT_RATIO)
-        if (int rc = levels(true, r)) return rc;
+    if (!levels(false, r)) return set_err(CMS2D_ERR_ARG, "grid too large for the multigrid hierarchy");
+    // (a side over 32768 cells is not one cell yet on the last level there is)
+    if (r > MG_SHORT_RATIO && !levels(true, r)) levels(false, r);
     float4 *ac;
     float *dc;
     if (int rc = dalloc(F, &ac, ncoarse)) return rc;

@@ -121,6 +121,18 @@ def test_multigrid_shapes_match_oracle(gpu_available, shape, precision):
 
 
 @pytest.mark.gpu
+def test_long_grid_of_stiff_coefficients_is_accepted(gpu_available):
+    """A grid too long to be coarsened to one cell in the levels there are, with
+    g h dt^2/dx^2 at 1e10 (deep water, a long step): it takes the hierarchy that
+    ends sooner, as grids of smaller coefficients do, and is not refused."""
+    c = cases.basin(nx=33000, ny=3, dx=1.0, seed=0, dt=900.0)
+    c.zb = np.full(c.ncells, -1300.0)
+    print(f"long grid {c.nx}x{c.ny}", flush=True)
+    g = FlowStep(c)
+    g.close()
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("shape", [(3, 3), (3, 40), (40, 3), (3, 5), (7, 3)],
                          ids=lambda s: f"{s[0]}x{s[1]}")
 def test_small_shapes_match_oracle(gpu_available, shape):
