@@ -178,8 +178,8 @@ struct cms2d_flow {
     // graphs, one per Krylov system (indexed like d_sc)
     bool use_graphs = false;
     hipGraphExec_t kgraph[6]{};
-    int mg_tile = 128;         // level-0 tile width of the multigrid cycle (timed at creation)
-    int mg_tile_small = 0;     // its 64-wide tile has 8 rows, not 32
+    int mg_tile = 0;           // level-0 tile of the multigrid cycle (MG_TILES; timed at creation)
+    int mg_tile_coarse = -1;   // that of the tiled levels below (-1: by their size)
     // the reference's cell order for the three order-dependent loops: the
     // buffers of consecutive passes (dry-to-wet u, v, vis; fix-up face values
     // [4*npad]; corner values)
@@ -515,21 +515,54 @@ static void mg_level_tile(cms2d_flow *F, KTimer *tm, bool down, const MgLevel &L
     if (down) tlaunch(tm, TG_MG_DOWN0, k_mg_down<TX, TY, NT, TB>, tiles, tb, 0, F->st, L, b, C, sc);
     else tlaunch(tm, TG_MG_UP0, k_mg_up<TX, TY, NT, TB>, tiles, tb, 0, F->st, L, b, C, sc);
 }
+// The tiles there are.
+static constexpr struct { int x, y; } MG_TILES[] = {{64, 8}, {64, 32}, {128, 16}, {256, 8}, {64, 16}};
+enum { MGT_64X8, MGT_64X32, MGT_128X16, MGT_256X8, MGT_64X16, MGT_COUNT, MGT_TIMED = MGT_64X16 };
+template <class TB>
+static void mg_level_on(int tile, cms2d_flow *F, KTimer *tm, bool down, const MgLevel &L, const TB *b,
+                        const MgLevel &C, const KryScal *sc) {
+    switch (tile) {
+    case MGT_64X8: mg_level_tile<64, 8, 128>(F, tm, down, L, b, C, sc); break;
+    case MGT_64X32: mg_level_tile<64, 32, 256>(F, tm, down, L, b, C, sc); break;
+    case MGT_128X16: mg_level_tile<128, 16, 256>(F, tm, down, L, b, C, sc); break;
+    case MGT_256X8: mg_level_tile<256, 8, 256>(F, tm, down, L, b, C, sc); break;
+    default: mg_level_tile<64, 16, 256>(F, tm, down, L, b, C, sc);
+    }
+}
 template <class TB>
 static void mg_level0(cms2d_flow *F, KTimer *tm, bool down, const MgLevel &L0, const TB *b0, const KryScal *sc) {
-    const MgLevel &C = F->mg.L[1];
-    if (F->mg_tile == 64 && F->mg_tile_small) mg_level_tile<64, 8, 128>(F, tm, down, L0, b0, C, sc);
-    else if (F->mg_tile == 64) mg_level_tile<64, 32, 256>(F, tm, down, L0, b0, C, sc);
-    else if (F->mg_tile == 256) mg_level_tile<256, 8, 256>(F, tm, down, L0, b0, C, sc);
-    else mg_level_tile<128, 16, 256>(F, tm, down, L0, b0, C, sc);
+    mg_level_on(F->mg_tile, F, tm, down, L0, b0, F->mg.L[1], sc);
 }
 // Levels 1 .. lt-1 (64 x 16 needs 400 workgroups to fill the chip: 5.7 us on
 // 750 000 cells, 6.6 with 64 x 8).
 static void mg_level(cms2d_flow *F, bool down, int l, const KryScal *sc) {
-    const MgLevel &L = F->mg.L[l], &C = F->mg.L[l + 1];
-    const float *b = L.b;
-    if ((long)L.nx * L.ny >= 400000) mg_level_tile<64, 16, 256>(F, nullptr, down, L, b, C, sc);
-    else mg_level_tile<64, 8, 128>(F, nullptr, down, L, b, C, sc);
+    const MgLevel &L = F->mg.L[l];
+    const int tile = F->mg_tile_coarse >= 0              ? F->mg_tile_coarse
+                     : (long)L.nx * L.ny >= 400000 ? MGT_64X16
+                                                   : MGT_64X8;
+    mg_level_on(tile, F, nullptr, down, L, (const float *)L.b, F->mg.L[l + 1], sc);
+}
+// The level-0 tile of a grid of n cells before any timing; true if the
+// environment fixes it (tests): CMS2D_MG_TILE=64, 128 or 256, a width on level
+// 0, or one of MG_TILES (64x32, say) on every tiled level.
+static bool mg_tile_fixed(cms2d_flow *F, int n, int large) {
+    F->mg_tile = n < MG_SMALL_LEVEL0 ? MGT_64X8 : large;
+    const char *e = getenv("CMS2D_MG_TILE");
+    if (!e) return false;
+    int x = 0, y = 0;
+    const int got = sscanf(e, "%dx%d", &x, &y);
+    for (int t = 0; t < MGT_COUNT; t++) {
+        if (got == 2 && x == MG_TILES[t].x && y == MG_TILES[t].y) {
+            F->mg_tile = F->mg_tile_coarse = t;
+            return true;
+        }
+        const bool width = x == 64 ? t == (n < MG_SMALL_LEVEL0 ? MGT_64X8 : MGT_64X32) : x == MG_TILES[t].x;
+        if (got == 1 && width) {
+            F->mg_tile = t;
+            return true;
+        }
+    }
+    return false;
 }
 // A thread per block of the tail's first level.
 static int mg_tail_threads(int nblk) { return nblk <= 256 ? 256 : nblk <= 512 ? 512 : MG_TAIL_NT; }
@@ -569,15 +602,7 @@ static void mg_vcycle(cms2d_flow *F, const TB *b0, float *z0, const KryScal *sc)
 // Picks the level-0 tile of the cycle by timing the down and up launches of
 // each candidate on this grid; every tile gives the same values.
 static int tune_mg_tile(cms2d_flow *F) {
-    static constexpr struct { int tile, small; } cand[4] = {{64, 1}, {64, 0}, {128, 0}, {256, 0}};
-    F->mg_tile_small = F->g.nact < MG_SMALL_LEVEL0;
-    if (F->mg_tile_small) F->mg_tile = 64;
-    if (F->mg.lt == 0) return 0;
-    if (const char *e = getenv("CMS2D_MG_TILE")) {   // fixed width (tests)
-        const int t = atoi(e);
-        if (t == 64 || t == 128 || t == 256) { F->mg_tile = t; return 0; }
-    }
-    if (F->mg_tile_small) return 0;
+    if (mg_tile_fixed(F, F->g.nact, MGT_64X8) || F->mg.lt == 0 || F->g.nact < MG_SMALL_LEVEL0) return 0;
     MgLevel L0 = F->mg.L[0];
     L0.zo = F->Kpp.zp;
     const double *b0 = F->Kpp.p[0];
@@ -587,9 +612,8 @@ static int tune_mg_tile(cms2d_flow *F) {
     HIPCHK(hipEventCreate(&ev[1]));
     float best = 0.0f;
     int pick = 0;
-    for (int q = 0; q < 4; q++) {
-        F->mg_tile = cand[q].tile;
-        F->mg_tile_small = cand[q].small;
+    for (int q = 0; q < MGT_TIMED; q++) {
+        F->mg_tile = q;
         mg_level0(F, nullptr, true, L0, b0, F->d_sc);          // warm-up
         mg_level0(F, nullptr, false, L0, b0, F->d_sc);
         HIPCHK(hipEventRecord(ev[0], F->st));
@@ -605,8 +629,7 @@ static int tune_mg_tile(cms2d_flow *F) {
     }
     (void)hipEventDestroy(ev[0]);
     (void)hipEventDestroy(ev[1]);
-    F->mg_tile = cand[pick].tile;
-    F->mg_tile_small = cand[pick].small;
+    F->mg_tile = pick;
     return 0;
 }
 
@@ -2030,7 +2053,7 @@ extern "C" int cms2d_flow_set_wind(cms2d_flow *F, double wndx, double wndy) {
 
 extern "C" int cms2d_flow_tuning(cms2d_flow *F, int *mg_tile_x, int *graphs) {
     if (!F || !mg_tile_x || !graphs) return set_err(CMS2D_ERR_ARG, "null argument");
-    *mg_tile_x = F->mg.lt > 0 ? F->mg_tile : 0;
+    *mg_tile_x = F->mg.lt > 0 ? MG_TILES[F->mg_tile].x : 0;
     *graphs = F->use_graphs ? 1 : 0;
     return CMS2D_OK;
 }

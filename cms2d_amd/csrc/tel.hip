@@ -1438,12 +1438,7 @@ static int tel_create(const cms2d_flow_desc *d, const cms2d_tel_grid *tg, cms2d_
     if (int rc = mg_alloc(F, d->nx, d->ny, 0.0)) return rc;
     if (int rc = dalloc(F, &F->mg.L[0].zo, (size_t)(d->nx + 2) * (d->ny + 2))) return rc;
     if (int rc = dalloc(F, &H.b0, (size_t)(d->nx + 2) * (d->ny + 2))) return rc;
-    F->mg_tile = d->nx * d->ny < MG_SMALL_LEVEL0 ? 64 : 128;
-    F->mg_tile_small = d->nx * d->ny < MG_SMALL_LEVEL0;
-    if (const char *e = getenv("CMS2D_MG_TILE")) {
-        const int tt = atoi(e);
-        if (tt == 64 || tt == 128 || tt == 256) F->mg_tile = tt;
-    }
+    mg_tile_fixed(F, d->nx * d->ny, MGT_128X16);
     HIPCHK(hipHostMalloc((void **)&F->h_sc, 6 * sizeof(KryScal), hipHostMallocDefault));
     HIPCHK(hipHostMalloc((void **)&F->h_flags, 4 * sizeof(int), hipHostMallocDefault));
     memset(F->h_sc, 0, 6 * sizeof(KryScal));

@@ -282,6 +282,30 @@ def test_multigrid_tile_widths_match(gpu_available, monkeypatch):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("precision", [_lib.PREC_FP64, _lib.PREC_FP32_REFINE])
+@pytest.mark.parametrize("shape", [(301, 203), (257, 131)], ids=lambda s: f"{s[0]}x{s[1]}")
+def test_multigrid_tile_shapes_match(gpu_available, monkeypatch, shape, precision):
+    """Every tile of the cycle's kernels, the ones that only large levels pick
+    included, on every tiled level (two here) gives bitwise the same steps: FP64
+    and FP32 right-hand sides, sizes that leave a remainder in each tile and one
+    cell more than a whole number of them."""
+    c = cases.tidal(nx=shape[0], ny=shape[1], dx=20.0, seed=6)
+    runs = []
+    for tile in ("64x8", "64x16", "64x32", "128x16", "256x8"):
+        monkeypatch.setenv("CMS2D_MG_TILE", tile)
+        print(f"tile {tile} tidal {shape} precision {precision}, 4 steps", flush=True)
+        g = FlowStep(c, precision=precision)
+        assert g.tuning()[0] == int(tile.split("x")[0])
+        kry = [g.step(1)["kry"] for _ in range(4)]
+        runs.append((kry, [g.get(n) for n in ("eta", "u", "v", "p")]))
+        g.close()
+    for r in runs[1:]:
+        assert r[0] == runs[0][0]
+        for a, b in zip(r[1], runs[0][1]):
+            assert np.array_equal(a, b)
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("shape", [(3, 3), (250, 299), (250, 300), (251, 300)], ids=lambda s: f"{s[0]}x{s[1]}")
 def test_get_returns_what_was_set(gpu_available, shape):
     """cms2d_flow_get on both sides of the size from which fields are packed on
