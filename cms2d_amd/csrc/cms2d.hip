@@ -177,6 +177,7 @@ struct cms2d_flow {
     // launch-bound grids: BiCGStab iteration pairs replayed from captured
     // graphs, one per Krylov system (indexed like d_sc)
     bool use_graphs = false;
+    int fused = 0;             // KryCtx::fused
     hipGraphExec_t kgraph[6]{};
     int mg_tile = 0;           // level-0 tile of the multigrid cycle (MG_TILES; timed at creation)
     int mg_tile_coarse = -1;   // that of the tiled levels below (-1: by their size)
@@ -369,7 +370,13 @@ struct KryCtx {
     int *prev_iters, *last_iters;  // expected counts (0: unknown), and the last solve's
     KTimer *tm;                    // timed launches (or null)
     hipGraphExec_t *graph = nullptr;   // per-system graph slots (or null: direct launches)
+    int fused = KRY_FUSED;             // cells up to which the Jacobi iteration runs in three launches
 };
+// CMS2D_FUSED_CELLS in the environment sets that limit (tests: 0 for none).
+static int fused_cells() {
+    const char *e = getenv("CMS2D_FUSED_CELLS");
+    return e ? atoi(e) : KRY_FUSED;
+}
 
 // BiCGStab iterations from the third on replay pairs from a graph captured
 // at creation.  On small grids a launch lasts about as long as the host takes
@@ -407,7 +414,7 @@ template <class Op, int NS, int PREC, class T, class Pre>
 static void bicg_iter(const KryCtx &X, KrySys<NS, T> &K, Op A, Pre &pre, int i) {
     const dim3 grid(X.nblk), blk(KBLOCK);
     if (X.tm) X.tm->it = i;
-    if constexpr (PREC == 0 && Op::FUSED > 0) if (A.n() <= Op::FUSED) {
+    if constexpr (PREC == 0 && Op::FUSED) if (A.n() <= X.fused) {
         hipLaunchKernelGGL((k_bicg_f1<Op, NS, T>), grid, blk, 0, X.st, A, K, i, X.nblk, X.kmax, X.rtol, X.atol);
         hipLaunchKernelGGL((k_bicg_f2<Op, NS, T>), grid, blk, 0, X.st, A, K, i, X.nblk);
         hipLaunchKernelGGL((k_bicg_f3<Op, NS, T>), grid, blk, 0, X.st, A, K, i, X.nblk);
@@ -804,6 +811,7 @@ static KryCtx flow_ctx(cms2d_flow *F, bool timed) {
     X.last_iters = F->last_iters;
     X.tm = (timed && F->stats) ? &F->tm : nullptr;
     X.graph = F->use_graphs ? F->kgraph : nullptr;
+    X.fused = F->fused;
     return X;
 }
 
@@ -1439,6 +1447,7 @@ static int create_impl(const cms2d_flow_desc *d, cms2d_flow *F) {
     // 48 x 32 one walked three passes a block on 6 of them)
     F->nblk_kry = std::min(KRY_BLOCKS, std::max(F->nblk_act, (g.nx + KW_STRIP - 1) / KW_STRIP *
                                                                  ((g.ny + KW_ROWS - 1) / KW_ROWS)));
+    F->fused = fused_cells();
     F->use_graphs = true;
     if (const char *e = getenv("CMS2D_GRAPHS")) F->use_graphs = atoi(e) != 0;   // 0: direct launches, 1: graphs
     Par &P = F->P;
@@ -1548,7 +1557,7 @@ static int create_impl(const cms2d_flow_desc *d, cms2d_flow *F) {
             F->Kuv.dinv_w[q] = kv[q + 1][6];
         }
         F->Kuv.sc = F->d_sc + 1;
-        for (int q = 0; q < 2; q++)
+        for (int q = 0; q < 2 && g.nact <= F->fused; q++)
             if (int rc = dalloc(F, &F->Kuv.p2[q], N)) return rc;
         F->Kpp.p2[0] = F->Kuv.p2[0];       // (pp without a multigrid; solves do not overlap)
     }
@@ -1587,10 +1596,12 @@ static int create_impl(const cms2d_flow_desc *d, cms2d_flow *F) {
         if (F->precision == CMS2D_PREC_FP32_REFINE) {
             KrySys<2, float> &K2 = F->Kin2;
             for (int q = 0; q < 2; q++) {
-                float **vec[] = {&K2.x[q], &K2.r[q], &K2.r0[q], &K2.p[q], &K2.p2[q],
-                                 &K2.v[q], &K2.t[q], &K2.ap_w[q], &K2.dinv_w[q]};
+                float **vec[] = {&K2.x[q], &K2.r[q], &K2.r0[q], &K2.p[q], &K2.v[q],
+                                 &K2.t[q], &K2.ap_w[q], &K2.dinv_w[q]};
                 for (float **v : vec)
                     if (int rc = dalloc(F, v, N)) return rc;
+                if (g.nact <= F->fused)
+                    if (int rc = dalloc(F, &K2.p2[q], N)) return rc;
             }
             if (int rc = dalloc(F, &F->a32, N)) return rc;
             double *ri;
@@ -2238,6 +2249,7 @@ static int solve_device(const SolveBufs &B, hipStream_t st, int ncells, int nmax
     int prev = 0, last = 8;
     KryCtx X{st, nblk, kmax > 0 ? kmax : 4000, rtol > 0 ? rtol : 1e-10, atol >= 0 ? atol : 1e-12,
              B.sc, &h_sc, &prev, &last, nullptr};
+    X.fused = fused_cells();
     if (int rc = run_bicg(X, K, A, 0)) return rc;
     HIPCHK(hipStreamSynchronize(st));
     return 0;

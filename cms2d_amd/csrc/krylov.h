@@ -132,10 +132,11 @@ __device__ __forceinline__ void grid_walk(const Geo &g, F &&f) {
 }
 
 // Systems of up to this many cells take the Jacobi iteration in three launches
-// (k_bicg_f1): at 20 000 cells 24 us against 26 for two systems and 13 % of a
-// whole cms2d_solve call; equal at 120 000; at 3 M cells 349 against 275 us,
-// where forming p and s at every neighbour costs more loads than the sweeps
-// save.
+// (k_bicg_f1): at 20 000 cells 24 us against 26 for two systems; a cms2d_solve
+// call of 22 iterations, five launches and three, 965 and 828 us at 19 481 cells of
+// four faces, 2266 and 2140 at 23 837 of six, 2735 and 2593 at 43 520 of six; two
+// systems are equal at 120 000; at 3 M cells 349 against 275 us, where forming p
+// and s at every neighbour costs more loads than the sweeps save.
 constexpr int KRY_FUSED = 65536;
 
 // Matrix operators: y_i = ap_i z_i - sum_k a_k(i) z_nb(k).  apply() is the
@@ -145,7 +146,7 @@ constexpr int KRY_FUSED = 65536;
 // neighbours are read without a bounds test, whose branches would each wait
 // for their own load.
 struct StencilOp {
-    static constexpr int FUSED = KRY_FUSED;
+    static constexpr bool FUSED = true;   // the Jacobi iteration in three launches (k_bicg_f1)
     using C = double;
     Geo g;
     const C *aN, *aE, *aS, *aW;
@@ -153,13 +154,6 @@ struct StencilOp {
     __device__ __forceinline__ GridWalk walk() const { return GridWalk(g); }
     template <class F>
     __device__ __forceinline__ void each(F &&f) const { grid_walk(g, f); }
-    __device__ __forceinline__ Idx at(int t) const {
-        Idx x;
-        x.j = t / g.nx;
-        x.i = t - x.j * g.nx;
-        x.c = cidx(g, x.i, x.j);
-        return x;
-    }
     // sum_k a_k z_nb of NS vectors, get(q, nb) the value of vector q at cell nb
     // (V: their type)
     template <int NS, class V, class Get>
@@ -196,7 +190,7 @@ struct StencilOp {
 };
 // The same operator in FP32, the four coefficients of a cell side by side (N, E, S, W).
 struct StencilOp32 {
-    static constexpr int FUSED = KRY_FUSED;
+    static constexpr bool FUSED = true;   // the Jacobi iteration in three launches (k_bicg_f1)
     Geo g;
     const float4 *a;
     __host__ __device__ __forceinline__ int n() const { return g.nact; }
@@ -235,7 +229,7 @@ struct StencilOp32 {
 // (0-based, ghosts numbered from ncells, -1 for no face).
 constexpr int ELL_MAX_FACES = 8;   // nmaxfaces: 4 Cartesian, 6 telescoping (read_tel, geospatial.F90:433)
 struct EllOp {
-    static constexpr int FUSED = KRY_FUSED;
+    static constexpr bool FUSED = true;   // the Jacobi iteration in three launches (k_bicg_f1)
     int ncells, nf;      // cells, faces per cell (row stride of c2c and a)
     const int *c2c;
     const double *a;
@@ -279,7 +273,7 @@ struct EllOp {
 template <int NS, class T = double>
 struct KrySys {
     T *x[NS], *r[NS], *r0[NS], *p[NS], *v[NS], *t[NS];
-    T *p2[NS];         // second buffer of p in the fused form (k_bicg_f1)
+    T *p2[NS];         // second buffer of p in the fused form (k_bicg_f1; null on larger systems)
     T *ap_w[NS];       // diagonal ap of each system (written by the prologue)
     T *dinv_w[NS];     // 1/ap (Jacobi form)
     float *zp, *zs;    // M^-1 p and M^-1 s of system 0 (explicit preconditioner only)

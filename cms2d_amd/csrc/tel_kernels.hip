@@ -623,7 +623,7 @@ __global__ void k_tl_defcor_skew(TelG T, TelS s, const double *dux, const double
 // over active neighbours (z = 0 on ghost cells, pbicgstab.f90:55,76).
 template <class CA>
 struct TelOpT {
-    static constexpr int FUSED = 0;       // (six faces a cell: not measured to gain)
+    static constexpr bool FUSED = false;  // (six faces a cell: not measured to gain)
     int nc, nd;
     const int *c2c;
     const uint64_t *meta;

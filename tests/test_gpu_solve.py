@@ -8,8 +8,8 @@ import numpy as np
 import pytest
 
 from cell_list import cart_cell_list, dense_system, tel_cell_list
-from cms2d_amd import cases
-from cms2d_amd.flow import solve
+from cms2d_amd import _lib, cases
+from cms2d_amd.flow import FlowStep, solve, solve_adjoint
 from pyoracle import D, I, Oracle, lib as olib
 
 
@@ -172,3 +172,59 @@ def test_jacobi_iterations_within_five_times_block_lu():
     _, _, it_g = solve(acoef, c2c, np.ones(nd, dtype=np.int32), ss.copy(), sp, phi.copy(), 1.0, ncells=n)
     print("GPU Jacobi-BiCGStab", it_g, "block dense-LU BiCGStab", it[0], flush=True)
     assert it_g < 5 * it[0]
+
+
+def _flow_fields(c, steps, **kw):
+    g = FlowStep(c, **kw)
+    kry = [g.step(1)["kry"] for _ in range(steps)]
+    out = [g.get(n) for n in ("eta", "u", "v", "p")]
+    g.close()
+    return kry, out
+
+
+def _list_solves(faces):
+    if faces == 4:
+        n, nd, c2c, acoef, sp, ss, phi, iwet = make_system(7, nx=61, ny=43)
+    else:
+        refined = np.zeros((30, 40), bool)
+        refined[6:20, 0:14] = True
+        n, nd, c2c, _, _ = tel_cell_list(refined)
+        rng = np.random.default_rng(8)
+        acoef = np.where(c2c >= 0, rng.uniform(0.2, 2.0, c2c.shape), 0.0)
+        acoef[n:] = 0.0
+        sp, ss, phi, iwet = np.zeros(nd), np.zeros(nd), rng.normal(size=nd), np.ones(nd, dtype=np.int32)
+        sp[:n], ss[:n] = -rng.uniform(0.05, 0.5, n), rng.normal(size=n)
+    p = phi.copy()
+    res, rmom, it = solve(acoef, c2c, iwet, ss, sp, p, 0.8, ncells=n)
+    *grads, itg = solve_adjoint(acoef, c2c, sp, phi, p, 0.8, np.random.default_rng(9).normal(size=n), ncells=n)
+    return [it, itg], [p, ss, res, *grads]
+
+
+FUSED_FORMS = {
+    "fp64": lambda: _flow_fields(cases.tidal(nx=70, ny=45, dx=20.0, seed=2), 6),
+    "fp32": lambda: _flow_fields(cases.tidal(nx=70, ny=45, dx=20.0, seed=2), 6, precision=_lib.PREC_FP32_REFINE),
+    "jacobi": lambda: _flow_fields(cases.basin(nx=40, ny=20, dx=10.0, seed=0), 6, precond=_lib.PRECOND_JACOBI),
+    "strip": lambda: _flow_fields(cases.basin(nx=300, ny=5, dx=10.0, seed=0), 4, precond=_lib.PRECOND_JACOBI),
+    "list4": lambda: _list_solves(4),
+    "list6": lambda: _list_solves(6),
+}
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("form", list(FUSED_FORMS))
+def test_three_launch_iteration_equals_five_sweeps(gpu_available, monkeypatch, form):
+    """The Jacobi iteration in three launches (small systems) and in five
+    (larger ones, here by CMS2D_FUSED_CELLS=0) form the same values in the same
+    order: bitwise the same results and iteration counts for every solve that
+    takes it -- u/v of the FP64 and FP32 forms, pp without a multigrid, cell
+    lists of four and six faces and their reverse (the transposed u/v solves:
+    test_gpu_step_adjoint.py)."""
+    runs = []
+    for cells in ("65536", "0"):
+        monkeypatch.setenv("CMS2D_FUSED_CELLS", cells)
+        print(f"fused up to {cells} cells, {form}", flush=True)
+        runs.append(FUSED_FORMS[form]())
+    assert runs[0][0] == runs[1][0]
+    assert any(np.abs(a).max() > 0 for a in runs[0][1])
+    for a, b in zip(runs[0][1], runs[1][1]):
+        assert np.array_equal(a, b)

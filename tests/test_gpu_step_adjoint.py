@@ -122,6 +122,22 @@ def test_adjoint_matches_central_differences(gpu_available, name):
         assert abs(ad - fd) <= REL_DIR * abs(fd)
 
 
+def test_adjoint_on_the_five_sweeps(gpu_available, monkeypatch):
+    """The u/v solves and their transposed ones by five launches an iteration, as
+    on grids above 65 536 cells: the same forward bitwise, the gradients to the
+    rounding of the reverse kernels' atomic sums (the bound of the next test)."""
+    c, nsteps, gauges, _ = _case("square")
+    obs = np.zeros((nsteps, len(gauges)))
+    runs = []
+    for cells in ("65536", "0"):
+        monkeypatch.setenv("CMS2D_FUSED_CELLS", cells)
+        print(f"step adjoint, fused up to {cells} cells", flush=True)
+        runs.append(_adjoint(c, nsteps, gauges, obs, every=2))
+    assert np.array_equal(runs[0][0], runs[1][0]) and runs[0][1] == runs[1][1]
+    for a, b in zip(runs[0][2:], runs[1][2:]):
+        assert np.abs(a - b).max() <= 1e-12 * np.abs(a).max()
+
+
 def test_adjoint_checkpoint_interval_and_state(gpu_available):
     """Every checkpoint interval recomputes the same forward: the gradients
     agree to rounding (the reverse kernels' atomic sums), and the flow is
