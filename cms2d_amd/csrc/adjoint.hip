@@ -35,7 +35,8 @@ struct Tape {
 
 static size_t state_bytes(const cms2d_flow *F) {
     size_t n = 0;
-    for (auto &a : F->state) n += a.second;
+    for (auto &a : F->state)
+        if (a.first) n += a.second;
     return n;
 }
 // Copies gathered into launches of k_copy_list on the flow's stream.
@@ -71,6 +72,7 @@ static int snap_save(cms2d_flow *F, Snap &S) {
     Copies C(F);
     size_t off = 0;
     for (auto &a : F->state) {
+        if (!a.first) continue;
         C.add(S.dev + off, a.first, a.second);
         off += a.second;
     }
@@ -83,6 +85,7 @@ static int snap_load(cms2d_flow *F, const Snap &S) {
     Copies C(F);
     size_t off = 0;
     for (auto &a : F->state) {
+        if (!a.first) continue;
         C.add(a.first, S.dev + off, a.second);
         off += a.second;
     }
@@ -101,6 +104,7 @@ static St snap_view(const cms2d_flow *F, const Snap &S) {
     for (int k = 0; k < NP; k++) {
         size_t off = 0;
         for (auto &a : F->state) {
+            if (!a.first) continue;
             if (a.first == slot[k]) { slot[k] = S.dev + off; break; }
             off += a.second;
         }

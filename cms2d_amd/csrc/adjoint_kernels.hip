@@ -1065,7 +1065,7 @@ __global__ void k_r_zbk(Geo g, Ad A) {
 }
 
 // Copies of up to COPY_MAX arrays in one launch (blockIdx.y the array), 16 B a
-// thread where both sides allow it.  A state snapshot is 67 arrays and an outer
+// thread where both sides allow it.  A state snapshot is 70 arrays and an outer
 // iteration keeps 26 more: as copies of their own each was a launch, 2.2 us and
 // the gap after it at 400 x 300 cells.
 constexpr int COPY_MAX = 64;

@@ -155,7 +155,9 @@ struct cms2d_flow {
     KryScal *h_sc = nullptr;   // pinned mirror
     int *h_flags = nullptr;    // pinned
     std::vector<void *> allocs;
-    std::vector<std::pair<void *, size_t>> state;   // device arrays of the model state (checkpointed)
+    // device arrays of the model state (checkpointed); null: room that the checkpoint's
+    // layout keeps for an array that is no longer there
+    std::vector<std::pair<void *, size_t>> state;
     int npad = 0, nblk_act = 0, nblk_pad = 0, nblk_kry = 0;
     int ntc = 0;
     double amp[8]{}, speed[8]{}, phase[8]{};
@@ -1484,15 +1486,16 @@ static int create_impl(const cms2d_flow_desc *d, cms2d_flow *F) {
     St &s = F->s;
     const size_t N = F->npad;
     double **dfields[] = {&s.u, &s.v, &s.p, &s.h, &s.pp, &s.zb, &s.vis, &s.visb, &s.visc, &s.u1, &s.v1, &s.p1,
-                          &s.h1, &s.eta, &s.dppx, &s.dppy, &s.dux, &s.duy, &s.dvx, &s.dvy, &s.dpx, &s.dpy,
-                          &s.coefman, &s.cfrict, &s.z0, &s.uv, &s.uelwc, &s.bsvel, &s.su, &s.sv, &s.sp, &s.spu,
+                          &s.h1, &s.eta, nullptr, nullptr, &s.dux, &s.duy, &s.dvx, &s.dvy, &s.dpx, &s.dpy,
+                          &s.coefman, &s.cfrict, &s.z0, &s.uv, &s.uelwc, &s.bsvel, nullptr, nullptr, &s.sp, &s.spu,
                           &s.spv, &s.ssu0, &s.ssv0, &s.spuv0, &s.sppp0, &s.sspp0, &s.apuareap, &s.sumu, &s.Hu,
                           &s.Hv, &s.resu, &s.resv, &s.resp, &s.fluxE, &s.fluxN, &s.hkE, &s.hkN, &s.viskE,
                           &s.viskN, &s.zbkE, &s.zbkN, &s.aN, &s.aE, &s.aS, &s.aW, &s.wavestrx, &s.wavestry,
                           &s.tu, &s.tv, &s.tvis, &s.fluxE1, &s.fluxN1, &s.fc, &s.cbf, &s.maxeta};
     for (double **f : dfields) {
-        if (int rc = dalloc(F, f, N)) return rc;
-        F->state.push_back({*f, N * sizeof(double)});
+        if (f)
+            if (int rc = dalloc(F, f, N)) return rc;
+        F->state.push_back({f ? *f : nullptr, N * sizeof(double)});
     }
     if (int rc = dalloc(F, &s.wseadj, 4 * (size_t)P.lmax)) return rc;
     F->state.push_back({s.wseadj, 4 * (size_t)P.lmax * sizeof(double)});
@@ -2016,7 +2019,8 @@ extern "C" int cms2d_flow_checkpoint(cms2d_flow *F, void *buf, size_t *nbytes) {
     memcpy(q, &c, sizeof c);
     q += sizeof c;
     for (auto &a : F->state) {
-        HIPCHK(hipMemcpyAsync(q, a.first, a.second, hipMemcpyDeviceToHost, F->st));
+        if (a.first) HIPCHK(hipMemcpyAsync(q, a.first, a.second, hipMemcpyDeviceToHost, F->st));
+        else memset(q, 0, a.second);
         q += a.second;
     }
     HIPCHK(hipStreamSynchronize(F->st));
@@ -2042,7 +2046,7 @@ extern "C" int cms2d_flow_restore(cms2d_flow *F, const void *buf, size_t nbytes)
     HIPCHK(hipSetDevice(F->dev));
     HIPCHK(hipStreamSynchronize(F->st));
     for (auto &a : F->state) {
-        HIPCHK(hipMemcpyAsync(a.first, q, a.second, hipMemcpyHostToDevice, F->st));
+        if (a.first) HIPCHK(hipMemcpyAsync(a.first, q, a.second, hipMemcpyHostToDevice, F->st));
         q += a.second;
     }
     HIPCHK(hipStreamSynchronize(F->st));

@@ -8,11 +8,11 @@ namespace cms {
 // Device pointers of every field (padded cell arrays unless noted).
 struct St {
     double *u, *v, *p, *h, *pp, *zb, *vis, *visb, *visc, *u1, *v1, *p1, *h1, *eta;
-    double *dppx, *dppy, *dux, *duy, *dvx, *dvy, *dpx, *dpy;
+    double *dux, *duy, *dvx, *dvy, *dpx, *dpy;
     double *coefman, *cfrict, *z0, *uv, *uelwc, *bsvel;
     double *cbf;               // linear friction coefficient (cbotfric of mbedfric 4)
     double *maxeta;            // running maximum of eta (flow_def maxeta)
-    double *su, *sv, *sp, *spu, *spv, *ssu0, *ssv0, *spuv0, *sppp0, *sspp0;
+    double *sp, *spu, *spv, *ssu0, *ssv0, *spuv0, *sppp0, *sspp0;
     double *apuareap, *sumu, *Hu, *Hv, *resu, *resv, *resp;
     double *fluxE, *fluxN, *hkE, *hkN, *viskE, *viskN, *zbkE, *zbkN;   // unique faces
     double *aN, *aE, *aS, *aW;                                         // directed coefficients
