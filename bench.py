@@ -76,13 +76,13 @@ KERNEL_DESC = {
 
 def mg_level_cells(nx, ny):
     """Cells of the multigrid levels below level 0 (cell-centred 2x2
-    coarsening to at most 4096 cells, at least four levels: the hierarchy of
-    these workloads)."""
+    coarsening to a level of at most 1024 2x2 blocks, at least four levels: the
+    hierarchy of these workloads)."""
     out = []
     while True:
         nx, ny = (nx + 1) // 2, (ny + 1) // 2
         out.append(nx * ny)
-        if nx * ny <= 4096 and len(out) >= 3:
+        if ((nx + 1) // 2) * ((ny + 1) // 2) <= 1024 and len(out) >= 3:
             return out
 
 

@@ -1015,7 +1015,8 @@ static int flow_imp_once(cms2d_flow *F) {
             if (int rc = tape_snap(F, F->niter - 1)) return rc;
         river_vel(F);
         if (F->P.ndsch >= 5 && F->P.ndsch <= 9) LAUNCH(k_defcor, F->nblk_act, g, s, F->P);
-        hipLaunchKernelGGL(F->P.ndsch == 4 ? k_mom<4> : k_mom<-1>, dim3(F->nblk_kry), dim3(KBLOCK), 0, F->st, g, s, F->P, F->Kuv, keep);
+        hipLaunchKernelGGL(F->P.ndsch == 4 ? k_mom<4> : k_mom<-1>, dim3(F->nblk_kry), dim3(KBLOCK), 0, F->st, g, s,
+                           F->P, F->Kuv, keep);
         TAPE(TAPE_MOM);
         {
             KryCtx X = flow_ctx(F, false);
@@ -2442,8 +2443,8 @@ extern "C" int cms2d_solve_adjoint(int ncells, int ncellsD, int nmaxfaces, const
         HIPCHK(hipMemcpyAsync(gp, gphi, n * sizeof(double), hipMemcpyHostToDevice, st));
         const EllOp A{ncells, nmaxfaces, c2c, a};
         const unsigned nb = (unsigned)((n + BLOCK - 1) / BLOCK);
-        hipLaunchKernelGGL(k_adj_setup, dim3((unsigned)((nD + BLOCK - 1) / BLOCK)), dim3(BLOCK), 0, st, A, ncellsD, (const int *)bk, (const double *)spd, relax,
-                           (const double *)gp, B.a, B.sp, B.ss, B.phi);
+        hipLaunchKernelGGL(k_adj_setup, dim3((unsigned)((nD + BLOCK - 1) / BLOCK)), dim3(BLOCK), 0, st, A, ncellsD,
+                           (const int *)bk, (const double *)spd, relax, (const double *)gp, B.a, B.sp, B.ss, B.phi);
         hipLaunchKernelGGL(k_set_int, dim3(nb), dim3(BLOCK), 0, st, B.w, ncells, 1);
         KryScal h_sc{};
         if (int r = solve_device(B, st, ncells, nmaxfaces, 1.0, rtol, atol, kmax, h_sc, 0.0)) return r;

@@ -97,8 +97,8 @@ struct KryStart {
 // batch so the host can read the state; the next batch repeats the same
 // finish (same inputs, same result) before its first p update.
 template <class Op, int NS, class T = double>
-__global__ void __launch_bounds__(KBLOCK, NS == 2 ? 8 : 1) k_bicg_p(Op A, KrySys<NS, T> K, int it, int nb, int kmax, double rtol,
-                                                  double atol, int fin_only) {
+__global__ void __launch_bounds__(KBLOCK, NS == 2 ? 8 : 1)
+k_bicg_p(Op A, KrySys<NS, T> K, int it, int nb, int kmax, double rtol, double atol, int fin_only) {
     auto w = A.walk();
     Idx x;
     T r[NS], p[NS], v[NS];

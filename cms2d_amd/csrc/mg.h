@@ -13,9 +13,11 @@
 //     cells at ratio 55 and 10.5 pp BiCGStab iterations a solve with the short
 //     one, 5.4 with three more levels; 2000 x 1500 cells of 20 m at dt 30 s:
 //     63 x 47 at 0.3, where more levels save nothing.)  The FP32 form and the
-//     telescoping grids stay with the short one: there their solves stop with
-//     a smooth error of up to 2e-7 of the rms velocity at wet/dry edges, which
-//     the deep one changes by as much;
+//     telescoping grids stay with the short one.  With the deep one their pp
+//     iterations would fall (200 x 100 FP32 at dt 60 s: 96 -> 51 a step; 301 x 211
+//     telescoping at dt 60 s: 86 -> 52) and their results move, by up to 1.8e-10 of
+//     a field and 6e-9 of its rms value in a cell over 42 such grids: no further
+//     from solves to rtol 1e-13 (1.3e-9 with either) than those of the short one;
 //   * smoother: one red-black Gauss-Seidel sweep before (red first, from a zero
 //     guess) and after (red first) the coarse correction;
 //   * restriction: sum of the children's residuals (the equations are cell
